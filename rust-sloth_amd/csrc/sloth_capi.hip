@@ -457,50 +457,80 @@ static int join_streams(hipStream_t from, hipStream_t to, hipEvent_t ev)
     return SLOTH_OK;
 }
 
-// Device scratch of the flush encoders.
+// Scratch of the flush encoders and their host side.
 struct Encoder {
-    DevBuf d_off, d_block, d_total, d_out;
+    DevBuf d_len, d_off, d_out;
+    PinBuf h_off;   // frame offsets of the stream
+    PinBuf h_one;   // bytes of a small stream, written by the kernel
 
-    // n cells of one frame; a terminal-mode frame (image false) starts with
-    // crossterm's MoveTo(0, 0), CSI "1;1H" (context.rs:53-55)
-    int run(const uint32_t* d_cells, uint64_t n, bool image, int mode, char* out, uint64_t cap, uint64_t* len,
-            hipStream_t s)
+    // Bytes of a stream that are on the device at once.
+    static constexpr uint64_t GROUP_BYTES = 256ull << 20;
+
+    // The stream of frames [first, first + count) (flat: their flushes in
+    // `mode`; framing: the -j export of them).  *len gets its length; out
+    // (null: the length only) takes it and holds cap bytes.
+    int run(const Job& job, uint32_t first, uint32_t count, bool framing, int mode, char* out, uint64_t cap,
+            uint64_t* len, hipStream_t s)
     {
-        if (mode != SLOTH_ENCODE_TEXT && mode != SLOTH_ENCODE_ANSI && mode != SLOTH_ENCODE_HTML)
-            return fail(SLOTH_EINVAL, "encode mode must be SLOTH_ENCODE_TEXT, SLOTH_ENCODE_ANSI or SLOTH_ENCODE_HTML");
-        static const char MOVE_TO_ORIGIN[] = "\x1b[1;1H";
-        const uint64_t pre = image ? 0 : sizeof MOVE_TO_ORIGIN - 1;
+        uint64_t most = 0;
+        for (uint32_t f = first; f < first + count; ++f) most = std::max(most, frame_cells(job.frames[f]));
+        EncodeJob j;
+        j.cells = job.d_cells.as<uint32_t>();
+        j.frames = job.d_frames.as<Frame>();
+        j.first = first;
+        j.count = count;
+        j.max_blocks = encode_blocks(most);
+        j.mode = mode;
+        j.framing = framing ? 1 : 0;
+        const bool one = count == 1 && most <= ENC_ONE_CELLS;
+        const uint64_t blocks = (uint64_t)count * j.max_blocks;
         int rc;
-        const uint64_t nb = encode_blocks(n);
-        if ((rc = d_off.reserve(std::max<uint64_t>(8, n * 8))) || (rc = d_block.reserve(std::max<uint64_t>(8, nb * 8))) ||
-            (rc = d_total.reserve(8)))
-            return rc;
-        uint64_t total = 0;
-        if (n) {
-            if ((rc = launch_encode_size(d_cells, n, mode, d_off.as<uint64_t>(), d_block.as<uint64_t>(),
-                                         d_total.as<uint64_t>(), s)))
-                return rc;
-            HIP_TRY(hipMemcpyAsync(&total, d_total.p, 8, hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
+        if ((rc = h_off.reserve(((uint64_t)count + 1) * 8))) return rc;
+        j.frame_off = h_off.as<uint64_t>();
+        if (one) {
+            j.block_len = nullptr;
+            j.block_off = nullptr;
+            if (out && (rc = h_one.reserve(encode_bound(most, mode)))) return rc;
+            if ((rc = launch_encode_one(j, out ? h_one.as<uint8_t>() : nullptr, s))) return rc;
+        } else {
+            if ((rc = d_len.reserve(blocks * 4)) || (rc = d_off.reserve(blocks * 8))) return rc;
+            j.block_len = d_len.as<uint32_t>();
+            j.block_off = d_off.as<uint64_t>();
+            if ((rc = launch_encode_len(j, s))) return rc;
         }
-        const uint64_t full = pre + total + (mode == SLOTH_ENCODE_TEXT ? 1 : 0);   // println!'s newline
-        if (len) *len = full;
+        HIP_TRY(hipStreamSynchronize(s));
+        const uint64_t* off = h_off.as<uint64_t>();
+        const uint64_t total = off[count];
+        if (len) *len = total;
         if (!out) return SLOTH_OK;
-        if (cap < full) return fail(SLOTH_EINVAL, "encode buffer holds %llu bytes, %llu needed",
-                                    (unsigned long long)cap, (unsigned long long)full);
-        memcpy(out, MOVE_TO_ORIGIN, pre);
-        if (total) {
-            if ((rc = d_out.reserve(total))) return rc;
-            if ((rc = launch_encode_write(d_cells, n, mode, d_off.as<uint64_t>(), d_block.as<uint64_t>(),
-                                          d_out.as<uint8_t>(), s)))
-                return rc;
-            HIP_TRY(hipMemcpyAsync(out + pre, d_out.p, total, hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
+        if (cap < total)
+            return fail(SLOTH_EINVAL, "encode buffer holds %llu bytes, %llu needed", (unsigned long long)cap,
+                        (unsigned long long)total);
+        if (one) {
+            memcpy(out, h_one.p, total);
+            return SLOTH_OK;
         }
-        if (mode == SLOTH_ENCODE_TEXT) out[pre + total] = '\n';
+        // groups of whole frames of up to GROUP_BYTES (one frame at least)
+        for (uint32_t f0 = 0; f0 < count;) {
+            uint32_t f1 = f0 + 1;
+            while (f1 < count && off[f1 + 1] - off[f0] <= GROUP_BYTES) ++f1;
+            const uint64_t bytes = off[f1] - off[f0];
+            if ((rc = d_out.reserve(bytes))) return rc;
+            if ((rc = launch_encode_write(j, f0, f1, off[f0], d_out.as<uint8_t>(), s))) return rc;
+            HIP_TRY(hipMemcpyAsync(out + off[f0], d_out.p, bytes, hipMemcpyDeviceToHost, s));
+            HIP_TRY(hipStreamSynchronize(s));
+            f0 = f1;
+        }
         return SLOTH_OK;
     }
 };
+
+static int check_encode_mode(int mode)
+{
+    if (mode != SLOTH_ENCODE_TEXT && mode != SLOTH_ENCODE_ANSI && mode != SLOTH_ENCODE_HTML)
+        return fail(SLOTH_EINVAL, "encode mode must be SLOTH_ENCODE_TEXT, SLOTH_ENCODE_ANSI or SLOTH_ENCODE_HTML");
+    return SLOTH_OK;
+}
 
 // ---------------------------------------------------------------------------
 // contexts
@@ -1004,10 +1034,8 @@ int sloth_context_encode(sloth_context* ctx, int mode, char* out, uint64_t cap, 
     ARG_CHECK(ctx, "null context");
     int rc = sloth_context_read(ctx, nullptr, nullptr, nullptr);   // render + overflow check
     if (rc) return rc;
-    // the frame's own cells (the layout pads the buffer past them)
-    const Frame& fr = ctx->job.frames[0];
-    return ctx->enc.run(ctx->job.d_cells.as<uint32_t>(), frame_cells(fr), fr.image != 0, mode, out, cap, len,
-                        ctx->stream);
+    if ((rc = check_encode_mode(mode))) return rc;
+    return ctx->enc.run(ctx->job, 0, 1, false, mode, out, cap, len, ctx->stream);
 }
 
 int sloth_context_device_buffers(sloth_context* ctx, uint32_t** d_cells, float** d_z, uint64_t* n_cells,
@@ -1221,9 +1249,8 @@ int sloth_batch_encode_frame(sloth_batch* b, uint32_t frame, int mode, char* out
     if (!b->ran) return fail(SLOTH_ESTATE, "batch has not been run");
     int rc = sloth_batch_sync(b);
     if (rc) return rc;
-    const Frame& fr = b->job.frames[frame];
-    const uint64_t nc = frame_cells(fr);
-    return b->enc.run(b->job.d_cells.as<uint32_t>() + fr.cell_off, nc, fr.image != 0, mode, out, cap, len, b->stream);
+    if ((rc = check_encode_mode(mode))) return rc;
+    return b->enc.run(b->job, frame, 1, false, mode, out, cap, len, b->stream);
 }
 
 int sloth_batch_encode_export(sloth_batch* b, uint32_t first, uint32_t count, int mode, char* out, uint64_t cap,
@@ -1239,37 +1266,7 @@ int sloth_batch_encode_export(sloth_batch* b, uint32_t first, uint32_t count, in
     if (rc) return rc;
     // main.rs:55-58, 85-106: the header, then per frame a backtick line, the
     // frame's flush and "`," -- "`];" after the last one
-    static const char HEAD[] = "let frames = [\n", OPEN[] = "`\n", NEXT[] = "`,\n", LAST[] = "`];\n";
-    uint64_t pos = 0;
-    auto put = [&](const char* txt, uint64_t n) -> int {
-        if (out) {
-            if (pos + n > cap)
-                return fail(SLOTH_EINVAL, "export buffer holds %llu bytes, more are needed", (unsigned long long)cap);
-            memcpy(out + pos, txt, n);
-        }
-        pos += n;
-        return SLOTH_OK;
-    };
-    if ((rc = put(HEAD, sizeof HEAD - 1))) return rc;
-    for (uint32_t f = first; f < first + count; ++f) {
-        if ((rc = put(OPEN, sizeof OPEN - 1))) return rc;
-        const Frame& fr = b->job.frames[f];
-        uint64_t n = 0;
-        if ((rc = b->enc.run(b->job.d_cells.as<uint32_t>() + fr.cell_off, frame_cells(fr), fr.image != 0, mode,
-                             nullptr, 0, &n, b->stream)))
-            return rc;
-        if (out) {
-            if (pos + n > cap)
-                return fail(SLOTH_EINVAL, "export buffer holds %llu bytes, more are needed", (unsigned long long)cap);
-            if ((rc = b->enc.run(b->job.d_cells.as<uint32_t>() + fr.cell_off, frame_cells(fr), fr.image != 0, mode,
-                                 out + pos, cap - pos, &n, b->stream)))
-                return rc;
-        }
-        pos += n;
-        if ((rc = f + 1 < first + count ? put(NEXT, sizeof NEXT - 1) : put(LAST, sizeof LAST - 1))) return rc;
-    }
-    *len = pos;
-    return SLOTH_OK;
+    return b->enc.run(b->job, first, count, true, mode, out, cap, len, b->stream);
 }
 
 int sloth_batch_device_frame(sloth_batch* b, uint32_t frame, uint32_t** d_cells, float** d_z)
