@@ -23,6 +23,7 @@
 #include "sloth_kernels.h"
 #include "sloth_models.h"
 #include "sloth_shade.h"
+#include "sloth_stage.h"
 #include "sloth_tiled.h"
 
 using namespace sloth;
@@ -193,7 +194,23 @@ struct Job {
     std::vector<Draw> draws;
     uint64_t n_cells = 0, n_z = 0, n_rows = 0, n_items = 0;
 
-    DevBuf d_frames, d_draws, d_ramps, d_cells, d_z, d_keys, d_nl, d_win;
+    // frames, draws and shaders, one after another: one copy uploads them
+    DevBuf d_tables;
+    // pinned, kept while the job lives: the tables' host copy, then the
+    // frames' overflow flags (TiledPlan::overflow)
+    PinLease pin;
+    size_t draws_at = 0, ramps_at = 0, table_bytes = 0, pin_tables = 0;
+    hipEvent_t uploaded = nullptr;   // the tables have been copied
+    const Frame* dev_frames() const { return d_tables.as<Frame>(); }
+    const Draw* dev_draws() const { return (const Draw*)(d_tables.as<uint8_t>() + draws_at); }
+    const Ramp* dev_ramps() const { return (const Ramp*)(d_tables.as<uint8_t>() + ramps_at); }
+    DevBuf d_cells, d_z, d_keys, d_nl, d_win;
+    ~Job()
+    {
+        if (!uploaded) return;
+        (void)hipEventSynchronize(uploaded);
+        (void)hipEventDestroy(uploaded);
+    }
     TiledPlan tiled;
     int path = PATH_GLOBAL;
     bool laid_out = false;
@@ -207,8 +224,9 @@ struct Job {
     }
 
     // Lays out frames and draws (draws grouped by frame, order within a frame
-    // kept) and allocates device tables and outputs.
-    int layout()
+    // kept) and allocates device tables and outputs.  Renders run on `s` (or
+    // are joined to it).
+    int layout(hipStream_t s)
     {
         const uint32_t F = (uint32_t)fin.size();
         std::vector<uint32_t> order(din.size());
@@ -271,9 +289,23 @@ struct Job {
         // frames of either width parity (or both) take it
         path = (small_frames && ramps.size() < 256 && !force_global()) ? PATH_TILED : PATH_GLOBAL;
         int rc;
-        if ((rc = d_frames.reserve(sizeof(Frame) * std::max<size_t>(1, frames.size())))) return rc;
-        if ((rc = d_draws.reserve(sizeof(Draw) * std::max<size_t>(1, draws.size())))) return rc;
-        if ((rc = d_ramps.reserve(sizeof(Ramp) * std::max<size_t>(1, ramps.size())))) return rc;
+        auto room = [](size_t n) { return (n + 255) & ~(size_t)255; };
+        draws_at = room(sizeof(Frame) * std::max<size_t>(1, frames.size()));
+        ramps_at = draws_at + room(sizeof(Draw) * std::max<size_t>(1, draws.size()));
+        table_bytes = ramps_at + room(sizeof(Ramp) * std::max<size_t>(1, ramps.size()));
+        if ((rc = d_tables.reserve(table_bytes))) return rc;
+        if (table_bytes > pin_tables) {
+            HIP_TRY(hipStreamSynchronize(s));   // nothing in flight uses the old block
+            pin_tables = table_bytes;
+            const size_t flags = sizeof(uint32_t) * std::max<size_t>(1, frames.size());
+            if ((rc = pin.take(pin_tables + flags, s))) {
+                pin_tables = 0;
+                return rc;
+            }
+            pin.done();   // whoever reuses or ends it waits first
+            tiled.overflow = (uint32_t*)(pin.as<uint8_t>() + pin_tables);
+            memset(tiled.overflow, 0, flags);
+        }
         if ((rc = d_cells.reserve(sizeof(uint32_t) * n_cells))) return rc;
         if ((rc = d_z.reserve(sizeof(float) * n_z))) return rc;
         if (path == PATH_GLOBAL) {
@@ -301,20 +333,17 @@ struct Job {
         return e && e[0] == '1';
     }
 
+    // Enqueues the tables' copy on `s`; they have been taken on return.
     int upload(hipStream_t s)
     {
-        if (!frames.empty())
-            HIP_TRY(hipMemcpyAsync(d_frames.p, frames.data(), sizeof(Frame) * frames.size(), hipMemcpyHostToDevice, s));
-        if (!draws.empty())
-            HIP_TRY(hipMemcpyAsync(d_draws.p, draws.data(), sizeof(Draw) * draws.size(), hipMemcpyHostToDevice, s));
-        if (!ramps.empty())
-            HIP_TRY(hipMemcpyAsync(d_ramps.p, ramps.data(), sizeof(Ramp) * ramps.size(), hipMemcpyHostToDevice, s));
-        if (path == PATH_TILED) {
-            int rc = tiled.upload(s);
-            if (rc) return rc;
-        }
-        // the host vectors may change after return: wait for the copies
-        HIP_TRY(hipStreamSynchronize(s));
+        if (!uploaded) HIP_TRY(hipEventCreateWithFlags(&uploaded, hipEventDisableTiming));
+        else HIP_TRY(hipEventSynchronize(uploaded));   // the last copy no longer reads them
+        uint8_t* h = pin.as<uint8_t>();
+        if (!frames.empty()) memcpy(h, frames.data(), sizeof(Frame) * frames.size());
+        if (!draws.empty()) memcpy(h + draws_at, draws.data(), sizeof(Draw) * draws.size());
+        if (!ramps.empty()) memcpy(h + ramps_at, ramps.data(), sizeof(Ramp) * ramps.size());
+        HIP_TRY(hipMemcpyAsync(d_tables.p, h, table_bytes, hipMemcpyHostToDevice, s));
+        HIP_TRY(hipEventRecord(uploaded, s));
         return SLOTH_OK;
     }
 
@@ -346,8 +375,8 @@ struct Job {
         for (uint32_t d = d_lo; d < d_hi; ++d) max_n = std::max(max_n, draws[d].n);
         for (uint32_t d = d_lo; d < d_hi && max_n; d += 65535u) {
             const uint32_t nd = std::min<uint32_t>(65535u, d_hi - d);
-            hipLaunchKernelGGL(k_raster_global, dim3(blocks_for(max_n), nd), dim3(256), 0, s, d_draws.as<Draw>(), d,
-                               d_frames.as<Frame>(), d_keys.as<uint64_t>(), d_nl.as<int32_t>());
+            hipLaunchKernelGGL(k_raster_global, dim3(blocks_for(max_n), nd), dim3(256), 0, s, dev_draws(), d,
+                               dev_frames(), d_keys.as<uint64_t>(), d_nl.as<int32_t>());
             HIP_TRY(hipGetLastError());
         }
         if (ev) HIP_TRY(hipEventRecord((*ev)[2], s));
@@ -360,8 +389,8 @@ struct Job {
         }
         for (uint32_t f = f_lo; f < f_hi && max_wh; f += 65535u) {
             const uint32_t nf = std::min<uint32_t>(65535u, f_hi - f);
-            hipLaunchKernelGGL(k_winner_global, dim3(blocks_for(max_wh), nf), dim3(256), 0, s, d_draws.as<Draw>(),
-                               d_ramps.as<Ramp>(), d_frames.as<Frame>(), f, d_keys.as<uint64_t>(), d_z.as<float>(), win,
+            hipLaunchKernelGGL(k_winner_global, dim3(blocks_for(max_wh), nf), dim3(256), 0, s, dev_draws(),
+                               dev_ramps(), dev_frames(), f, d_keys.as<uint64_t>(), d_z.as<float>(), win,
                                win_raw ? 1u : 0u);
             HIP_TRY(hipGetLastError());
         }
@@ -369,7 +398,7 @@ struct Job {
         for (uint32_t f = f_lo; f < f_hi && max_cells; f += 65535u) {
             const uint32_t nf = std::min<uint32_t>(65535u, f_hi - f);
             hipLaunchKernelGGL(k_resolve_global, dim3(blocks_for(max_cells), nf), dim3(256), 0, s,
-                               d_frames.as<Frame>(), f, d_keys.as<uint64_t>(), d_nl.as<int32_t>(),
+                               dev_frames(), f, d_keys.as<uint64_t>(), d_nl.as<int32_t>(),
                                d_cells.as<uint32_t>());
             HIP_TRY(hipGetLastError());
         }
@@ -382,7 +411,7 @@ struct Job {
     int prepare(hipStream_t s)
     {
         if (path == PATH_TILED && !tiled.sized)
-            return tiled.size(frames, draws, d_frames.as<Frame>(), d_draws.as<Draw>(), s);
+            return tiled.size(frames, draws, dev_frames(), dev_draws(), s);
         return SLOTH_OK;
     }
 
@@ -413,7 +442,7 @@ struct Job {
     {
         if (f_lo >= f_hi) return SLOTH_OK;
         if (path == PATH_TILED)
-            return tiled.launch(frames, draws, d_frames.as<Frame>(), d_draws.as<Draw>(), d_ramps.as<Ramp>(), f_lo,
+            return tiled.launch(frames, draws, dev_frames(), dev_draws(), dev_ramps(), f_lo,
                                 f_hi, d_cells.as<uint32_t>(), d_z.as<float>(), win, win_raw, (uint32_t)ramps.size(), s,
                                 ev, s2, join);
         return launch_global(f_lo, f_hi, s, win, win_raw, ev);
@@ -460,8 +489,6 @@ static int join_streams(hipStream_t from, hipStream_t to, hipEvent_t ev)
 // Scratch of the flush encoders and their host side.
 struct Encoder {
     DevBuf d_len, d_off, d_out;
-    PinBuf h_off;   // frame offsets of the stream
-    PinBuf h_one;   // bytes of a small stream, written by the kernel
 
     // Bytes of a stream that are on the device at once.
     static constexpr uint64_t GROUP_BYTES = 256ull << 20;
@@ -476,7 +503,7 @@ struct Encoder {
         for (uint32_t f = first; f < first + count; ++f) most = std::max(most, frame_cells(job.frames[f]));
         EncodeJob j;
         j.cells = job.d_cells.as<uint32_t>();
-        j.frames = job.d_frames.as<Frame>();
+        j.frames = job.dev_frames();
         j.first = first;
         j.count = count;
         j.max_blocks = encode_blocks(most);
@@ -484,14 +511,17 @@ struct Encoder {
         j.framing = framing ? 1 : 0;
         const bool one = count == 1 && most <= ENC_ONE_CELLS;
         const uint64_t blocks = (uint64_t)count * j.max_blocks;
+        // pinned: the frame offsets, and a small stream's bytes after them
+        PinLease pin;
+        const uint64_t off_bytes = (((uint64_t)count + 1) * 8 + 255) & ~255ull;
         int rc;
-        if ((rc = h_off.reserve(((uint64_t)count + 1) * 8))) return rc;
-        j.frame_off = h_off.as<uint64_t>();
+        if ((rc = pin.take(off_bytes + (one && out ? encode_bound(most, mode) : 0), s))) return rc;
+        j.frame_off = pin.as<uint64_t>();
+        uint8_t* h_one = pin.as<uint8_t>() + off_bytes;
         if (one) {
             j.block_len = nullptr;
             j.block_off = nullptr;
-            if (out && (rc = h_one.reserve(encode_bound(most, mode)))) return rc;
-            if ((rc = launch_encode_one(j, out ? h_one.as<uint8_t>() : nullptr, s))) return rc;
+            if ((rc = launch_encode_one(j, out ? h_one : nullptr, s))) return rc;
         } else {
             if ((rc = d_len.reserve(blocks * 4)) || (rc = d_off.reserve(blocks * 8))) return rc;
             j.block_len = d_len.as<uint32_t>();
@@ -499,7 +529,8 @@ struct Encoder {
             if ((rc = launch_encode_len(j, s))) return rc;
         }
         HIP_TRY(hipStreamSynchronize(s));
-        const uint64_t* off = h_off.as<uint64_t>();
+        pin.done();
+        const uint64_t* off = pin.as<uint64_t>();
         const uint64_t total = off[count];
         if (len) *len = total;
         if (!out) return SLOTH_OK;
@@ -507,7 +538,7 @@ struct Encoder {
             return fail(SLOTH_EINVAL, "encode buffer holds %llu bytes, %llu needed", (unsigned long long)cap,
                         (unsigned long long)total);
         if (one) {
-            memcpy(out, h_one.p, total);
+            memcpy(out, h_one, total);
             return SLOTH_OK;
         }
         // groups of whole frames of up to GROUP_BYTES (one frame at least)
@@ -517,8 +548,8 @@ struct Encoder {
             const uint64_t bytes = off[f1] - off[f0];
             if ((rc = d_out.reserve(bytes))) return rc;
             if ((rc = launch_encode_write(j, f0, f1, off[f0], d_out.as<uint8_t>(), s))) return rc;
-            HIP_TRY(hipMemcpyAsync(out + off[f0], d_out.p, bytes, hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
+            const Span whole{out + off[f0], d_out.p, bytes};
+            if ((rc = copy_out(&whole, 1, s))) return rc;
             f0 = f1;
         }
         return SLOTH_OK;
@@ -536,6 +567,7 @@ static int check_encode_mode(int mode)
 // contexts
 // ---------------------------------------------------------------------------
 struct sloth_context {
+    PinPoolUser pin_user;
     Job job;
     float U[16];
     hipStream_t stream = nullptr;
@@ -555,6 +587,7 @@ struct sloth_context {
 // batches
 // ---------------------------------------------------------------------------
 struct sloth_batch {
+    PinPoolUser pin_user;
     Job job;
     std::vector<float> U;       // per frame utransform
     hipStream_t stream = nullptr;
@@ -979,7 +1012,7 @@ static int context_render(sloth_context* ctx, hipStream_t s, bool want_win)
 {
     int rc;
     if (!ctx->rendered) {
-        if ((rc = ctx->job.layout())) return rc;
+        if ((rc = ctx->job.layout(ctx->stream))) return rc;
         if ((rc = ctx->job.upload(ctx->stream))) return rc;
         if ((rc = ctx->job.prepare(ctx->stream))) return rc;
         if (want_win && (rc = ctx->job.ensure_win())) return rc;
@@ -1000,6 +1033,18 @@ static int context_render(sloth_context* ctx, hipStream_t s, bool want_win)
     return SLOTH_OK;
 }
 
+// Checks the last render for tile-list overflow, once; *again: the frame has
+// been rendered anew.
+static int context_check(sloth_context* ctx, bool& again)
+{
+    again = false;
+    if (ctx->checked) return SLOTH_OK;
+    int rc = ctx->job.finish(0, 1, ctx->stream, ctx->win_valid ? ctx->job.d_win.as<int32_t>() : nullptr, &again);
+    if (rc) return rc;
+    ctx->checked = true;
+    return SLOTH_OK;
+}
+
 int sloth_context_render(sloth_context* ctx, void* stream)
 {
     ARG_CHECK(ctx, "null context");
@@ -1015,27 +1060,37 @@ int sloth_context_read(sloth_context* ctx, uint32_t* cells, float* z, int32_t* w
     if (rc) return rc;
     hipStream_t s = ctx->stream;
     if ((rc = context_render(ctx, s, winners != nullptr))) return rc;
-    if (!ctx->checked) {
-        if ((rc = ctx->job.finish(0, 1, s, ctx->win_valid ? ctx->job.d_win.as<int32_t>() : nullptr))) return rc;
-        ctx->checked = true;
-    }
-    const Job& j = ctx->job;
-    const uint64_t nc = frame_cells(j.frames[0]);   // the buffer is padded past the frame's cells
-    if (cells && nc) HIP_TRY(hipMemcpyAsync(cells, j.d_cells.p, sizeof(uint32_t) * nc, hipMemcpyDeviceToHost, s));
-    if (z && j.n_z) HIP_TRY(hipMemcpyAsync(z, j.d_z.p, sizeof(float) * j.n_z, hipMemcpyDeviceToHost, s));
-    if (winners && j.n_z)
-        HIP_TRY(hipMemcpyAsync(winners, j.d_win.p, sizeof(int32_t) * j.n_z, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return SLOTH_OK;
+    auto copies = [&]() -> int {
+        const Job& j = ctx->job;
+        const uint64_t nc = frame_cells(j.frames[0]);   // the buffer is padded past the frame's cells
+        Span v[3];
+        int n = 0;
+        if (cells && nc) v[n++] = Span{cells, j.d_cells.p, sizeof(uint32_t) * nc};
+        if (z && j.n_z) v[n++] = Span{z, j.d_z.p, sizeof(float) * j.n_z};
+        if (winners && j.n_z) v[n++] = Span{winners, j.d_win.p, sizeof(int32_t) * j.n_z};
+        if (n) return copy_out(v, n, s);
+        HIP_TRY(hipStreamSynchronize(s));
+        return SLOTH_OK;
+    };
+    if ((rc = copies())) return rc;
+    bool again = false;   // a tile list had overflowed: the frame was rendered again
+    if ((rc = context_check(ctx, again))) return rc;
+    return again ? copies() : SLOTH_OK;
 }
 
 int sloth_context_encode(sloth_context* ctx, int mode, char* out, uint64_t cap, uint64_t* len)
 {
     ARG_CHECK(ctx, "null context");
-    int rc = sloth_context_read(ctx, nullptr, nullptr, nullptr);   // render + overflow check
+    int rc = ensure_device();
     if (rc) return rc;
+    if ((rc = context_render(ctx, ctx->stream, false))) return rc;
     if ((rc = check_encode_mode(mode))) return rc;
-    return ctx->enc.run(ctx->job, 0, 1, false, mode, out, cap, len, ctx->stream);
+    // the stream's wait serves the overflow check too
+    rc = ctx->enc.run(ctx->job, 0, 1, false, mode, out, cap, len, ctx->stream);
+    bool again = false;
+    const int rc2 = context_check(ctx, again);
+    if (rc2) return rc2;
+    return again ? ctx->enc.run(ctx->job, 0, 1, false, mode, out, cap, len, ctx->stream) : rc;
 }
 
 int sloth_context_device_buffers(sloth_context* ctx, uint32_t** d_cells, float** d_z, uint64_t* n_cells,
@@ -1043,7 +1098,7 @@ int sloth_context_device_buffers(sloth_context* ctx, uint32_t** d_cells, float**
 {
     ARG_CHECK(ctx, "null context");
     if (!ctx->job.laid_out) {
-        int rc = ctx->job.layout();
+        int rc = ctx->job.layout(ctx->stream);
         if (rc) return rc;
     }
     if (d_cells) *d_cells = ctx->job.d_cells.as<uint32_t>();
@@ -1103,7 +1158,7 @@ int sloth_batch_create(const sloth_frame_desc* frames, uint32_t n_frames, const 
         di.ramp = ri;
         b->job.din.push_back(di);
     }
-    if ((rc = b->job.layout()) || (rc = b->job.upload(b->stream))) {
+    if ((rc = b->job.layout(b->stream)) || (rc = b->job.upload(b->stream))) {
         delete b;
         return rc;
     }
@@ -1122,7 +1177,7 @@ int sloth_batch_set_transforms(sloth_batch* b, const float* transforms16)
     }
     // the draw table is grouped by frame; recompute it in the same order
     int rc;
-    if ((rc = b->job.layout()) || (rc = b->job.upload(b->stream))) return rc;
+    if ((rc = b->job.layout(b->stream)) || (rc = b->job.upload(b->stream))) return rc;
     // the frames on the device show the old transforms: a read must follow a
     // run, whose overflow check covers the new ones
     b->ran = false;
@@ -1233,11 +1288,12 @@ int sloth_batch_read_frame(sloth_batch* b, uint32_t frame, uint32_t* cells, floa
         if (replanned) drop_graph(b);
         b->win_valid[frame] = true;
     }
-    if (cells)
-        HIP_TRY(hipMemcpyAsync(cells, b->job.d_cells.as<uint32_t>() + fr.cell_off, 4 * nc, hipMemcpyDeviceToHost, s));
-    if (z) HIP_TRY(hipMemcpyAsync(z, b->job.d_z.as<float>() + fr.z_off, 4 * WH, hipMemcpyDeviceToHost, s));
-    if (winners)
-        HIP_TRY(hipMemcpyAsync(winners, b->job.d_win.as<int32_t>() + fr.z_off, 4 * WH, hipMemcpyDeviceToHost, s));
+    Span v[3];
+    int n = 0;
+    if (cells) v[n++] = Span{cells, b->job.d_cells.as<uint32_t>() + fr.cell_off, 4 * nc};
+    if (z) v[n++] = Span{z, b->job.d_z.as<float>() + fr.z_off, 4 * WH};
+    if (winners) v[n++] = Span{winners, b->job.d_win.as<int32_t>() + fr.z_off, 4 * WH};
+    if (n) return copy_out(v, n, s);
     HIP_TRY(hipStreamSynchronize(s));
     return SLOTH_OK;
 }
@@ -1363,7 +1419,7 @@ int sloth_batch_set_tile(sloth_batch* b, uint32_t tile_w, uint32_t tile_h)
     int rc = b->job.tiled.set_tile(tile_w, tile_h);
     if (rc) return rc;
     if (!b->job.tiled.sized) {
-        if ((rc = b->job.layout()) || (rc = b->job.upload(b->stream))) return rc;
+        if ((rc = b->job.layout(b->stream)) || (rc = b->job.upload(b->stream))) return rc;
         drop_graph(b);
         b->ran = false;
     }
@@ -1534,6 +1590,7 @@ int sloth_batch_destroy(sloth_batch* b)
 }  // extern "C"
 
 struct sloth_shading {
+    PinPoolUser pin_user;
     sloth_batch* b = nullptr;
     uint32_t n_tris = 0, n_verts = 0;
     uint64_t n_slots = 0;
@@ -1551,9 +1608,9 @@ static ShadeArgs shade_args(sloth_shading* sh, bool with_target, float* out)
 {
     ShadeArgs a;
     Job& j = sh->b->job;
-    a.frames = j.d_frames.as<Frame>();
+    a.frames = j.dev_frames();
     a.n_frames = (uint32_t)j.frames.size();
-    a.draws = j.d_draws.as<Draw>();
+    a.draws = j.dev_draws();
     a.vis = sh->d_vis.as<int32_t>();
     a.faces = sh->d_faces.as<uint32_t>();
     a.vcolor = sh->d_vcolor.as<float>();
@@ -1701,10 +1758,14 @@ int sloth_shading_set_target(sloth_shading* sh, const float* target)
     return SLOTH_OK;
 }
 
-static int shading_reduce(sloth_shading* sh, double* loss, double* dlight)
+// Copies the results out and sums the per-block partials (in order) into the
+// loss and the light gradient (either may be null).
+static int shading_results(sloth_shading* sh, Span* spans, int n, double* loss, double* dlight)
 {
     const uint32_t nb = sh->n_partials;
-    if (nb) HIP_TRY(hipMemcpy(sh->partial.data(), sh->d_partial.p, (size_t)nb * 32, hipMemcpyDeviceToHost));
+    if (nb) spans[n++] = Span{sh->partial.data(), sh->d_partial.p, (size_t)nb * 32};
+    int rc = copy_out(spans, n, sh->b->stream);
+    if (rc) return rc;
     double acc[4] = {0, 0, 0, 0};
     for (uint32_t i = 0; i < nb; ++i)
         for (int k = 0; k < 4; ++k) acc[k] += sh->partial[(size_t)i * 4 + k];
@@ -1714,14 +1775,14 @@ static int shading_reduce(sloth_shading* sh, double* loss, double* dlight)
     return SLOTH_OK;
 }
 
-static int shading_params(sloth_shading* sh, const float* vcolor, const float* vnormal, const float* light)
+static int shading_params(sloth_shading* sh, const float* vcolor, const float* vnormal, const float* light,
+                          PinLease& pin)
 {
-    hipStream_t s = sh->b->stream;
-    if (sh->n_verts) {
-        HIP_TRY(hipMemcpyAsync(sh->d_vcolor.p, vcolor, (size_t)sh->n_verts * 12, hipMemcpyHostToDevice, s));
-        HIP_TRY(hipMemcpyAsync(sh->d_vnormal.p, vnormal, (size_t)sh->n_verts * 12, hipMemcpyHostToDevice, s));
-    }
-    HIP_TRY(hipMemcpyAsync(sh->d_light.p, light, 12, hipMemcpyHostToDevice, s));
+    const size_t nv = (size_t)sh->n_verts * 12;
+    const Span v[3] = {{(void*)vcolor, sh->d_vcolor.p, nv}, {(void*)vnormal, sh->d_vnormal.p, nv},
+                       {(void*)light, sh->d_light.p, 12}};
+    int rc = copy_in(v, 3, pin, sh->b->stream);
+    if (rc) return rc;
     sh->has_params = true;
     return SLOTH_OK;
 }
@@ -1741,14 +1802,13 @@ static int shading_backward_launch(sloth_shading* sh)
 // Copies the gradients out and sums the per-block loss and light partials.
 static int shading_gradients(sloth_shading* sh, double* loss, float* d_vcolor, float* d_vnormal, float* d_light)
 {
-    hipStream_t s = sh->b->stream;
-    if (d_vcolor && sh->n_verts)
-        HIP_TRY(hipMemcpyAsync(d_vcolor, sh->d_dcolor.p, (size_t)sh->n_verts * 12, hipMemcpyDeviceToHost, s));
-    if (d_vnormal && sh->n_verts)
-        HIP_TRY(hipMemcpyAsync(d_vnormal, sh->d_dnormal.p, (size_t)sh->n_verts * 12, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    Span v[3];
+    int n = 0;
+    const size_t nv = (size_t)sh->n_verts * 12;
+    if (d_vcolor && nv) v[n++] = Span{d_vcolor, sh->d_dcolor.p, nv};
+    if (d_vnormal && nv) v[n++] = Span{d_vnormal, sh->d_dnormal.p, nv};
     double dl[3];
-    int rc = shading_reduce(sh, loss, dl);
+    int rc = shading_results(sh, v, n, loss, dl);
     if (rc) return rc;
     if (d_light)
         for (int k = 0; k < 3; ++k) d_light[k] = (float)dl[k];
@@ -1762,7 +1822,8 @@ int sloth_shading_forward(sloth_shading* sh, const float* vcolor, const float* v
     int rc = ensure_device();
     if (rc) return rc;
     hipStream_t s = sh->b->stream;
-    if ((rc = shading_params(sh, vcolor, vnormal, light))) return rc;
+    PinLease pin;
+    if ((rc = shading_params(sh, vcolor, vnormal, light, pin))) return rc;
     float* d_out = nullptr;
     if (out_rgb) {
         if ((rc = sh->d_out.reserve(std::max<size_t>(4, sh->n_slots * 12)))) return rc;
@@ -1771,9 +1832,12 @@ int sloth_shading_forward(sloth_shading* sh, const float* vcolor, const float* v
     }
     if ((rc = launch_shade(shade_args(sh, sh->has_target, d_out), false, s))) return rc;
     sh->n_partials = shade_blocks(sh->n_slots);
-    if (out_rgb) HIP_TRY(hipMemcpyAsync(out_rgb, sh->d_out.p, sh->n_slots * 12, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return shading_reduce(sh, loss, nullptr);
+    Span v[2];
+    int n = 0;
+    if (out_rgb) v[n++] = Span{out_rgb, sh->d_out.p, sh->n_slots * 12};
+    if ((rc = shading_results(sh, v, n, loss, nullptr))) return rc;
+    pin.done();
+    return SLOTH_OK;
 }
 
 int sloth_shading_backward(sloth_shading* sh, float* d_vcolor, float* d_vnormal, float* d_light)
@@ -1794,9 +1858,12 @@ int sloth_shading_step(sloth_shading* sh, const float* vcolor, const float* vnor
     if (!sh->has_target) return fail(SLOTH_ESTATE, "a step needs a target (sloth_shading_set_target)");
     int rc = ensure_device();
     if (rc) return rc;
-    if ((rc = shading_params(sh, vcolor, vnormal, light))) return rc;
+    PinLease pin;
+    if ((rc = shading_params(sh, vcolor, vnormal, light, pin))) return rc;
     if ((rc = shading_backward_launch(sh))) return rc;
-    return shading_gradients(sh, loss, d_vcolor, d_vnormal, d_light);
+    if ((rc = shading_gradients(sh, loss, d_vcolor, d_vnormal, d_light))) return rc;
+    pin.done();
+    return SLOTH_OK;
 }
 
 int sloth_shading_time(sloth_shading* sh, uint32_t steps, uint32_t warmup, float* ms)

@@ -46,38 +46,6 @@ struct DevBuf {
     template <class T> T* as() const { return (T*)p; }
 };
 
-// Pinned host memory owned by a handle, which kernels write and copies land
-// in; grow-only, contents not preserved.
-struct PinBuf {
-    void* p = nullptr;
-    size_t bytes = 0;
-    PinBuf() = default;
-    PinBuf(const PinBuf&) = delete;
-    PinBuf& operator=(const PinBuf&) = delete;
-    ~PinBuf() { release(); }
-    void release()
-    {
-        if (p) (void)hipHostFree(p);
-        p = nullptr;
-        bytes = 0;
-    }
-    int reserve(size_t n)
-    {
-        if (n <= bytes && p) return SLOTH_OK;
-        release();
-        if (n == 0) return SLOTH_OK;
-        hipError_t e = hipHostMalloc(&p, n, hipHostMallocDefault);
-        if (e != hipSuccess) {
-            p = nullptr;
-            (void)hipGetLastError();
-            return fail(SLOTH_ENOMEM, "hipHostMalloc(%zu bytes): %s", n, hipGetErrorString(e));
-        }
-        bytes = n;
-        return SLOTH_OK;
-    }
-    template <class T> T* as() const { return (T*)p; }
-};
-
 }  // namespace sloth
 
 #define HIP_TRY(expr)                                                                                  \

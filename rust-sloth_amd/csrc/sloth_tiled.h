@@ -67,7 +67,8 @@ struct TiledPlan {
     bool sized = false;              // pool offsets match the current layout
     uint64_t generation = 0;         // bumped whenever size() runs (device pointers may change)
     std::vector<uint64_t> off;       // host copy of the per-tile pool offsets (n_tiles + 1)
-    DevBuf d_cursor, d_off, d_pool, d_nl, d_overflow;
+    DevBuf d_cursor, d_off, d_pool, d_nl;
+    uint32_t* overflow = nullptr;    // per frame, the job's pinned memory: kernels write it (rarely), the host reads it after a wait
     // triangles whose candidate box k_careful computes: (frame, triangle,
     // screen vertices) in, 32 bytes each, (triangle, box) out; capacity from
     // the counting run plus headroom
@@ -130,8 +131,6 @@ struct TiledPlan {
     // pool offsets with headroom.
     int size(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
              const Draw* d_draws, hipStream_t s);
-
-    int upload(hipStream_t s) { (void)s; return SLOTH_OK; }
 
     // clear + bin + careful + raster over frames [f_lo, f_hi).  ev (optional)
     // gets 5 events recorded around the 4 stages.  With a second stream s2

@@ -1400,7 +1400,6 @@ int TiledPlan::plan(std::vector<Frame>& frames, uint64_t rows)
     if ((rc = d_cursor.reserve(sizeof(uint32_t) * std::max<uint64_t>(1, n_tiles)))) return rc;
     if ((rc = d_off.reserve(sizeof(uint64_t) * (n_tiles + 1)))) return rc;
     if ((rc = d_nl.reserve(sizeof(int32_t) * std::max<uint64_t>(1, n_rows)))) return rc;
-    if ((rc = d_overflow.reserve(sizeof(uint32_t) * std::max<size_t>(1, frames.size())))) return rc;
     if ((rc = d_careful_cnt.reserve(sizeof(uint32_t) * (TALL_CNT + 1)))) return rc;
     if (has_odd && (rc = d_edges.reserve(sizeof(uint4) * 2 * std::max<uint64_t>(1, n_tiles) * TH))) return rc;
     return SLOTH_OK;
@@ -1415,7 +1414,7 @@ int TiledPlan::launch_clear(const std::vector<Frame>& frames, uint32_t f_lo, uin
     uint64_t n = std::max(t_hi - t_lo, r_hi - r_lo);
     unsigned g = std::max(1u, std::min(blocks(n, 256), 4096u));
     hipLaunchKernelGGL(k_tile_clear, dim3(g), dim3(256), 0, s, d_cursor.as<uint32_t>() + t_lo, t_hi - t_lo,
-                       d_nl.as<int32_t>() + r_lo, r_hi - r_lo, d_overflow.as<uint32_t>() + f_lo, f_hi - f_lo,
+                       d_nl.as<int32_t>() + r_lo, r_hi - r_lo, overflow + f_lo, f_hi - f_lo,
                        d_careful_cnt.as<uint32_t>());
     HIP_TRY(hipGetLastError());
     return SLOTH_OK;
@@ -1430,7 +1429,7 @@ int TiledPlan::launch_bin(const std::vector<Frame>& frames, const std::vector<Dr
         auto run = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, dim3(BIN_BLOCK), 0, s, d_draws, d0, d_frames, tws, ths,
                                d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
-                               d_nl.as<int32_t>(), d_overflow.as<uint32_t>(), d_careful_cnt.as<uint32_t>(),
+                               d_nl.as<int32_t>(), overflow, d_careful_cnt.as<uint32_t>(),
                                d_careful_in.as<uint4>(), careful_cap, flat);
         };
         // the counting run takes the tree variant (it counts the tall triangles)
@@ -1474,12 +1473,12 @@ int TiledPlan::launch_careful(const Frame* d_frames, const Draw* d_draws, bool c
     if (count_only)
         hipLaunchKernelGGL(k_careful<true>, grid, dim3(256), 0, s, d_frames, tws, ths,
                            d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
-                           d_overflow.as<uint32_t>(), d_careful_cnt.as<uint32_t>(), group, d_careful_in.as<uint4>(),
+                           overflow, d_careful_cnt.as<uint32_t>(), group, d_careful_in.as<uint4>(),
                            d_careful_box.as<uint4>(), careful_cap);
     else
         hipLaunchKernelGGL(k_careful<false>, grid, dim3(256), 0, s, d_frames, tws, ths,
                            d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
-                           d_overflow.as<uint32_t>(), d_careful_cnt.as<uint32_t>(), group, d_careful_in.as<uint4>(),
+                           overflow, d_careful_cnt.as<uint32_t>(), group, d_careful_in.as<uint4>(),
                            d_careful_box.as<uint4>(), careful_cap);
     HIP_TRY(hipGetLastError());
     return SLOTH_OK;
@@ -1729,10 +1728,8 @@ int TiledPlan::launch(const std::vector<Frame>& frames, const std::vector<Draw>&
 int TiledPlan::overflowed(uint32_t nf, hipStream_t s, bool& ovf)
 {
     ovf = false;
-    std::vector<uint32_t> h(nf);
-    if (nf) HIP_TRY(hipMemcpyAsync(h.data(), d_overflow.p, sizeof(uint32_t) * nf, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    for (uint32_t v : h) ovf |= (v != 0);
+    for (uint32_t f = 0; f < nf; ++f) ovf |= (((volatile uint32_t*)overflow)[f] != 0);
     return SLOTH_OK;
 }
 

@@ -11,4 +11,4 @@ S=$ROOT/rust-sloth_amd/csrc
   -Xclang -target-feature -Xclang -packed-fp32-ops \
   -Xarch_host -fsanitize=address -Xarch_host -fsanitize=undefined -Xarch_host -fno-omit-frame-pointer -I "$ROOT/include" -I "$S" \
   "$S/sloth_capi.hip" "$S/sloth_global.hip" "$S/sloth_tiled.hip" "$S/sloth_shade.hip" "$S/sloth_encode.hip" \
-  "$S/sloth_models.hip" "$HERE/asan_batch.cpp" -o "$HERE/asan_batch"
+  "$S/sloth_models.hip" "$S/sloth_stage.hip" "$HERE/asan_batch.cpp" -o "$HERE/asan_batch"
