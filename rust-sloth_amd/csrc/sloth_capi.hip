@@ -1597,11 +1597,11 @@ struct sloth_shading {
     bool has_target = false;
     bool has_params = false;
     DevBuf d_faces, d_vis, d_G, d_vcolor, d_vnormal, d_light, d_target, d_out, d_partial, d_vert_acc;
-    DevBuf d_bwd_tile;            // backward tiles per frame (prefix, n_frames + 1)
-    uint64_t n_bwd_tiles = 0;
-    DevBuf d_dcolor, d_dnormal;
-    std::vector<double> partial;
-    uint32_t n_partials = 0;   // per-block partial sums the last pass wrote
+    // the visibility as fragment lists (k_frag_plan)
+    DevBuf d_seg, d_entries, d_chunks;
+    uint64_t n_chunks = 0;
+    DevBuf d_dcolor, d_dnormal, d_sum;
+    bool acc_zero = false;        // d_vert_acc is zero, as a backward pass leaves it
 };
 
 static ShadeArgs shade_args(sloth_shading* sh, bool with_target, float* out)
@@ -1624,8 +1624,10 @@ static ShadeArgs shade_args(sloth_shading* sh, bool with_target, float* out)
     a.n_slots = sh->n_slots;
     a.n_tris = sh->n_tris;
     a.n_verts = sh->n_verts;
-    a.bwd_tile_begin = sh->d_bwd_tile.as<uint64_t>();
-    a.n_bwd_tiles = sh->n_bwd_tiles;
+    a.entries = sh->d_entries.as<uint4>();
+    a.chunks = sh->d_chunks.as<uint4>();
+    a.n_chunks = sh->n_chunks;
+    a.chunks_per_block = bwd_chunks_per_block(sh->n_chunks);
     return a;
 }
 
@@ -1652,6 +1654,44 @@ static void normal_map(const float* M, float* G)
         for (int c = 0; c < 3; ++c) G[r * 3 + c] = (float)(cof[r][c] / k);
 }
 
+// The fragment lists of the visibility: counted, sized, filled.
+static int shading_lists(sloth_shading* sh)
+{
+    Job& j = sh->b->job;
+    hipStream_t s = sh->b->stream;
+    const uint64_t segs = frag_segments(sh->n_tris, (uint32_t)j.draws.size());
+    int rc;
+    if ((rc = sh->d_seg.reserve(std::max<uint64_t>(1, segs) * 32))) return rc;
+    PinLease totals;
+    if ((rc = totals.take(16, s))) return rc;
+    FragPlan p;
+    p.frames = j.dev_frames();
+    p.draws = j.dev_draws();
+    p.n_draws = (uint32_t)j.draws.size();
+    p.vis = sh->d_vis.as<int32_t>();
+    p.n_segs = segs;
+    p.seg_count = sh->d_seg.as<uint4>();
+    p.seg_first = (uint64_t*)(p.seg_count + segs);
+    p.seg_chunk = p.seg_first + segs;
+    p.totals = totals.as<uint64_t>();
+    p.entries = nullptr;
+    p.chunks = nullptr;
+    sh->n_chunks = 0;
+    if ((rc = launch_frag_count(p, sh->n_tris, s))) return rc;
+    HIP_TRY(hipStreamSynchronize(s));
+    totals.done();
+    const uint64_t n_entries = p.totals[0], n_chunks = p.totals[1];
+    if ((rc = sh->d_entries.reserve(std::max<uint64_t>(1, n_entries) * sizeof(uint4))) ||
+        (rc = sh->d_chunks.reserve(std::max<uint64_t>(1, n_chunks) * sizeof(uint4))) ||
+        (rc = sh->d_partial.reserve(std::max<uint64_t>(shade_blocks(sh->n_slots), bwd_blocks(n_chunks)) * 32 + 32)))
+        return rc;
+    p.entries = sh->d_entries.as<uint4>();
+    p.chunks = sh->d_chunks.as<uint4>();
+    if ((rc = launch_frag_fill(p, sh->n_tris, s))) return rc;
+    sh->n_chunks = n_chunks;
+    return SLOTH_OK;
+}
+
 // Renders the batch keeping (triangle << 1 | sub) per z slot.
 static int shading_visibility(sloth_shading* sh)
 {
@@ -1667,7 +1707,7 @@ static int shading_visibility(sloth_shading* sh)
     if (replanned) drop_graph(b);
     b->ran = true;
     b->checked = true;
-    return SLOTH_OK;
+    return shading_lists(sh);
 }
 
 extern "C" {
@@ -1691,19 +1731,13 @@ int sloth_shading_create(sloth_batch* b, const uint32_t* faces, uint32_t n_tris,
     sh->n_slots = j.n_z;
     std::vector<float> G(j.draws.size() * 9);
     for (size_t d = 0; d < j.draws.size(); ++d) normal_map(j.draws[d].M, &G[d * 9]);
-    const uint32_t nb = shade_blocks(sh->n_slots);
-    sh->partial.resize((size_t)nb * 4);
-    std::vector<uint64_t> tile_begin(j.frames.size() + 1);
-    bwd_tiles(j.frames.data(), (uint32_t)j.frames.size(), tile_begin.data());
-    sh->n_bwd_tiles = tile_begin.back();
-    if ((rc = sh->d_bwd_tile.reserve(tile_begin.size() * 8)) ||
-        (rc = sh->d_faces.reserve(std::max<size_t>(4, (size_t)n_tris * 12))) ||
+    if ((rc = sh->d_faces.reserve(std::max<size_t>(4, (size_t)n_tris * 12))) ||
         (rc = sh->d_vis.reserve(std::max<size_t>(4, sh->n_slots * 4))) ||
         (rc = sh->d_G.reserve(std::max<size_t>(4, G.size() * 4))) ||
         (rc = sh->d_vcolor.reserve(std::max<size_t>(4, (size_t)n_verts * 12))) ||
         (rc = sh->d_vnormal.reserve(std::max<size_t>(4, (size_t)n_verts * 12))) ||
         (rc = sh->d_light.reserve(16)) ||
-        (rc = sh->d_partial.reserve(std::max<size_t>(8, (size_t)nb * 32))) ||
+        (rc = sh->d_sum.reserve(32)) ||
         (rc = sh->d_vert_acc.reserve(std::max<size_t>(8, (size_t)n_verts * 6 * 8))) ||
         (rc = sh->d_dcolor.reserve(std::max<size_t>(4, (size_t)n_verts * 12))) ||
         (rc = sh->d_dnormal.reserve(std::max<size_t>(4, (size_t)n_verts * 12)))) {
@@ -1713,7 +1747,6 @@ int sloth_shading_create(sloth_batch* b, const uint32_t* faces, uint32_t n_tris,
     hipError_t e = hipSuccess;
     if (n_tris) e = hipMemcpy(sh->d_faces.p, faces, (size_t)n_tris * 12, hipMemcpyHostToDevice);
     if (e == hipSuccess && !G.empty()) e = hipMemcpy(sh->d_G.p, G.data(), G.size() * 4, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(sh->d_bwd_tile.p, tile_begin.data(), tile_begin.size() * 8, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         delete sh;
         return fail(SLOTH_EHIP, "shading upload: %s", hipGetErrorString(e));
@@ -1758,20 +1791,17 @@ int sloth_shading_set_target(sloth_shading* sh, const float* target)
     return SLOTH_OK;
 }
 
-// Copies the results out and sums the per-block partials (in order) into the
-// loss and the light gradient (either may be null).
+// Copies the results out, with the loss and the light gradient (either may
+// be null).
 static int shading_results(sloth_shading* sh, Span* spans, int n, double* loss, double* dlight)
 {
-    const uint32_t nb = sh->n_partials;
-    if (nb) spans[n++] = Span{sh->partial.data(), sh->d_partial.p, (size_t)nb * 32};
+    double sum[4];
+    spans[n++] = Span{sum, sh->d_sum.p, sizeof sum};
     int rc = copy_out(spans, n, sh->b->stream);
     if (rc) return rc;
-    double acc[4] = {0, 0, 0, 0};
-    for (uint32_t i = 0; i < nb; ++i)
-        for (int k = 0; k < 4; ++k) acc[k] += sh->partial[(size_t)i * 4 + k];
-    if (loss) *loss = acc[0];
+    if (loss) *loss = sum[0];
     if (dlight)
-        for (int k = 0; k < 3; ++k) dlight[k] = acc[k + 1];
+        for (int k = 0; k < 3; ++k) dlight[k] = sum[k + 1];
     return SLOTH_OK;
 }
 
@@ -1787,19 +1817,22 @@ static int shading_params(sloth_shading* sh, const float* vcolor, const float* v
     return SLOTH_OK;
 }
 
-// Backward launches (accumulator clear, per-tile backward with the loss,
-// conversion of the vertex sums) on the shading's stream.
+// Backward launches (the lists' pass with the loss, the sums, the conversion
+// of the vertex sums) on the shading's stream.
 static int shading_backward_launch(sloth_shading* sh)
 {
     hipStream_t s = sh->b->stream;
     const ShadeArgs a = shade_args(sh, true, nullptr);
-    int rc = launch_shade(a, true, s);
-    if (rc) return rc;
-    sh->n_partials = bwd_blocks(sh->n_slots, sh->n_bwd_tiles);
-    return launch_shade_finish(a, sh->d_dcolor.as<float>(), sh->d_dnormal.as<float>(), s);
+    int rc;
+    if (!sh->acc_zero && (rc = launch_shade_zero(a, s))) return rc;
+    sh->acc_zero = false;
+    if ((rc = launch_shade_bwd(a, sh->d_dcolor.as<float>(), sh->d_dnormal.as<float>(), sh->d_sum.as<double>(), s)))
+        return rc;
+    sh->acc_zero = true;
+    return SLOTH_OK;
 }
 
-// Copies the gradients out and sums the per-block loss and light partials.
+// Copies the gradients, the loss and the light gradient out.
 static int shading_gradients(sloth_shading* sh, double* loss, float* d_vcolor, float* d_vnormal, float* d_light)
 {
     Span v[3];
@@ -1830,8 +1863,7 @@ int sloth_shading_forward(sloth_shading* sh, const float* vcolor, const float* v
         d_out = sh->d_out.as<float>();
         HIP_TRY(hipMemsetAsync(sh->d_out.p, 0, sh->n_slots * 12, s));
     }
-    if ((rc = launch_shade(shade_args(sh, sh->has_target, d_out), false, s))) return rc;
-    sh->n_partials = shade_blocks(sh->n_slots);
+    if ((rc = launch_shade_fwd(shade_args(sh, sh->has_target, d_out), sh->d_sum.as<double>(), s))) return rc;
     Span v[2];
     int n = 0;
     if (out_rgb) v[n++] = Span{out_rgb, sh->d_out.p, sh->n_slots * 12};

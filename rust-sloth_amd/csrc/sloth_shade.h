@@ -25,17 +25,42 @@ struct ShadeArgs {
     double* vert_acc;         // [n_verts][6]: d color, d normal (binary64 sums)
     uint64_t n_slots;
     uint32_t n_tris, n_verts;
-    const uint64_t* bwd_tile_begin;   // per frame (+1): first backward tile
-    uint64_t n_bwd_tiles;
+    const uint4* entries;     // fragment lists (k_frag_plan)
+    const uint4* chunks;
+    uint64_t n_chunks;
+    uint32_t chunks_per_block;
+};
+
+// The fragment lists: which pixels of each triangle are visible.
+struct FragPlan {
+    const Frame* frames;
+    const Draw* draws;
+    uint32_t n_draws;
+    const int32_t* vis;
+    uint64_t n_segs;
+    uint4* seg_count;         // per segment: entries of its wavefronts
+    uint64_t* seg_first;      // its first entry
+    uint64_t* seg_chunk;      // its first chunk
+    uint64_t* totals;         // entries, chunks (host memory)
+    uint4* entries;
+    uint4* chunks;
 };
 
 uint32_t shade_blocks(uint64_t n_slots);
-// workgroups (and per-block partial sums) of the backward pass
-uint32_t bwd_blocks(uint64_t n_slots, uint64_t n_bwd_tiles);
-// Backward tiles per frame, prefix-summed: begin[0..n_frames]
-void bwd_tiles(const Frame* frames, uint32_t n_frames, uint64_t* begin);
-int launch_shade(const ShadeArgs& a, bool backward, hipStream_t s);
-// binary64 vertex sums -> binary32 gradients
-int launch_shade_finish(const ShadeArgs& a, float* d_color, float* d_normal, hipStream_t s);
+uint64_t frag_segments(uint32_t n_tris, uint32_t n_draws);
+// chunks per workgroup of the backward pass, and its workgroups (per-block
+// partial sums)
+uint32_t bwd_chunks_per_block(uint64_t n_chunks);
+uint32_t bwd_blocks(uint64_t n_chunks);
+// Entries of every segment, their offsets and totals; then the lists.  Every
+// draw has n_tris triangles.
+int launch_frag_count(const FragPlan& p, uint32_t n_tris, hipStream_t s);
+int launch_frag_fill(const FragPlan& p, uint32_t n_tris, hipStream_t s);
+// sum: loss, and from the backward pass the light gradient
+int launch_shade_fwd(const ShadeArgs& a, double* sum, hipStream_t s);
+// vert_acc to zero
+int launch_shade_zero(const ShadeArgs& a, hipStream_t s);
+// vert_acc is zero before and after
+int launch_shade_bwd(const ShadeArgs& a, float* d_color, float* d_normal, double* sum, hipStream_t s);
 
 }  // namespace sloth
