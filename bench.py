@@ -10,7 +10,7 @@ Workload (a "step" = one pass of the raster path over the whole sweep):
   run before the warmup.
 
 Forms timed:
-  batched  all 256 frames by one launch sequence captured in a HIP graph
+  batched  all 256 frames by one launch sequence
            (sloth_batch_run)                                  -> `value`
   plain    one launch sequence per frame, device sync after each
   cpu      the oracle (C restatement of the reference) on a bounded sample of
@@ -117,7 +117,7 @@ def main() -> int:
     ap.add_argument("--uneven-only", default=None, metavar="WxH,WALK,TPT",
                     help="only the uneven-batch leg, at this plan instead of the autotuner's (for profilers)")
     ap.add_argument("--graph-only", action="store_true",
-                    help="only the batched graph renders (for profilers): no plain, stage, CPU or other legs")
+                    help="only the batched renders (for profilers): no plain, stage, CPU or other legs")
     ap.add_argument("--no-extra", action="store_true", help="skip the 4K, uneven-batch and shading legs")
     args = ap.parse_args()
     if args.graph_only:
@@ -172,7 +172,7 @@ def main() -> int:
         tune_s = time.perf_counter() - t0
     plan = batch.plan()
 
-    log("bench: batched (graph) timing")
+    log("bench: batched timing")
     ms = batch.time(args.steps, args.warmup, per_frame=False)
     ms_step = ms / args.steps
     fps = F / (ms_step / 1e3)
@@ -188,7 +188,7 @@ def main() -> int:
         pms = batch.time(args.plain_steps, 1, per_frame=True)
         plain_fps = F / (pms / args.plain_steps / 1e3)
 
-    # leave the batch holding one graph render for the parity spot check
+    # leave the batch holding one batched render for the parity spot check
     batch.run()
     batch.sync()
 
@@ -289,7 +289,7 @@ def main() -> int:
         "dtype": "f32",
         "data": "synthetic",
         "config": {"workload": f"sweep_1080p: displaced icosphere s7 ({N} tris, seed 2), {F} frames "
-                               f"1920x1080 image mode, turntable schedule, one HIP graph per sweep",
+                               f"1920x1080 image mode, turntable schedule, one launch sequence per sweep",
                    "frames": F, "triangles": N, "width": W, "height": H},
         "plan": dict(plan, autotune_s=round(tune_s, 2) if tune_s else None),
         "ms_per_step_median": round(ms_median, 4),
@@ -321,7 +321,7 @@ def _frac(alg_bytes, ms):
 def leg_4k(sloth_amd, meshgen, args):
     """One 3840x2160 frame of the 8-subdivision displaced icosphere
     (1,310,720 triangles, seed 1): plain form (launch sequence + sync) and
-    graph replay, median of 5 timings of 10 frames each."""
+    batched form (the keys `_graph`), median of 5 timings of 10 frames each."""
     log("bench: 4K frame leg")
     m, W, H, U, R = meshgen.workload_icosphere_4k()
     mesh = sloth_amd.SimpleMesh.from_mesh(m)

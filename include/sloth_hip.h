@@ -229,14 +229,14 @@ int sloth_batch_create(const sloth_frame_desc *frames, uint32_t n_frames, const 
  * sloth_batch_run / _run_per_frame; reading before that returns SLOTH_ESTATE.
  * If the new transforms need longer tile lists than the ones sized so far,
  * the next synchronising call (sloth_batch_sync, _read_frame, _encode_frame)
- * re-sizes them, renders again and re-captures the graph at the next run. */
+ * re-sizes them and renders again. */
 int sloth_batch_set_transforms(sloth_batch *b, const float *transforms16);
 
-/* Renders all frames on `stream` (NULL = the batch's own stream).  The first
- * call captures the launch sequence into a HIP graph; later calls replay it.
- * Returns without waiting.  On a caller's stream the launch waits for the
- * batch's own pending work, and the batch's stream waits for the launch, so
- * the synchronising calls below also wait for it. */
+/* Renders all frames on `stream` (NULL = the batch's own stream), by one
+ * launch sequence for all of them.  Returns without waiting.  On a caller's
+ * stream the launch waits for the batch's own pending work, and the batch's
+ * stream waits for the launch, so the synchronising calls below also wait for
+ * it. */
 int sloth_batch_run(sloth_batch *b, void *stream);
 
 /* Renders every frame with one launch sequence per frame and a device
@@ -268,7 +268,7 @@ int sloth_batch_encode_export(sloth_batch *b, uint32_t first, uint32_t count, in
  * 256-byte boundary) and z (W*H). */
 int sloth_batch_device_frame(sloth_batch *b, uint32_t frame, uint32_t **d_cells, float **d_z);
 
-/* Times each stage of one (non-graph) run with HIP events on the batch's
+/* Times each stage of one run with HIP events on the batch's
  * stream: out_ms[i] = milliseconds of stage i, names[i] its kernel name;
  * *n_stages in: capacity, out: count.  On the tiled path the first stage
  * (k_tile_clear) runs only for batches with frames of odd width; otherwise
@@ -276,7 +276,7 @@ int sloth_batch_device_frame(sloth_batch *b, uint32_t frame, uint32_t **d_cells,
 int sloth_batch_profile(sloth_batch *b, float *out_ms, const char **names, uint32_t *n_stages);
 
 /* Runs `warmup` untimed renders, then `steps` timed renders bracketed by HIP
- * events on the batch's stream, and waits.  mode 0: graph replay
+ * events on the batch's stream, and waits.  mode 0: batched
  * (sloth_batch_run); mode 1: one launch sequence per frame with a device
  * synchronisation after each (sloth_batch_run_per_frame).  *ms = elapsed
  * milliseconds of the timed renders. */
@@ -304,10 +304,11 @@ int sloth_batch_set_bin(sloth_batch *b, uint32_t tris_per_thread);
 
 /* Renders the batch with each candidate tile size that fits -- 16, 32, 64,
  * 128, 256 or 512 cells (8..256 logical pixels) wide by 8, 16, 32 or 64 rows
- * -- timed with HIP events as the least of three runs of 3 graph renders
- * each, keeps the fastest, then times the tile raster with and without the
+ * -- timed with HIP events as the least of three runs of 3 renders each,
+ * keeps the fastest, then times the tile raster with and without the
  * wavefront walk of big boxes at that size and keeps the faster, then the
- * binning kernel with 4, 2 and 1 triangles per thread.  The choice is remembered for batches of the same
+ * binning kernel with 4, 2 and 1 triangles per thread.  The choice is
+ * remembered for batches of the same
  * class (frame sizes, cell count and log2 of the triangle count) in this
  * process and reused without timing.  Writes the chosen size to tile_w /
  * tile_h (may be NULL; 0 for batches on the general path, which has no

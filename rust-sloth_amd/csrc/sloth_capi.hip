@@ -2,8 +2,8 @@
 //
 // A "job" is a set of frames (Contexts) and their draw_mesh calls, laid out in
 // device tables (Frame, Draw, Ramp) plus the output buffers of all frames.
-// A context is a job with one frame; a batch is a job with many, whose launch
-// sequence is captured once into a HIP graph and replayed.
+// A context is a job with one frame; a batch is a job with many, rendered by
+// one launch sequence.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -312,7 +312,7 @@ struct Job {
             if ((rc = d_keys.reserve(sizeof(uint64_t) * n_z))) return rc;
             if ((rc = d_nl.reserve(sizeof(int32_t) * std::max<uint64_t>(1, n_rows)))) return rc;
         } else {
-            if ((rc = tiled.plan(frames, n_rows))) return rc;
+            if ((rc = tiled.plan(frames, draws, n_rows))) return rc;
         }
         laid_out = true;
         return SLOTH_OK;
@@ -324,8 +324,8 @@ struct Job {
         return e && e[0] == '1';
     }
 
-    // SLOTH_PIPELINE=1 captures batch graphs as a two-stream pipeline of
-    // frame groups (bins of one group beside the raster of the previous one).
+    // SLOTH_PIPELINE=1 launches batches as a two-stream pipeline of frame
+    // groups (bins of one group beside the raster of the previous one).
     // Off by default: measured slower than one stream on the 1080p sweep.
     static bool pipeline()
     {
@@ -406,8 +406,8 @@ struct Job {
         return SLOTH_OK;
     }
 
-    // Work that must precede a launch and cannot be captured in a graph: the
-    // counting run that sizes the tile lists.
+    // Work that must precede a launch and waits for the device: the counting
+    // run that sizes the tile lists.
     int prepare(hipStream_t s)
     {
         if (path == PATH_TILED && !tiled.sized)
@@ -591,20 +591,15 @@ struct sloth_batch {
     Job job;
     std::vector<float> U;       // per frame utransform
     hipStream_t stream = nullptr;
-    hipStream_t stream2 = nullptr;       // second branch of the captured pipeline
+    hipStream_t stream2 = nullptr;       // second branch of the pipelined launch
     std::vector<hipEvent_t> join;        // its fork / join events
     hipEvent_t join_ev = nullptr;        // joins a caller's stream to `stream`
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    uint64_t exec_generation = 0;   // tile plan generation the graph was captured with
     bool ran = false;
     std::vector<bool> win_valid;
     bool checked = false;           // the last render was checked for tile-list overflow
     Encoder enc;
     ~sloth_batch()
     {
-        if (exec) (void)hipGraphExecDestroy(exec);
-        if (graph) (void)hipGraphDestroy(graph);
         for (hipEvent_t e : join)
             if (e) (void)hipEventDestroy(e);
         if (join_ev) (void)hipEventDestroy(join_ev);
@@ -1186,22 +1181,10 @@ int sloth_batch_set_transforms(sloth_batch* b, const float* transforms16)
     return SLOTH_OK;
 }
 
-static void drop_graph(sloth_batch* b)
-{
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
-    b->exec = nullptr;
-    b->graph = nullptr;
-}
-
 // Checks the finished renders for tile-list overflow and re-renders if needed.
 static int batch_finish(sloth_batch* b)
 {
-    bool replanned = false;
-    int rc = b->job.finish(0, (uint32_t)b->job.frames.size(), b->stream, nullptr, &replanned);
-    if (rc) return rc;
-    if (replanned) drop_graph(b);
-    return SLOTH_OK;
+    return b->job.finish(0, (uint32_t)b->job.frames.size(), b->stream, nullptr);
 }
 
 int sloth_batch_run(sloth_batch* b, void* stream)
@@ -1211,25 +1194,14 @@ int sloth_batch_run(sloth_batch* b, void* stream)
     if (rc) return rc;
     hipStream_t s = stream ? (hipStream_t)stream : b->stream;
     if ((rc = b->job.prepare(b->stream))) return rc;
-    if (b->exec && b->exec_generation != b->job.tiled.generation) drop_graph(b);
-    if (!b->exec) {
-        HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        const bool pipe = Job::pipeline();
-        rc = b->job.launch(0, (uint32_t)b->job.frames.size(), b->stream, nullptr, nullptr, false,
-                           pipe ? b->stream2 : nullptr, pipe ? &b->join : nullptr);
-        hipGraph_t g = nullptr;
-        hipError_t e = hipStreamEndCapture(b->stream, &g);
-        if (rc) {
-            if (g) (void)hipGraphDestroy(g);
-            return rc;
-        }
-        if (e != hipSuccess) return fail(SLOTH_EHIP, "graph capture: %s", hipGetErrorString(e));
-        b->graph = g;
-        HIP_TRY(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
-        b->exec_generation = b->job.tiled.generation;
-    }
     if ((rc = join_streams(b->stream, s, b->join_ev))) return rc;
-    HIP_TRY(hipGraphLaunch(b->exec, s));
+    // three or four kernels: launched one by one they cost the host less than
+    // a graph of them (12 against 16 us) and start on the device 5 us sooner
+    // (32 frames of 320x240: 22.8 us a render against 27.5 replayed)
+    const bool pipe = Job::pipeline();
+    if ((rc = b->job.launch(0, (uint32_t)b->job.frames.size(), s, nullptr, nullptr, false, pipe ? b->stream2 : nullptr,
+                            pipe ? &b->join : nullptr)))
+        return rc;
     if ((rc = join_streams(s, b->stream, b->join_ev))) return rc;
     b->ran = true;
     b->checked = false;
@@ -1282,10 +1254,8 @@ int sloth_batch_read_frame(sloth_batch* b, uint32_t frame, uint32_t* cells, floa
         if ((rc = b->job.ensure_win())) return rc;
         if ((rc = b->job.launch(frame, frame + 1, s, b->job.d_win.as<int32_t>()))) return rc;
         // the lists were sized for these transforms by the checked run, but a
-        // re-plan here must still re-render the frame and drop the graph
-        bool replanned = false;
-        if ((rc = b->job.finish(frame, frame + 1, s, b->job.d_win.as<int32_t>(), &replanned))) return rc;
-        if (replanned) drop_graph(b);
+        // re-plan here must still re-render the frame
+        if ((rc = b->job.finish(frame, frame + 1, s, b->job.d_win.as<int32_t>()))) return rc;
         b->win_valid[frame] = true;
     }
     Span v[3];
@@ -1370,17 +1340,14 @@ int sloth_batch_profile(sloth_batch* b, float* out_ms, const char** names, uint3
     bool replanned = false;
     if ((rc = b->job.finish(0, (uint32_t)b->job.frames.size(), b->stream, nullptr, &replanned))) return rc;
     b->checked = true;
-    if (replanned) {
-        drop_graph(b);
-        return fail(SLOTH_ESTATE, "tile lists were re-sized during profiling; profile again");
-    }
+    if (replanned) return fail(SLOTH_ESTATE, "tile lists were re-sized during profiling; profile again");
     return SLOTH_OK;
 }
 
 int sloth_batch_time(sloth_batch* b, uint32_t steps, uint32_t warmup, int mode, float* ms)
 {
     ARG_CHECK(b && ms, "null argument");
-    ARG_CHECK(mode == 0 || mode == 1, "mode must be 0 (graph) or 1 (per frame)");
+    ARG_CHECK(mode == 0 || mode == 1, "mode must be 0 (batched) or 1 (per frame)");
     int rc = ensure_device();
     if (rc) return rc;
     for (int attempt = 0; attempt < 3; ++attempt) {
@@ -1408,7 +1375,7 @@ int sloth_batch_time(sloth_batch* b, uint32_t steps, uint32_t warmup, int mode, 
             *ms = t;
             return SLOTH_OK;
         }
-        drop_graph(b);   // tile lists were re-sized: the timed renders were redone; time again
+        // tile lists were re-sized: the timed renders were redone; time again
     }
     return fail(SLOTH_ESTATE, "tile lists kept re-sizing while timing");
 }
@@ -1420,7 +1387,6 @@ int sloth_batch_set_tile(sloth_batch* b, uint32_t tile_w, uint32_t tile_h)
     if (rc) return rc;
     if (!b->job.tiled.sized) {
         if ((rc = b->job.layout(b->stream)) || (rc = b->job.upload(b->stream))) return rc;
-        drop_graph(b);
         b->ran = false;
     }
     return SLOTH_OK;
@@ -1503,7 +1469,7 @@ int sloth_batch_autotune(sloth_batch* b, uint32_t* tile_w, uint32_t* tile_h)
     // Tiles of 8..256 logical pixels wide (a logical pixel is two cells
     // wide) by 8..64 rows: 16..512 cells by 8..64 rows, those the raster's
     // workgroup can take.  Each candidate is timed as the
-    // least of three runs of 3 graph renders, after one untimed render (which
+    // least of three runs of 3 renders, after one untimed render (which
     // also sizes the lists): single runs differ by a few per cent, as much
     // as neighbouring candidates do.
     auto time_it = [&](float& ms) -> int {
@@ -1701,10 +1667,7 @@ static int shading_visibility(sloth_shading* sh)
     if ((rc = j.prepare(b->stream))) return rc;
     if ((rc = j.launch(0, (uint32_t)j.frames.size(), b->stream, sh->d_vis.as<int32_t>(), nullptr, true))) return rc;
     HIP_TRY(hipStreamSynchronize(b->stream));
-    bool replanned = false;
-    if ((rc = j.finish(0, (uint32_t)j.frames.size(), b->stream, sh->d_vis.as<int32_t>(), &replanned, true)))
-        return rc;
-    if (replanned) drop_graph(b);
+    if ((rc = j.finish(0, (uint32_t)j.frames.size(), b->stream, sh->d_vis.as<int32_t>(), nullptr, true))) return rc;
     b->ran = true;
     b->checked = true;
     return shading_lists(sh);

@@ -65,7 +65,6 @@ struct TiledPlan {
     uint64_t n_tiles = 0;
     uint64_t n_rows = 0;
     bool sized = false;              // pool offsets match the current layout
-    uint64_t generation = 0;         // bumped whenever size() runs (device pointers may change)
     std::vector<uint64_t> off;       // host copy of the per-tile pool offsets (n_tiles + 1)
     DevBuf d_cursor, d_off, d_pool, d_nl;
     uint32_t* overflow = nullptr;    // per frame, the job's pinned memory: kernels write it (rarely), the host reads it after a wait
@@ -100,27 +99,32 @@ struct TiledPlan {
     // wavefront walk of big boxes (set by the autotuner)
     int walk_force = -1;
 
+    // What a launch over frames [f_lo, f_hi) needs to know of them; that of
+    // the whole job is made by plan(), so that launching it does not look at
+    // every frame and draw again.
+    struct Range {
+        uint32_t max_draw = 0;                     // triangles of the largest draw
+        uint32_t tiles_x = 0, tiles_y = 0, H = 0;  // of the largest frame, each
+        bool one = true;                           // every frame has exactly one draw
+        bool even = false, odd = false;            // width parities
+    };
+    Range whole;
+    uint32_t n_frames = 0;
+    Range range(const std::vector<Frame>& frames, const std::vector<Draw>& draws, uint32_t f_lo, uint32_t f_hi) const;
+
     // Sets the tile grid of every frame and allocates per-tile and per-row
     // state.  Pool offsets become invalid until size() runs.
-    int plan(std::vector<Frame>& frames, uint64_t rows);
+    int plan(std::vector<Frame>& frames, const std::vector<Draw>& draws, uint64_t rows);
 
     // Tile size in cells: TW a power of two in 8..512, TH in 4..64.
     int set_tile(uint32_t tw, uint32_t th);
     // The raster variant the next launches use (-1 = the sizing run's choice).
-    void set_walk(int mode)
-    {
-        if (mode != walk_force) ++generation;   // captured graphs hold the old variant
-        walk_force = mode;
-    }
+    void set_walk(int mode) { walk_force = mode; }
     // the even-width instance's variant (the odd one has no big-box walk)
     bool walk() const { return has_even && (walk_force >= 0 ? walk_force == 1 : big_walk); }
     // Triangles per thread of k_bin: 1, 2 or 4 (set by the autotuner).
     int bin_tpt = 4;
-    void set_bin_tpt(int t)
-    {
-        if (t != bin_tpt) ++generation;   // captured graphs hold the old launch
-        bin_tpt = t;
-    }
+    void set_bin_tpt(int t) { bin_tpt = t; }
     // LDS of the even- or odd-width raster instance at the current tile size
     size_t raster_lds(bool odd) const;
     // Both parities' instances the job needs can take the current tile size
@@ -152,7 +156,7 @@ struct TiledPlan {
     int launch_bin(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
                    const Draw* d_draws, uint32_t f_lo, uint32_t f_hi, bool count_only, hipStream_t s);
     int launch_careful(const Frame* d_frames, const Draw* d_draws, bool count_only, uint32_t group, hipStream_t s);
-    int launch_raster(const std::vector<Frame>& frames, const Frame* d_frames, const Draw* d_draws,
+    int launch_raster(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames, const Draw* d_draws,
                       const Ramp* d_ramps, uint32_t f_lo, uint32_t f_hi, uint32_t* cells, float* z, int32_t* win,
                       bool win_raw, uint32_t n_ramps, bool reset_careful, hipStream_t s);
 };

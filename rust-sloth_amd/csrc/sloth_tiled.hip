@@ -1377,7 +1377,24 @@ bool TiledPlan::tile_fits() const
     return (!has_even || fits(false)) && (!has_odd || fits(true));
 }
 
-int TiledPlan::plan(std::vector<Frame>& frames, uint64_t rows)
+TiledPlan::Range TiledPlan::range(const std::vector<Frame>& frames, const std::vector<Draw>& draws, uint32_t f_lo,
+                                  uint32_t f_hi) const
+{
+    if (f_lo == 0 && f_hi == n_frames) return whole;
+    Range r;
+    for (uint32_t f = f_lo; f < f_hi; ++f) {
+        const Frame& fr = frames[f];
+        r.tiles_x = std::max(r.tiles_x, fr.tiles_x);
+        r.tiles_y = std::max(r.tiles_y, fr.tiles_y);
+        r.H = std::max(r.H, fr.H);
+        r.one = r.one && fr.draw_end - fr.draw_begin == 1;
+        ((fr.W & 1u) ? r.odd : r.even) = true;
+        for (uint32_t d = fr.draw_begin; d < fr.draw_end; ++d) r.max_draw = std::max(r.max_draw, draws[d].n);
+    }
+    return r;
+}
+
+int TiledPlan::plan(std::vector<Frame>& frames, const std::vector<Draw>& draws, uint64_t rows)
 {
     bool ev = false, od = false;
     for (const Frame& f : frames) ((f.W & 1u) ? od : ev) = true;
@@ -1393,6 +1410,9 @@ int TiledPlan::plan(std::vector<Frame>& frames, uint64_t rows)
         f.tile_begin = tiles;
         tiles += (uint64_t)f.tiles_x * f.tiles_y;
     }
+    n_frames = UINT32_MAX;   // not the whole, while that is made
+    whole = range(frames, draws, 0, (uint32_t)frames.size());
+    n_frames = (uint32_t)frames.size();
     if (tiles != n_tiles) sized = false;
     n_tiles = tiles;
     n_rows = rows;
@@ -1451,10 +1471,9 @@ int TiledPlan::launch_bin(const std::vector<Frame>& frames, const std::vector<Dr
         return SLOTH_OK;
     }
     int rc;
+    const uint32_t max_n = range(frames, draws, f_lo, f_hi).max_draw;
     for (uint32_t d0 = d_lo; d0 < d_hi; d0 += 65535u) {
         const uint32_t d1 = std::min(d_hi, d0 + 65535u);
-        uint32_t max_n = 0;
-        for (uint32_t d = d0; d < d1; ++d) max_n = std::max(max_n, draws[d].n);
         if (max_n == 0) continue;
         if ((rc = go(dim3(blocks(max_n, BIN_BLOCK * (uint32_t)bin_tpt), d1 - d0), d0, nullptr))) return rc;
     }
@@ -1529,10 +1548,8 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     // in 256 spans more than TALL_ROWS rows (a wavefront's row loop lasts as
     // long as its tallest triangle's)
     const bool tree = (uint64_t)cnt[TALL_CNT] * 256 >= n_tri && cnt[TALL_CNT] > 0;
-    bool want_tree = tree;
-    if (const char* e = getenv("SLOTH_BIN_TREE")) want_tree = e[0] == '1';
-    if (want_tree != bin_tree) ++generation;   // captured graphs hold the other variant
-    bin_tree = want_tree;
+    bin_tree = tree;
+    if (const char* e = getenv("SLOTH_BIN_TREE")) bin_tree = e[0] == '1';
     if (n_careful > careful_cap) {
         // 2. room for the careful list, then count again so that it is filled
         careful_cap = n_careful + n_careful / 4 + 256;
@@ -1586,7 +1603,6 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     if ((rc = launch_clear(frames, 0, F, s))) return rc;
     HIP_TRY(hipStreamSynchronize(s));
     sized = true;
-    ++generation;
     return SLOTH_OK;
 }
 
@@ -1604,8 +1620,8 @@ static auto raster_kernel(bool walk, bool one)
                     : (one ? k_tile_raster<false, true, false, FLAT> : k_tile_raster<false, false, false, FLAT>);
 }
 
-int TiledPlan::launch_raster(const std::vector<Frame>& frames, const Frame* d_frames, const Draw* d_draws,
-                             const Ramp* d_ramps, uint32_t f_lo, uint32_t f_hi, uint32_t* cells, float* z, int32_t* win,
+int TiledPlan::launch_raster(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
+                             const Draw* d_draws, const Ramp* d_ramps, uint32_t f_lo, uint32_t f_hi, uint32_t* cells, float* z, int32_t* win,
                              bool win_raw, uint32_t n_ramps, bool reset_careful, hipStream_t s)
 {
     // the first raster launch resets the careful list's length (k_careful
@@ -1615,18 +1631,10 @@ int TiledPlan::launch_raster(const std::vector<Frame>& frames, const Frame* d_fr
     // at most 65535 frames per launch
     for (uint32_t f0 = f_lo; f0 < f_hi; f0 += 65535u) {
         const uint32_t f1 = std::min(f_hi, f0 + 65535u);
-        uint32_t mx = 0, my = 0;
-        for (uint32_t f = f0; f < f1; ++f) {
-            mx = std::max(mx, frames[f].tiles_x);
-            my = std::max(my, frames[f].tiles_y);
-        }
+        const Range rg = range(frames, draws, f0, f1);
+        const uint32_t mx = rg.tiles_x, my = rg.tiles_y;
         if (mx == 0 || my == 0) continue;
-        bool one = true;   // every frame of the range has exactly one draw
-        bool ev = false, od = false;
-        for (uint32_t f = f0; f < f1; ++f) {
-            one = one && frames[f].draw_end - frames[f].draw_begin == 1;
-            ((frames[f].W & 1u) ? od : ev) = true;
-        }
+        const bool one = rg.one, ev = rg.even, od = rg.odd;
         // one launch per width parity in the range; each skips the other's
         // frames.  The grid: (tile x, tile y, frame) over the largest tile
         // grid, or one workgroup per tile when the frames' tile grids differ
@@ -1656,9 +1664,7 @@ int TiledPlan::launch_raster(const std::vector<Frame>& frames, const Frame* d_fr
                                d_edges.as<uint4>(), careful_reset, tf, (uint32_t)t_lo);
             HIP_TRY(hipGetLastError());
             careful_reset = nullptr;
-            uint32_t mh = 0;
-            for (uint32_t f = f0; f < f1; ++f) mh = std::max(mh, frames[f].H);
-            hipLaunchKernelGGL(k_tile_edges, dim3(blocks(mh, 256), mx, f1 - f0), dim3(256), 0, s, d_frames, f0,
+            hipLaunchKernelGGL(k_tile_edges, dim3(blocks(rg.H, 256), mx, f1 - f0), dim3(256), 0, s, d_frames, f0,
                                log2u(TW), log2u(TH), (const uint4*)d_edges.as<uint4>(),
                                (const int32_t*)d_nl.as<int32_t>(), cells);
             HIP_TRY(hipGetLastError());
@@ -1689,8 +1695,7 @@ int TiledPlan::launch(const std::vector<Frame>& frames, const std::vector<Draw>&
         // (k_tile_raster resets what it has read; size() ends with a
         // clear), so only ranges with odd widths, whose newline rows
         // k_tile_edges reads after the raster, are cleared first.
-        bool odd = false;
-        for (uint32_t f = f_lo; f < f_hi; ++f) odd = odd || (frames[f].W & 1u);
+        const bool odd = range(frames, draws, f_lo, f_hi).odd;
         if (ev) HIP_TRY(hipEventRecord((*ev)[0], s));
         if (odd && (rc = launch_clear(frames, f_lo, f_hi, s))) return rc;
         if (ev) HIP_TRY(hipEventRecord((*ev)[1], s));
@@ -1698,7 +1703,7 @@ int TiledPlan::launch(const std::vector<Frame>& frames, const std::vector<Draw>&
         if (ev) HIP_TRY(hipEventRecord((*ev)[2], s));
         if ((rc = launch_careful(d_frames, d_draws, false, 0, s))) return rc;
         if (ev) HIP_TRY(hipEventRecord((*ev)[3], s));
-        if ((rc = launch_raster(frames, d_frames, d_draws, d_ramps, f_lo, f_hi, cells, z, win, win_raw, n_ramps, true,
+        if ((rc = launch_raster(frames, draws, d_frames, d_draws, d_ramps, f_lo, f_hi, cells, z, win, win_raw, n_ramps, true,
                                 s)))
             return rc;
         if (ev) HIP_TRY(hipEventRecord((*ev)[4], s));
@@ -1716,7 +1721,7 @@ int TiledPlan::launch(const std::vector<Frame>& frames, const std::vector<Draw>&
         HIP_TRY(hipEventRecord((*join)[g], s));
         HIP_TRY(hipStreamWaitEvent(s2, (*join)[g], 0));
         // the last group's raster runs after every group's careful pass
-        if ((rc = launch_raster(frames, d_frames, d_draws, d_ramps, a, b, cells, z, win, win_raw, n_ramps,
+        if ((rc = launch_raster(frames, draws, d_frames, d_draws, d_ramps, a, b, cells, z, win, win_raw, n_ramps,
                                 g + 1 == groups, s2)))
             return rc;
     }

@@ -553,7 +553,7 @@ class DrawSpec:
 
 
 class Batch:
-    """Many frames rendered by one launch sequence (captured in a HIP graph)."""
+    """Many frames rendered by one launch sequence."""
 
     def __init__(self, frames: list, draws: list, shader: Shader = default_shader):
         _ensure_init()
