@@ -79,6 +79,7 @@ struct TiledPlan {
     // k_bin takes one block per (draw, BIN_BLOCK * TPT triangles) from a
     // table per TPT, the raster one workgroup per tile of the range.
     bool flat_bin = false, flat_raster = false;
+    std::vector<uint32_t> flat_draws;            // the draws' sizes that the flat_bin tables are of
     DevBuf d_bin_blocks[3];                      // per TPT 1, 2, 4: (draw, first triangle) of each block
     std::vector<uint64_t> bin_block_begin[3];    // per TPT: each draw's first block (draws + 1)
     // flat raster grids: workgroup i of a launch over tiles [t_lo, t_hi) takes

@@ -1410,6 +1410,10 @@ int TiledPlan::plan(std::vector<Frame>& frames, const std::vector<Draw>& draws, 
         f.tile_begin = tiles;
         tiles += (uint64_t)f.tiles_x * f.tiles_y;
     }
+    // a context's draws may have changed since the tables were made: the
+    // padded grid takes any
+    flat_bin = flat_bin && flat_draws.size() == draws.size();
+    for (size_t d = 0; flat_bin && d < draws.size(); ++d) flat_bin = draws[d].n == flat_draws[d];
     n_frames = UINT32_MAX;   // not the whole, while that is made
     whole = range(frames, draws, 0, (uint32_t)frames.size());
     n_frames = (uint32_t)frames.size();
@@ -1514,6 +1518,8 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     flat_bin = false;
     for (const Draw& d : draws) flat_bin = flat_bin || d.n != draws[0].n;
     if (flat_bin) {
+        flat_draws.resize(draws.size());
+        for (size_t d = 0; d < draws.size(); ++d) flat_draws[d] = draws[d].n;
         for (int ti = 0; ti < 3; ++ti) {
             const uint32_t per = (uint32_t)BIN_BLOCK << ti;
             std::vector<uint2> tbl;
