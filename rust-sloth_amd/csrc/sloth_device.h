@@ -65,7 +65,7 @@ struct Tri {
     float x1, y1, z1, x2, y2, z2, x3, y3, z3;
     float A0, B0, A1, B1, A2, B2;   // edge deltas of orient(v2,v3,.), orient(v3,v1,.), orient(v1,v2,.)
     float a;                        // 1 / orient(v1,v2,v3)      rasterizer.rs:67
-    float minx, maxx;               // the vertices' x extent
+    float minx, maxx, miny, maxy;   // the vertices' extent
     int x0, x1d, y0, y1d;           // pixel domain [x0,x1d) x [y0,y1d)  rasterizer.rs:58-66
 };
 
@@ -125,12 +125,12 @@ __device__ __forceinline__ void tri_finish(uint32_t W, uint32_t H, Tri& t)
 {
     t.minx = fminf(t.x1, fminf(t.x2, t.x3));
     t.maxx = fmaxf(t.x1, fmaxf(t.x2, t.x3));
-    const float miny = fminf(t.y1, fminf(t.y2, t.y3));
-    const float maxy = fmaxf(t.y1, fmaxf(t.y2, t.y3));
+    t.miny = fminf(t.y1, fminf(t.y2, t.y3));
+    t.maxy = fmaxf(t.y1, fmaxf(t.y2, t.y3));
     t.x0 = sat_index(ceilf(fmaxf(t.minx, 1.0f)));
-    t.y0 = sat_index(ceilf(fmaxf(miny, 1.0f)));
+    t.y0 = sat_index(ceilf(fmaxf(t.miny, 1.0f)));
     t.x1d = sat_index(ceilf(fminf(t.maxx * 2.0f, (float)(W - 1))));
-    t.y1d = sat_index(ceilf(fminf(maxy, (float)(H - 1))));
+    t.y1d = sat_index(ceilf(fminf(t.maxy, (float)(H - 1))));
     t.A0 = t.x3 - t.x2;
     t.B0 = t.y3 - t.y2;
     t.A1 = t.x1 - t.x3;
@@ -141,24 +141,33 @@ __device__ __forceinline__ void tri_finish(uint32_t W, uint32_t H, Tri& t)
     t.a = 1.0f / o;
 }
 
-__device__ __forceinline__ void setup_tri(const float* M, const float* pv, uint32_t W, uint32_t H, Tri& t)
-{
-    setup_tri_from(M, global_ptr(pv), W, H, t);
-}
-
-// Triangle `local` of a draw: a soup's 9 consecutive floats, or the vertex
-// rows an indexed mesh's face names (the same floats, so the same results).
-__device__ __forceinline__ void setup_draw_tri(const Draw& dr, uint32_t local, uint32_t W, uint32_t H, Tri& t)
+// The 9 model-space coordinates of triangle `local` of a draw: a soup's 9
+// consecutive floats, or the vertex rows an indexed mesh's face names (the
+// same floats, so the same results).
+__device__ __forceinline__ void load_draw_tri(const Draw& dr, uint32_t local, float* v)
 {
     if (dr.faces) {
         const auto* f = global_ptr(dr.faces + (size_t)local * 3);
         const auto* vp = global_ptr(dr.xyz);
         const uint32_t a = 3u * f[0], b = 3u * f[1], c = 3u * f[2];
-        const float v[9] = {vp[a], vp[a + 1], vp[a + 2], vp[b], vp[b + 1], vp[b + 2], vp[c], vp[c + 1], vp[c + 2]};
-        setup_tri_from(dr.M, v, W, H, t);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            v[k] = vp[a + k];
+            v[3 + k] = vp[b + k];
+            v[6 + k] = vp[c + k];
+        }
     } else {
-        setup_tri(dr.M, dr.xyz + (size_t)local * 9, W, H, t);
+        const auto* q = global_ptr(dr.xyz + (size_t)local * 9);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) v[k] = q[k];
     }
+}
+
+__device__ __forceinline__ void setup_draw_tri(const Draw& dr, uint32_t local, uint32_t W, uint32_t H, Tri& t)
+{
+    float v[9];
+    load_draw_tri(dr, local, v);
+    setup_tri_from(dr.M, v, W, H, t);
 }
 
 // The three edge functions at integer pixel (x, y) (rasterizer.rs:71-74).
@@ -253,18 +262,22 @@ __device__ __forceinline__ uint8_t ramp_glyph(const Ramp& r, float s)
 
 // Order-preserving map of a depth that passed `z < f32::MAX` to 32 bits.
 // -0 and +0 compare equal in the reference's `<`, so both map to +0's code.
-__device__ __forceinline__ uint32_t depth_code(float z)
+// Negative values have every bit flipped and the others the sign bit.
+__device__ __forceinline__ uint32_t depth_bits_code(uint32_t u)
 {
-    // z + 0 turns -0 into +0 (and changes no other value), so that -0 == +0;
-    // then negative values have every bit flipped and the others the sign bit
-    const uint32_t u = __float_as_uint(z + 0.0f);
     return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
+__device__ __forceinline__ uint32_t depth_code(float z)
+{
+    // z + 0 turns -0 into +0 (and changes no other value), so that -0 == +0
+    return depth_bits_code(__float_as_uint(z + 0.0f));
+}
 
-// Inverse of depth_code for every depth but -0 (whose code is +0's).
+// Inverse of depth_code for every depth but -0 (whose code is +0's): codes
+// with the sign bit lose it, the others are flipped.
 __device__ __forceinline__ float depth_of_code(uint32_t code)
 {
-    return __uint_as_float((code & 0x80000000u) ? (code & 0x7FFFFFFFu) : ~code);
+    return __uint_as_float(code ^ (~(uint32_t)((int32_t)code >> 31) | 0x80000000u));
 }
 constexpr uint32_t DEPTH_CODE_ZERO = 0x80000000u;   // depth_code(+0) = depth_code(-0)
 
@@ -298,13 +311,11 @@ enum : uint32_t { CLS_EMPTY = 0, CLS_BOX = 1, CLS_SPANS = 2, CLS_FULL = 3, CLS_T
 // DX = max(|X1 - minx|, |X0 - maxx|) (|X0 - x| <= X1 - minx when x <= X0,
 // <= maxx - X0 otherwise; likewise for X1), so the sum is at most
 // (sum |A_k|) DY + (sum |B_k|) DX.  Its few roundings (relative error 2^-24
-// each) are within the margins of the bounds that use it.  miny, maxy: the
-// vertices' y extent.
-__device__ __forceinline__ float edge_terms_bound(const Tri& t, float X0, float X1, float Y0, float Y1, float miny,
-                                                  float maxy)
+// each) are within the margins of the bounds that use it.
+__device__ __forceinline__ float edge_terms_bound(const Tri& t, float X0, float X1, float Y0, float Y1)
 {
     const float DX = fmaxf(fabsf(X1 - t.minx), fabsf(X0 - t.maxx));
-    const float DY = fmaxf(fabsf(Y1 - miny), fabsf(Y0 - maxy));
+    const float DY = fmaxf(fabsf(Y1 - t.miny), fabsf(Y0 - t.maxy));
     return (fabsf(t.A0) + fabsf(t.A1) + fabsf(t.A2)) * DY + (fabsf(t.B0) + fabsf(t.B1) + fabsf(t.B2)) * DX;
 }
 
@@ -346,8 +357,7 @@ __device__ __forceinline__ uint32_t setup_class(const Tri& t)
     const float K = 8.0f * 5.9604645e-08f;
     // a non-empty domain has X0 <= X1 and Y0 <= Y1 (an empty one is CLS_EMPTY)
     const float X0 = (float)t.x0, X1 = (float)(t.x1d - 1), Y0 = (float)t.y0, Y1 = (float)(t.y1d - 1);
-    const float bound = K * edge_terms_bound(t, X0, X1, Y0, Y1, fminf(t.y1, fminf(t.y2, t.y3)),
-                                             fmaxf(t.y1, fmaxf(t.y2, t.y3)));
+    const float bound = K * edge_terms_bound(t, X0, X1, Y0, Y1);
     float ey = t.y3 - t.y1, ex = t.x3 - t.x1;
     float o = t.A2 * ey - t.B2 * ex;
     float eo = K * (fabsf(t.A2) * fabsf(ey) + fabsf(t.B2) * fabsf(ex));
@@ -359,61 +369,6 @@ __device__ __forceinline__ uint32_t setup_class(const Tri& t)
     c = o + eo < -bound ? CLS_EMPTY : c;           // back face, provably uncovered
     c = finite ? c : CLS_FULL;
     return no_pixels ? CLS_EMPTY : c;
-}
-
-// Per-row candidate spans of a CLS_BOX / CLS_TIGHT triangle, for walking a
-// box [bx0, bx1] x [by0, by1] row by row from row y_first over at most 64 rows.
-//
-// Edge k (anchor (xk, yk), coefficients A, B as in Tri) passes in FP32 only
-// where its exact value E = A (py - yk) - B (px - xk) is >= -err, with err <=
-// 3.0001 u (|A| |py - yk| + |B| |px - xk|) (three roundings of the
-// reference's expression, u = 2^-24) <= e = 4u (|A| Dy + |B| Dx) over the box
-// (Dx, Dy the largest distances from the anchor).  So a passing pixel has
-// px <= T(py) = xk + (A (py - yk) + e) / B when B > 0, and px >= T(py) when
-// B < 0; B = 0 gives no limit.  T is linear in py (slope s = A / B): it is
-// evaluated at y_first and stepped by s per row.  The float evaluation (a
-// hardware reciprocal within 1 ulp, a few roundings, up to 64 steps) errs by
-// well under 2^-17 of the magnitudes involved (M below); the limits are moved
-// outward by d = 2^-13 M + 2^-12 pixel, so every pixel that can pass lies
-// within [ceil(max L), floor(min H)] of its row.  Overflow or NaN in any of
-// these values only removes the limit (min / max ignore NaN; +-inf limits are
-// no limit), so the span is never narrower than the passing set; the walk
-// still evaluates the reference's test on every pixel of it.
-struct RowSpans {
-    float H[3], L[3], s[3];   // per edge: upper / lower limit at the current row (or +-inf), step per row
-};
-
-__device__ __forceinline__ void row_spans_begin(const Tri& t, int bx0, int bx1, int by0, int by1, int y_first,
-                                                RowSpans& r)
-{
-    const float ax[3] = {t.x2, t.x3, t.x1}, ay[3] = {t.y2, t.y3, t.y1};
-    const float A[3] = {t.A0, t.A1, t.A2}, B[3] = {t.B0, t.B1, t.B2};
-    const float X0 = (float)bx0, X1 = (float)bx1, Y0 = (float)by0, Y1 = (float)by1, Yf = (float)y_first;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const float rB = __builtin_amdgcn_rcpf(B[k]);
-        const float sk = A[k] * rB;
-        const float Dy = fmaxf(fabsf(Y0 - ay[k]), fabsf(Y1 - ay[k]));
-        const float Dx = fmaxf(fabsf(X0 - ax[k]), fabsf(X1 - ax[k]));
-        const float e = 0x1p-22f * (fabsf(A[k]) * Dy + fabsf(B[k]) * Dx) + 0x1p-120f;
-        const float T = ax[k] + (A[k] * (Yf - ay[k]) + e) * rB;
-        const float M = fabsf(ax[k]) + (fabsf(A[k]) * Dy + e) * fabsf(rB) + fabsf(sk) * 64.0f;
-        const float d = 0x1p-13f * M + 0x1p-12f;
-        r.s[k] = sk;
-        r.H[k] = B[k] > 0.0f ? T + d : INFINITY;
-        r.L[k] = B[k] < 0.0f ? T - d : -INFINITY;
-    }
-}
-
-// No limits (careful entries, whose boxes k_careful computed).
-__device__ __forceinline__ void row_spans_none(RowSpans& r)
-{
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        r.s[k] = 0.0f;
-        r.H[k] = INFINITY;
-        r.L[k] = -INFINITY;
-    }
 }
 
 // x range of the candidate box of a CLS_BOX / CLS_TIGHT triangle, clipped to

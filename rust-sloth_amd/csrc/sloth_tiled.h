@@ -20,17 +20,17 @@
 //   k_careful      one wavefront per careful triangle: exact box from row
 //                  spans, then its tile entries
 //   k_tile_raster  one 256-thread workgroup per tile, grid (tile x, tile y,
-//                  frame): each list entry's transformed triangle goes to the
-//                  LDS row of its lane, its fragments do a 64-bit LDS
-//                  atomicMin of packed keys that also name that row, then
-//                  every slot re-evaluates its winner from the row its key
-//                  names and stores its two cells and depths (coalesced,
-//                  streaming stores).  Lists
-//                  longer than the 256 LDS rows run in chunks, storing winners
-//                  after each chunk.  The image-mode tail cells are written by
-//                  the frame's first tile.  When many boxes are big, a variant
-//                  has each wavefront walk its lanes' big boxes with all 64
-//                  lanes.
+//                  frame): each list entry is set up by a lane and its row
+//                  kept in LDS, its fragments do a 64-bit LDS atomicMin of
+//                  packed keys that also name that row, then a thread takes
+//                  two slots at a time: cells from the rows their keys name
+//                  (evaluated per pixel only where the glyph is not constant
+//                  over the box), depths from the keys, 16-byte streaming
+//                  stores.  Lists longer than the 256 LDS rows run in chunks,
+//                  whose winners' cells are put aside in LDS.  The image-mode
+//                  tail cells are written by the frame's first tile.  When
+//                  many boxes are big, a variant has each wavefront walk its
+//                  lanes' big boxes with all 64 lanes.
 //
 // Tile lists live in one pool at fixed per-tile offsets, sized from an exact
 // counting run of k_bin plus headroom.  If a later run would exceed a tile's
@@ -61,6 +61,7 @@ struct TiledPlan {
     // z slot on every cell column, resolve cells from two slots and finish
     // first-column cells in k_tile_edges.
     bool has_even = true, has_odd = false;
+    bool multi = false;              // set by size(): some tile's list may grow past one chunk of the raster
     DevBuf d_edges;                  // odd: per tile and row, the first and last column slots' winners
     uint64_t n_tiles = 0;
     uint64_t n_rows = 0;

@@ -616,22 +616,40 @@ __global__ void __launch_bounds__(256) k_careful(const Frame* __restrict__ frame
 // k_tile_raster
 // ---------------------------------------------------------------------------
 constexpr uint32_t CHUNK = RASTER_BLOCK;   // list entries whose triangles sit in LDS at once (one per thread)
-constexpr uint32_t CACHE_WORDS = 12;
+// An entry's LDS row, an array per part (parts that are read together lie
+// together, and rows drawn at random then spread over all banks): the shade
+// factor or finished cell with the shader or ROW_CONST flag; the screen
+// vertices' x and y; and, read by the big-box walk only, the depth terms.
+struct Rows {
+    uint2* end;
+    float4* v12;
+    float2* v3;
+    float4* depth;
+};
+__host__ __device__ constexpr uint32_t row_bytes(bool big) { return big ? 48 : 32; }
+// end.y of a row whose triangle has one glyph over its box (end.x is then the
+// finished cell); ROW_NEGZ: its first vertex's depth is -0.  Other rows have the shader index (below 255) in the low byte.
+constexpr uint32_t ROW_CONST = 0xFFu, ROW_NEGZ = 0x100u, ROW_MASK = 0x1FFu;
 constexpr uint32_t LDS_RAMPS = 4;          // shaders staged in LDS per tile
-constexpr uint32_t SPAN_MIN_W = 6;         // box width (pixels) from which a wavefront walks row spans
 static_assert(CHUNK <= 256, "tile keys hold a cache row index in one byte");
 
 // A tile's z-test key: (depth code, frame triangle, sub) decide the order
 // exactly as make_key's do; below them a `stored` flag and the cache row p
 // of the entry that wrote the key (its lane in the chunk).  Two fragments
 // with equal (depth code, triangle, sub) are the same fragment, so the low
-// bits never change a comparison, and the resolve finds the winner's
-// transformed triangle from the key alone.  `stored` is set on keys whose
-// winner a multi-chunk tile has already stored.
+// bits never change a comparison, and the resolve finds the winner's row from
+// the key alone.  `stored` is set on keys whose winner's cell a multi-chunk
+// tile has already put aside.
 constexpr uint64_t TILE_KEY_STORED = 1u << 8;
+// An empty slot: the code of f32::MAX, which no fragment reaches, so that its
+// depth decodes like any other, and a low word of ones, which no fragment has
+// (TILED_MAX_TRIS); its flag reads as stored.
+constexpr uint64_t TILE_EMPTY = ((uint64_t)0xFF7FFFFFu << 32) | 0xFFFFFFFFu;
+__device__ __forceinline__ bool tile_empty(uint64_t k) { return (uint32_t)k == 0xFFFFFFFFu; }
+// (z is not -0: see walk_rect)
 __device__ __forceinline__ uint64_t make_tile_key(float z, uint32_t tri, uint32_t sub, uint32_t p)
 {
-    return ((uint64_t)depth_code(z) << 32) | (uint64_t)((tri << 10) | (sub << 9) | p);
+    return ((uint64_t)depth_bits_code(__float_as_uint(z)) << 32) | (uint64_t)((tri << 10) | (sub << 9) | p);
 }
 __device__ __forceinline__ uint32_t tile_key_tri(uint64_t k) { return (uint32_t)k >> 10; }
 __device__ __forceinline__ uint32_t tile_key_sub(uint64_t k) { return ((uint32_t)k >> 9) & 1u; }
@@ -660,72 +678,87 @@ struct TileGeom {
     int W;
 };
 
-// Calls f(px, py, slot, sub) for the pixels (x, y) in [xa, xb] x [ya, yb],
-// px = x and py = y as floats, slot = row0 + ((y - ya) << sws) + (x - xa) * xs.
-// Pixel coordinates are below 2^16, so stepping px by 1.0f is exact (one add
-// instead of a conversion per pixel).
-template <class Fn>
-__device__ __forceinline__ void walk_rect(int xa, int xb, int ya, int yb, int row0, int sws, int xs, uint32_t sub,
-                                          Fn&& f)
+// Tests the pixels (x, y) in [xa, xb] x [ya, yb] of triangle t with the
+// expressions of edges() and depth() and calls hit(slot, z, sub) for the
+// covered ones: slot = row0 + ((y - ya) << sws) + (x - xa) * XS.
+//
+// WALK_COLS columns are taken at a time, all rows of them.  An edge function
+// is fl(fl(A (py - ay)) - fl(B (px - ax))): its second product does not depend
+// on the row, so the three of each column are made once and a pixel costs
+// three subtractions of its own instead of nine operations; the slots of a
+// row's columns differ by constants.  Columns past xb get an infinite product,
+// which no pixel passes (the difference is -infinity or NaN).  Most boxes of a
+// dense mesh are at most four wide: 1080p sweep, 4 columns 1.095 ms, 2 or 3
+// 1.105, 5 1.09 and 6 1.12; a batch of unlike jobs 0.200, 0.221, 0.211, 0.202
+// and 0.205 ms.  (Nine operations a pixel, one at a time: 1.195 and 0.241.)
+//
+// z is that of depth() but for -0, which reads +0: x + y is -0 only for two
+// negative zeros, so adding +0 to the first vertex's depth is enough.  CHECK:
+// z < f32::MAX (the z buffer's first value never loses, NaN never wins) is
+// tested per pixel; without it the caller knows (depth_safe).
+constexpr int WALK_COLS = 4;
+template <int XS, bool CHECK, class Hit>
+__device__ __forceinline__ void walk_rect(const Tri& t, int xa, int xb, int ya, int yb, int row0, int sws, uint32_t sub,
+                                          Hit&& hit)
 {
-    const float fxb = (float)xb;
-    for (int y = ya; y <= yb; ++y, row0 += 1 << sws) {
-        const float py = (float)y;
-        int slot = row0;
-        for (float px = (float)xa; px <= fxb; px += 1.0f, slot += xs) f(px, py, slot, sub);
-    }
-}
-
-// walk_rect over the direct region with each row cut to its candidate span
-// (row_spans_begin, started at row ya): slot = row0 + ((y - ya) << sws) +
-// (x - xa) * xs as there.
-template <class Fn>
-__device__ __forceinline__ void walk_rect_spans(int xa, int xb, int ya, int yb, int row0, int sws, int xs,
-                                                RowSpans& r, Fn&& f)
-{
-    const float fxa = (float)xa, fxb = (float)xb, fxe = fxb + 1.0f;
-    for (int y = ya; y <= yb; ++y, row0 += 1 << sws) {
-        // lo within [xa, xb + 1] (an empty row when above hi), so that its
-        // integer conversion is exact
-        const float lo = fminf(fmaxf(fmaxf(fmaxf(r.L[0], r.L[1]), r.L[2]), fxa), fxe);
-        const float hi = fminf(fminf(fminf(r.H[0], r.H[1]), r.H[2]), fxb);
-        const float py = (float)y, px0 = ceilf(lo), px1 = floorf(hi);
-        int slot = row0 + ((int)px0 - xa) * xs;
-        for (float px = px0; px <= px1; px += 1.0f, slot += xs) f(px, py, slot, 1u);
+    const float z1 = t.z1 + 0.0f, dz2 = t.z2 - t.z1, dz3 = t.z3 - t.z1;
+    for (int x = xa; x <= xb; x += WALK_COLS, row0 += WALK_COLS * XS) {
+        float q0[WALK_COLS], q1[WALK_COLS], q2[WALK_COLS];
+        float px = (float)x;   // below 2^16: stepping by 1.0f is exact
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            r.H[k] += r.s[k];
-            r.L[k] += r.s[k];
+        for (int c = 0; c < WALK_COLS; ++c, px += 1.0f) {
+            q0[c] = c == 0 || x + c <= xb ? t.B0 * (px - t.x2) : INFINITY;
+            q1[c] = t.B1 * (px - t.x3);
+            q2[c] = t.B2 * (px - t.x1);
+        }
+        int slot = row0;
+        for (int y = ya; y <= yb; ++y, slot += 1 << sws) {
+            const float py = (float)y;
+            const float p0 = t.A0 * (py - t.y2), p1 = t.A1 * (py - t.y3), p2 = t.A2 * (py - t.y1);
+#pragma unroll
+            for (int c = 0; c < WALK_COLS; ++c) {
+                const float w0 = p0 - q0[c], w1 = p1 - q1[c], w2 = p2 - q2[c];
+                const float z = z1 + t.a * (w1 * dz2 + w2 * dz3);
+                if (inside(w0, w1, w2) && (!CHECK || z < F32_MAX)) hit(slot + c * XS, z, sub);
+            }
         }
     }
 }
 
-// Calls f(px, py, slot, sub) for every logical pixel of the box that lands in
-// the tile's wrapped region (column 2x - W in [tc0,tc1), row y + 1).
-template <class Fn>
-__device__ __forceinline__ void walk_wrapped(const TileGeom& g, int bx0, int bx1, int by0, int by1, Fn&& f)
+// Every pixel of a CLS_BOX / CLS_TIGHT triangle's box has a finite depth below
+// f32::MAX: vertices within 2^22 and pixels below 2^16 give |w| < 2^47, so
+// |z| < 2^60 + 2^15 2 2^47 2^61.
+__device__ __forceinline__ bool depth_safe(const Tri& t)
+{
+    // (the IEEE 754-2019 maximum propagates NaN)
+    const float m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(t.z1), fabsf(t.z2)), fabsf(t.z3));
+    return m < 0x1p60f && fabsf(t.a) < 0x1p15f;
+}
+
+// walk_rect over the box's pixels that land in the tile's wrapped region
+// (column 2x - W in [tc0,tc1), row y + 1).
+template <int XS, class Hit>
+__device__ __forceinline__ void walk_wrapped(const TileGeom& g, const Tri& t, int bx0, int bx1, int by0, int by1,
+                                             Hit&& hit)
 {
     const int xa = max(bx0, (g.tc0 + g.W + 1) >> 1), xb = min(bx1, (g.tc1 - 1 + g.W) >> 1);
     const int ya = max(by0, g.tr0 - 1), yb = min(by1, g.tr1 - 2);
-    walk_rect(xa, xb, ya, yb, ((ya + 1 - g.tr0) << g.sws) + ((2 * xa - g.W - g.tc0) >> g.cs), g.sws, 2 >> g.cs, 0u,
-              f);
+    walk_rect<XS, true>(t, xa, xb, ya, yb, ((ya + 1 - g.tr0) << g.sws) + ((2 * xa - g.W - g.tc0) >> g.cs), g.sws, 0u, hit);
 }
 
-// Calls f(px, py, slot, sub) for the candidate pixels of the box that land in
-// the tile: the direct region (column 2x in [tc0,tc1), row y) with each row
-// cut to its span (spans started at row max(by0, tr0)), then the wrapped one.
-template <class Fn>
-__device__ __forceinline__ void walk_tile(const TileGeom& g, int bx0, int bx1, int by0, int by1, bool use_spans,
-                                          RowSpans& r, Fn&& f)
+// Walks the candidate pixels of the box that land in the tile: the direct
+// region (column 2x in [tc0,tc1), row y; safe: every lane is depth_safe), then
+// the wrapped one.
+template <int XS, class Hit>
+__device__ __forceinline__ void walk_tile(const TileGeom& g, const Tri& t, int bx0, int bx1, int by0, int by1,
+                                          bool safe, Hit&& hit)
 {
     const int xa = max(bx0, (g.tc0 + 1) >> 1), xb = min(bx1, (g.tc1 - 1) >> 1);
     const int ya = max(by0, g.tr0), yb = min(by1, g.tr1 - 1);
     const int row0 = ((ya - g.tr0) << g.sws) + ((2 * xa - g.tc0) >> g.cs);
-    if (use_spans)
-        walk_rect_spans(xa, xb, ya, yb, row0, g.sws, 2 >> g.cs, r, f);
-    else
-        walk_rect(xa, xb, ya, yb, row0, g.sws, 2 >> g.cs, 1u, f);
-    walk_wrapped(g, bx0, bx1, by0, by1, f);
+    if (safe) walk_rect<XS, false>(t, xa, xb, ya, yb, row0, g.sws, 1u, hit);
+    else walk_rect<XS, true>(t, xa, xb, ya, yb, row0, g.sws, 1u, hit);
+    walk_wrapped<XS>(g, t, bx0, bx1, by0, by1, hit);
 }
 
 // The direct part of the walk: the box clipped to the tile's logical pixels,
@@ -758,14 +791,22 @@ __device__ __forceinline__ uint32_t entry_tri(uint32_t e, const uint4* __restric
 // One workgroup per tile; grid (tile x, tile y, frame - f_lo).  Blocks past a
 // smaller frame's tile grid return at once.
 //
-// The tile's list is taken CHUNK entries at a time: each entry's transformed
-// triangle goes to the LDS row of its lane, and its fragments take a 64-bit
-// LDS atomicMin of packed (depth, triangle, sub, row) keys (make_tile_key).
-// With one chunk, every slot then re-evaluates its winner from the row its
-// key names and stores it.  With several, after each chunk the slots whose
-// key was written in that chunk store that winner and flag the key as stored
-// (the last store of a slot is its final winner's, since a later winner
-// comes from a later chunk), and the empty slots are stored at the end.
+// The tile's list is taken CHUNK entries at a time: each entry's row goes to
+// the LDS row of its lane, and its fragments take a 64-bit LDS atomicMin of
+// packed (depth, triangle, sub, row) keys (make_tile_key).  At the end every
+// slot's cell comes from the row its key names and its depth from the key's
+// code, and a thread stores two slots at a time.  With several chunks, after
+// each but the last the slots whose key was written in that chunk put their
+// cell aside in LDS and flag the key (a later winner comes from a later
+// chunk), so that the frame is still written once, in 16-byte stores.
+//
+// What bounds it: VALU issue (a wave64 instruction takes four cycles of its
+// SIMD).  A wavefront of entries costs about 240 instructions of set-up and 23
+// per step of its largest box, and a slot pair about 35 at the end.
+// 256 frames of 1920x1080, 327,680 triangles: 592M wavefront instructions on
+// 1024 SIMDs, 1.02 ms (the stores of its 4.26 GB alone take 0.75 ms).  Before,
+// with rows of 48 bytes, nine operations more per pixel and chunk by chunk
+// stores, 762M and 1.19 ms.
 //
 // BIG: an entry whose box covers more than BIG_BOX of the tile's pixels in
 // its direct region is not walked by its own lane; after its own walk, each
@@ -777,7 +818,7 @@ __device__ __forceinline__ uint32_t entry_tri(uint32_t e, const uint4* __restric
 // same for the whole workgroup and its fields come through scalar loads that
 // do not wait for the list entries.
 //
-// ODD: frames of odd width.  Every cell column holds a z slot (direct pixels
+// WRAP: frames of odd width.  Every cell column holds a z slot (direct pixels
 // on even columns, wrapped ones on odd columns) and a cell's final value is
 // the later write of two slots' winners: its own slot's and the one to its
 // left (rasterizer.rs:82-85 writes cells id and id + 1), and the row's
@@ -791,18 +832,18 @@ __device__ __forceinline__ uint32_t entry_tri(uint32_t e, const uint4* __restric
 // kernel its own copy of the lambdas below, which the compiler then inlines
 // as it does for a single caller (shared by the two kernels, they cost the
 // 3-D instances two VGPRs spilled to scratch).
-template <bool BIG, bool ONE, bool ODD, bool FLAT>
+template <bool BIG, bool ONE, bool WRAP, bool FLAT>
 __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, const Ramp* __restrict__ ramps,
-                                            const Ramp* s_ramp, const Frame& fr, uint32_t tx, uint32_t ty, uint64_t gt,
-                                            uint64_t o, uint32_t n, int tws, int ths, const uint32_t* __restrict__ pool,
-                                            const int32_t* __restrict__ nl, const uint4* __restrict__ careful_box,
-                                            uint32_t* __restrict__ cells, float* __restrict__ zbuf,
-                                            int32_t* __restrict__ win, uint32_t win_raw, uint4* __restrict__ edge_out,
-                                            uint64_t* smem)
+                                            const Ramp* s_ramp, uint32_t* s_negz, const Frame& fr, uint32_t tx,
+                                            uint32_t ty, uint64_t gt, uint64_t o, uint32_t n, int tws, int ths,
+                                            const uint32_t* __restrict__ pool, const int32_t* __restrict__ nl,
+                                            const uint4* __restrict__ careful_box, uint32_t* __restrict__ cells,
+                                            float* __restrict__ zbuf, int32_t* __restrict__ win, uint32_t win_raw,
+                                            uint4* __restrict__ edge_out, uint64_t* smem)
 {
-    static_assert(!(BIG && ODD), "the big-box walk maps slots of even widths only");
+    static_assert(!(BIG && WRAP), "the big-box walk maps slots of even columns only");
     const uint32_t W = fr.W, H = fr.H;
-    const int sws = tws - (ODD ? 0 : 1);
+    const int sws = tws - (WRAP ? 0 : 1);
     const uint32_t S = 1u << (sws + ths);
     TileGeom g;
     g.tc0 = (int)(tx << tws);
@@ -810,128 +851,107 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
     g.tr0 = (int)(ty << ths);
     g.tr1 = min((int)H, g.tr0 + (1 << ths));
     g.sws = sws;
-    g.cs = ODD ? 0 : 1;
+    g.cs = WRAP ? 0 : 1;
     g.W = (int)W;
 
     const uint32_t* list = pool + o;
+    uint64_t* keys = smem;
+    Rows rows;
+    rows.end = (uint2*)(keys + S);
+    rows.v12 = (float4*)(rows.end + CHUNK);
+    rows.v3 = (float2*)(rows.v12 + CHUNK);
+    rows.depth = (float4*)(rows.v3 + CHUNK);   // BIG only
+    // a cell per slot: WRAP, the winners' for the per-cell resolve; else, in
+    // tiles of several chunks, those put aside
+    uint32_t* wcell = (uint32_t*)(keys + S) + CHUNK * row_bytes(BIG) / 4;
 
     const int32_t* fnl = nl + fr.nl_off;
     uint32_t* fc = cells + fr.cell_off;
     float* fz = zbuf + fr.z_off;
-    // A thread owns the slots of one column of the tile, every row_step-th
-    // row (the block is at least one tile row of slots wide).
+    auto win_of = [&](uint64_t k) -> uint32_t {
+        // win_raw gives triangle << 1 | sub for the shading pass
+        return tile_empty(k) ? 0xFFFFFFFFu : win_raw ? (uint32_t)k >> 9 : tile_key_tri(k);
+    };
+    // WRAP: a thread owns the slots of one column of the tile, every
+    // row_step-th row (the block is at least one tile row of slots wide):
+    // fn(slot, row, id of the slot's first cell) over its slots in the frame.
     const uint32_t my_sc = threadIdx.x & ((1u << sws) - 1);
     const int my_col = g.tc0 + ((int)my_sc << g.cs);
-    const int row_step = (int)(blockDim.x >> sws);
-    const uint64_t id_step = (uint64_t)row_step * W;
-    // fn(slot, row, id of the slot's first cell) over this thread's slots
-    // inside the frame
     auto for_my_slots = [&](auto&& fn) {
         if (my_col >= g.tc1) return;
+        const int row_step = (int)(blockDim.x >> sws);
+        const uint64_t id_step = (uint64_t)row_step * W;
         int row = g.tr0 + (int)(threadIdx.x >> sws);
         uint64_t id = (uint64_t)row * W + (uint64_t)my_col;
         for (; row < g.tr1; row += row_step, id += id_step)
             fn(((uint32_t)(row - g.tr0) << sws) | my_sc, row, id);
     };
-    // ODD: the winners' cells of the tile's slots, for the per-cell resolve
-    uint32_t* wcell = (uint32_t*)(smem + S) + CHUNK * CACHE_WORDS;
-    // Stores the cells and depths of slot s from its winning cell (or
-    // blank); ODD: the depth and winner, and the cell into wcell.
-    auto store = [&](uint32_t s, int row, uint64_t id, uint64_t k, uint32_t cell, float z) {
-        if constexpr (ODD) {
-            const int32_t wt = (k == KEY_EMPTY) ? -1 : (int32_t)tile_key_tri(k);
-            __builtin_nontemporal_store(k == KEY_EMPTY ? F32_MAX : z, fz + id);
-            if (win) {
-                const int32_t wv = (k == KEY_EMPTY) ? -1 : (win_raw ? (int32_t)((uint32_t)wt << 1 | tile_key_sub(k)) : wt);
-                __builtin_nontemporal_store(wv, win + fr.z_off + id);
-            }
-            if (k != KEY_EMPTY) wcell[s] = cell;
-            return;
+    // WRAP: stores slot s's depth and winner, its cell into wcell.
+    auto store_slot = [&](uint32_t s, uint64_t id, uint64_t k, uint32_t cell, float z) {
+        __builtin_nontemporal_store(z, fz + id);
+        if (win) __builtin_nontemporal_store((int32_t)win_of(k), win + fr.z_off + id);
+        if (!tile_empty(k)) wcell[s] = cell;
+    };
+    // Otherwise a thread takes the slot pairs (2q, 2q + 1) of a row, q = thread
+    // mod (slots a row / 2), every (512 >> sws)-th row: fn(first slot, row, its
+    // first cell's column, that cell's byte offset from the tile's first cell,
+    // the second slot lies in the frame).  Addresses are the tile's (uniform)
+    // plus 32 bits a lane (a tile spans at most 64 rows of 65535 cells).
+    auto for_my_pairs = [&](auto&& fn) {
+        const uint32_t q = threadIdx.x & ((1u << (sws - 1)) - 1);
+        const int col = g.tc0 + ((int)q << 2);
+        if (col >= g.tc1) return;
+        const bool two = col + 2 < g.tc1;
+        const int step = (int)(blockDim.x >> (sws - 1));
+        int r = (int)(threadIdx.x >> (sws - 1));
+        uint32_t off = ((uint32_t)r * W + (q << 2)) * 4u;
+        for (; r < g.tr1 - g.tr0; r += step, off += (uint32_t)step * W * 4u)
+            fn(((uint32_t)r << sws) | (q << 1), g.tr0 + r, col, off, two);
+    };
+    const uint64_t tile0 = (uint64_t)g.tr0 * W + (uint64_t)g.tc0;
+    uint8_t* tile_cells = (uint8_t*)(fc + tile0);
+    uint8_t* tile_z = (uint8_t*)(fz + tile0);
+    uint8_t* tile_win = win ? (uint8_t*)(win + fr.z_off + tile0) : nullptr;
+    // Four words of a pair, or the first two (streaming stores: the frame is
+    // written once and not read back here).  Words need only their own
+    // alignment: a 16-byte store at any 4-byte address is one instruction.
+    auto put = [](uint8_t* p, uint32_t a, uint32_t b, uint32_t c, uint32_t d, bool two) {
+        typedef unsigned int v4u __attribute__((ext_vector_type(4), aligned(4)));
+        typedef unsigned int v2u __attribute__((ext_vector_type(2), aligned(4)));
+        if (two) {
+            const v4u v = {a, b, c, d};
+            __builtin_nontemporal_store(v, (v4u*)p);
+        } else {
+            const v2u v = {a, b};
+            __builtin_nontemporal_store(v, (v2u*)p);
         }
-        uint32_t c0 = CELL_BLANK, c1 = CELL_BLANK;
-        float z0 = F32_MAX;
-        int32_t wt = -1;
-        if (k != KEY_EMPTY) {
-            c0 = c1 = cell;
-            z0 = z;
-            wt = (int32_t)tile_key_tri(k);
-        }
-        if (fr.image && my_col == 0) {
+    };
+    const bool nl_here = fr.image && tx == 0;
+    // Stores a pair from its keys' low words, cells and depths.
+    auto store_pair = [&](int row, int col, uint32_t off, bool two, uint32_t k0, uint32_t c0, float z0, uint32_t k1,
+                          uint32_t c1, float z1) {
+        uint32_t c0b = c0;
+        if (nl_here && col == 0) {
             // cell row*W + 1: the newline of row `row` comes after every pixel
             // of its triangle's row and before its next row, so it overwrites
             // a wrapped pixel (drawn in row-1) of the same or an earlier
             // triangle
             const int32_t nlr = fnl[row];
-            if (nlr >= 0 && (k == KEY_EMPTY || nlr >= wt)) c1 = CELL_NEWLINE;
+            if (nlr >= 0 && (tile_empty(k0) || nlr >= (int32_t)tile_key_tri(k0))) c0b = CELL_NEWLINE;
         }
-        // streaming stores: the frame is written once and not read back here
-        __builtin_nontemporal_store((uint64_t)c0 | ((uint64_t)c1 << 32), (uint64_t*)(fc + id));
-        __builtin_nontemporal_store((uint64_t)__float_as_uint(z0) | ((uint64_t)__float_as_uint(F32_MAX) << 32),
-                                    (uint64_t*)(fz + id));
-        if (win) {
-            // win_raw gives triangle << 1 | sub for the shading pass
-            const int32_t wv = (k == KEY_EMPTY) ? -1 : (win_raw ? (int32_t)((uint32_t)wt << 1 | tile_key_sub(k)) : wt);
-            __builtin_nontemporal_store((uint64_t)(uint32_t)wv | ((uint64_t)0xFFFFFFFFu << 32),
-                                        (uint64_t*)(win + fr.z_off + id));
-        }
-    };
-    // Even widths, final stores: a thread takes the slot pairs (2q, 2q + 1) of
-    // a row, q = thread mod (slots a row / 2), every (512 >> sws)-th row, and
-    // writes a pair's 4 cells, 2 depth pairs and winners with one 16-byte
-    // store each where the address is 16-byte aligned (two 8-byte ones
-    // otherwise).  fn(first slot, row, id of its first cell, that cell's
-    // column, the second slot lies in the frame).
-    auto for_my_pairs = [&](auto&& fn) {
-        const uint32_t q = threadIdx.x & ((1u << (sws - 1)) - 1);
-        const int col = g.tc0 + ((int)q << 2);
-        if (col >= g.tc1) return;
-        const int step = (int)(blockDim.x >> (sws - 1));
-        int row = g.tr0 + (int)(threadIdx.x >> (sws - 1));
-        uint64_t id = (uint64_t)row * W + (uint64_t)col;
-        for (; row < g.tr1; row += step, id += (uint64_t)step * W)
-            fn(((uint32_t)(row - g.tr0) << sws) | (q << 1), row, id, col, col + 2 < g.tc1);
-    };
-    auto put_pair = [](uint32_t* p, uint32_t a, uint32_t b, uint32_t c, uint32_t d, bool first, bool second) {
-        typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-        if (first && second && ((uintptr_t)p & 15u) == 0) {
-            const v4u v = {a, b, c, d};
-            __builtin_nontemporal_store(v, (v4u*)p);
-            return;
-        }
-        if (first) __builtin_nontemporal_store((uint64_t)a | ((uint64_t)b << 32), (uint64_t*)p);
-        if (second) __builtin_nontemporal_store((uint64_t)c | ((uint64_t)d << 32), (uint64_t*)(p + 2));
-    };
-    // Stores the slots of a pair that `need0` / `need1` name, as store()
-    // stores one slot (winning cell or blank, depth or f32::MAX, winner).
-    auto store_pair = [&](int row, uint64_t id, int col, uint64_t k0, uint32_t c0, float z0, bool need0, uint64_t k1,
-                          uint32_t c1, float z1, bool need1) {
-        const int32_t t0 = (k0 == KEY_EMPTY) ? -1 : (int32_t)tile_key_tri(k0);
-        const int32_t t1 = (k1 == KEY_EMPTY) ? -1 : (int32_t)tile_key_tri(k1);
-        uint32_t c0b = c0;
-        if (fr.image && col == 0) {
-            // cell row*W + 1, as in store()
-            const int32_t nlr = fnl[row];
-            if (nlr >= 0 && (k0 == KEY_EMPTY || nlr >= t0)) c0b = CELL_NEWLINE;
-        }
-        put_pair(fc + id, c0, c0b, c1, c1, need0, need1);
-        put_pair((uint32_t*)(fz + id), __float_as_uint(z0), __float_as_uint(F32_MAX), __float_as_uint(z1),
-                 __float_as_uint(F32_MAX), need0, need1);
-        if (win) {
-            auto wv = [&](uint64_t k, int32_t t) -> uint32_t {
-                return (uint32_t)((k == KEY_EMPTY) ? -1 : (win_raw ? (int32_t)((uint32_t)t << 1 | tile_key_sub(k)) : t));
-            };
-            put_pair((uint32_t*)(win + fr.z_off + id), wv(k0, t0), 0xFFFFFFFFu, wv(k1, t1), 0xFFFFFFFFu, need0, need1);
-        }
+        put(tile_cells + off, c0, c0b, c1, c1, two);
+        put(tile_z + off, __float_as_uint(z0), __float_as_uint(F32_MAX), __float_as_uint(z1), __float_as_uint(F32_MAX), two);
+        if (win) put(tile_win + off, win_of(k0), 0xFFFFFFFFu, win_of(k1), 0xFFFFFFFFu, two);
     };
 
     if (n == 0) {
         // no triangle reaches the tile: blank cells, f32::MAX depths, and the
         // newline cells of column 1
-        if constexpr (ODD)
-            for_my_slots([&](uint32_t s, int row, uint64_t id) { store(s, row, id, KEY_EMPTY, CELL_BLANK, F32_MAX); });
+        if constexpr (WRAP)
+            for_my_slots([&](uint32_t s, int, uint64_t id) { store_slot(s, id, TILE_EMPTY, CELL_BLANK, F32_MAX); });
         else
-            for_my_pairs([&](uint32_t, int row, uint64_t id, int col, bool two) {
-                store_pair(row, id, col, KEY_EMPTY, CELL_BLANK, F32_MAX, true, KEY_EMPTY, CELL_BLANK, F32_MAX, two);
+            for_my_pairs([&](uint32_t, int row, int col, uint32_t off, bool two) {
+                store_pair(row, col, off, two, ~0u, CELL_BLANK, F32_MAX, ~0u, CELL_BLANK, F32_MAX);
             });
     } else {
         // glyph of shade sh under shader r: the first LDS_RAMPS shaders from
@@ -941,20 +961,21 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
             if (r < LDS_RAMPS) return ramp_glyph(s_ramp[r], sh);
             return ramp_glyph(ramps[r], sh);
         };
-        // The glyph a triangle gives every pixel of its box [X0,X1] x [Y0,Y1]
-        // when that is provably one glyph, else ~0u.  The pixel's shade is
-        // fl(na * S) with S = fl(fl(w0 + w1) + w2) (rasterizer.rs:76).  Each
-        // FP32 edge function errs from the exact one by at most
+        // The glyph a triangle gives every pixel of its box when that is
+        // provably one glyph, else ~0u.  The pixel's shade is fl(na * S) with
+        // S = fl(fl(w0 + w1) + w2) (rasterizer.rs:76).  Each FP32 edge
+        // function errs from the exact one by at most
         // 4.0003u (|A| |py - ay| + |B| |px - ax|) (u = 2^-24), the exact ones
         // sum to the exact orient, the two additions add at most 2.0001u of
         // their inputs' magnitudes, and the FP32 orient o errs from the exact
         // one by at most 4.0002u (|A2| |y3 - y1| + |B2| |x3 - x1|).  So every
         // S lies within E = 10u (Sb + Q) of o, with Sb the edge terms' sum
         // over the box and Q o's terms; 10u also covers the rounding of E
-        // and of o -+ E (Sb >= |o|).  fl(na * .) and the step index are
-        // monotone, so equal indices at the two ends mean one glyph for the
-        // whole box.  Shaders that are not non-decreasing, and non-finite
-        // values, take the per-pixel evaluation.
+        // and of o -+ E (Sb >= |o|).  `terms` is Sb + Q or more.  fl(na * .)
+        // and the step index are monotone, so equal indices at the two ends
+        // mean one glyph for the whole box.  Shaders that are not
+        // non-decreasing, and non-finite values, take the per-pixel
+        // evaluation.
         //
         // na comes here from the hardware reciprocal square root: na_h =
         // fl(fl(nz rsq(n2)) a), rsq within 1 ulp, so for n2 in [2^-100,
@@ -964,20 +985,11 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
         // 2^-19 (|o| + E).  The lower end's step index i is counted, and the
         // upper end compared with threshold i: both ends have index i when
         // it is at most thr[i] (thresholds are non-decreasing).
-        auto box_glyph = [&](const Ramp& rp, const Tri& t, float na, int bx0, int bx1, int by0, int by1) -> uint32_t {
+        auto box_glyph = [&](const Ramp& rp, const Tri& t, float na, float terms) -> uint32_t {
             if (!rp.sorted) return ~0u;
-            // the edge terms' exact maximum over the box, edge by edge (an
-            // empty box has no pixels, so its glyph is never used); the
-            // cheaper edge_terms_bound would also do, but its schedule costs
-            // this kernel a register spill
-            const float X0 = (float)bx0, X1 = (float)bx1, Y0 = (float)by0, Y1 = (float)by1;
-            const float Sb =
-                fabsf(t.A0) * fmaxf(fabsf(Y0 - t.y2), fabsf(Y1 - t.y2)) + fabsf(t.B0) * fmaxf(fabsf(X0 - t.x2), fabsf(X1 - t.x2)) +
-                fabsf(t.A1) * fmaxf(fabsf(Y0 - t.y3), fabsf(Y1 - t.y3)) + fabsf(t.B1) * fmaxf(fabsf(X0 - t.x3), fabsf(X1 - t.x3)) +
-                fabsf(t.A2) * fmaxf(fabsf(Y0 - t.y1), fabsf(Y1 - t.y1)) + fabsf(t.B2) * fmaxf(fabsf(X0 - t.x1), fabsf(X1 - t.x1));
             const float ey = t.y3 - t.y1, ex = t.x3 - t.x1;
             const float o = t.A2 * ey - t.B2 * ex;
-            const float E = 5.9604645e-07f * (Sb + fabsf(t.A2) * fabsf(ey) + fabsf(t.B2) * fabsf(ex));
+            const float E = 5.9604645e-07f * terms;
             const float E2 = E + 0x1p-19f * (fabsf(o) + E);
             const float s1 = na * (o - E2), s2 = na * (o + E2);
             // NaN or infinity anywhere fails the finite test (v_maximum3 propagates NaN)
@@ -988,45 +1000,61 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
             if (i < rp.n && !(hi <= rp.thr[i])) return ~0u;
             return i < rp.n ? rp.glyph[i] : rp.fallback;
         };
-        uint64_t* keys = smem;
-        float* cache = (float*)(keys + S);
         const bool one_draw = fr.draw_end - fr.draw_begin == 1;
         const bool multi = n > CHUNK;
-
-        // Winner of a slot with key k (written in the current chunk), from
-        // the cache row the key names.  A row whose triangle has one glyph
-        // over its box holds the finished cell (low byte of its last word
-        // 0xFF); the depth then comes from the key's code, except for a
-        // zero depth, whose sign the code does not keep.  Other winners are
-        // re-evaluated from the transformed triangle.
-        auto winner = [&](int col, int row, uint64_t k, uint32_t& cell, float& z) {
+        auto draw_of_tri = [&](uint32_t T) -> const Draw& {
+            return ONE ? draws[fr.draw_begin] : one_draw ? draws[fr.draw_begin] : draw_of_t(draws, fr, T);
+        };
+        // the pixel that key k denotes at the slot of cell (row, col)
+        auto pixel_of = [&](int col, int row, uint64_t k, float& px, float& py) {
             const uint32_t sub = tile_key_sub(k);
-            const float4* row4 = (const float4*)(cache + tile_key_row(k) * CACHE_WORDS);
-            const float4 q2 = row4[2];
-            const uint32_t cw = __float_as_uint(q2.w);
+            px = (float)(sub ? (col >> 1) : ((col + g.W) >> 1));
+            py = (float)(sub ? row : row - 1);
+        };
+        // The depth of slot (row, col)'s winner from its mesh: zero depths,
+        // whose sign the code does not keep.
+        auto mesh_depth = [&](int col, int row, uint64_t k) -> float {
+            const uint32_t T = tile_key_tri(k);
+            const Draw& dr = draw_of_tri(T);
+            Tri t;
+            setup_draw_tri(dr, T - dr.tri_begin, W, H, t);
+            float px, py, w0, w1, w2;
+            pixel_of(col, row, k, px, py);
+            edges(t, px, py, w0, w1, w2);
+            return depth(t, w1, w2);
+        };
+        // Cell and depth of a winner whose row is not plainly ROW_CONST: the
+        // expressions of edges() and shade_value() on the row's vertices.
+        // A zero depth is -0 only when its first vertex's is (x + y = -0 only
+        // for two negative zeros), so a ROW_CONST row without ROW_NEGZ never
+        // comes here for its sign.
+        auto winner_slow = [&](int col, int row, uint64_t k, uint32_t& cell, float& z) {
+            const uint32_t r = tile_key_row(k);
+            const uint2 end = rows.end[r];
+            const uint32_t cw = end.y;
             const uint32_t code = (uint32_t)(k >> 32);
-            const bool fast = (cw & 0xFFu) == 0xFFu;
-            if (fast && code != DEPTH_CODE_ZERO) {
-                cell = __float_as_uint(q2.z);
-                z = depth_of_code(code);
-                return;
-            }
-            const float4 q0 = row4[0], q1 = row4[1];
-            const float px = (float)(sub ? (col >> 1) : ((col + g.W) >> 1));
-            const float py = (float)(sub ? row : row - 1);
-            // the same expressions as edges(), depth() and shade_value()
-            const float x1 = q0.x, y1 = q0.y, x2 = q0.z, y2 = q0.w, x3 = q1.x, y3 = q1.y;
+            cell = end.x;
+            z = depth_of_code(code);
+            if (code == DEPTH_CODE_ZERO) z = mesh_depth(col, row, k);
+            if ((cw & 0xFFu) == ROW_CONST) return;
+            float px, py;
+            pixel_of(col, row, k, px, py);
+            const float4 v12 = rows.v12[r];
+            const float2 v3 = rows.v3[r];
+            const float x1 = v12.x, y1 = v12.y, x2 = v12.z, y2 = v12.w, x3 = v3.x, y3 = v3.y;
             const float w0 = (x3 - x2) * (py - y2) - (y3 - y2) * (px - x2);
             const float w1 = (x1 - x3) * (py - y3) - (y1 - y3) * (px - x3);
             const float w2 = (x2 - x1) * (py - y1) - (y2 - y1) * (px - x1);
-            z = q1.z + q2.y * (w1 * q1.w + w2 * q2.x);
-            const float sh = q2.z * (w0 + w1 + w2);
-            cell = fast ? __float_as_uint(q2.z) : glyph_of(cw & 0xFFu, sh) | (cw & 0xFFFFFF00u);
+            const float sh = __uint_as_float(end.x) * (w0 + w1 + w2);
+            cell = glyph_of(cw & 0xFFu, sh) | (cw & 0xFFFFFF00u);
         };
+        auto row_end = [&](uint64_t k) -> uint2 { return rows.end[tile_key_row(k)]; };
+        auto plain = [](uint2 w) { return (w.y & ROW_MASK) == ROW_CONST; };
 
-        for (uint32_t s = threadIdx.x; s < S; s += blockDim.x) keys[s] = KEY_EMPTY;
+        for (uint32_t s = threadIdx.x; s < S; s += blockDim.x) keys[s] = TILE_EMPTY;
+        if (!WRAP && threadIdx.x == 0) *s_negz = 0;
         for (uint32_t base = 0; base < n; base += CHUNK) {
-            __syncthreads();   // keys cleared / the previous chunk's winner stores no longer read its rows
+            __syncthreads();   // keys cleared / the previous chunk's cells no longer read its rows
             const uint32_t p = threadIdx.x;
             bool big = false;              // BIG: this lane's box is walked by its wavefront
             uint32_t big_T = 0, big_rect = 0;
@@ -1034,7 +1062,7 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                 int bx0, bx1, by0, by1;
                 bool given, tight;
                 const uint32_t T = entry_tri(list[base + p], careful_box, bx0, bx1, by0, by1, given, tight);
-                const Draw& dr = ONE ? draws[fr.draw_begin] : one_draw ? draws[fr.draw_begin] : draw_of_t(draws, fr, T);
+                const Draw& dr = draw_of_tri(T);
                 const uint32_t li = T - dr.tri_begin;
                 Tri t;
                 setup_draw_tri(dr, li, W, H, t);
@@ -1042,46 +1070,52 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                 normal_parts(t, nz, n2);
                 const auto* c = global_ptr(dr.rgb + (size_t)li * 3);
                 const uint32_t rgb = ((uint32_t)c[0] << 8) | ((uint32_t)c[1] << 16) | ((uint32_t)c[2] << 24);
+                // Sb + Q of the glyph proof.  Boxes of box_x lie within a
+                // pixel of the vertices' extent in x and inside it in y, the
+                // |A_k| sum to 2 wx and the |B_k| to 2 wy (the extents), and
+                // Q <= 2 wx wy: at most 2 wx wy + 2 wy (wx + 1) + 2 wx wy.
+                const float wx = t.maxx - t.minx, wy = t.maxy - t.miny;
+                float terms = wy * (6.0f * wx + 2.0f);
                 if (!given) {
                     box_x(t, tight, bx0, bx1);
                     by0 = t.y0;
                     by1 = t.y1d - 1;
+                } else {
+                    // careful boxes: the edge terms' exact maximum over the
+                    // box, edge by edge (an empty box has no pixels, so its
+                    // glyph is never used)
+                    const float X0 = (float)bx0, X1 = (float)bx1, Y0 = (float)by0, Y1 = (float)by1;
+                    terms = fabsf(t.A0) * fmaxf(fabsf(Y0 - t.y2), fabsf(Y1 - t.y2)) + fabsf(t.B0) * fmaxf(fabsf(X0 - t.x2), fabsf(X1 - t.x2)) +
+                            fabsf(t.A1) * fmaxf(fabsf(Y0 - t.y3), fabsf(Y1 - t.y3)) + fabsf(t.B1) * fmaxf(fabsf(X0 - t.x3), fabsf(X1 - t.x3)) +
+                            fabsf(t.A2) * fmaxf(fabsf(Y0 - t.y1), fabsf(Y1 - t.y1)) + fabsf(t.B2) * fmaxf(fabsf(X0 - t.x1), fabsf(X1 - t.x1)) +
+                            fabsf(t.A2) * fabsf(t.y3 - t.y1) + fabsf(t.B2) * fabsf(t.x3 - t.x1);
                 }
                 // a triangle with one glyph over its box keeps its finished
-                // cell where the shade factor would be, flagged by 0xFF
+                // cell where the shade factor would be
                 uint32_t bg = ~0u;
                 if (n2 >= 0x1p-100f && n2 <= 0x1p100f) {
                     const float na_h = nz * __builtin_amdgcn_rsqf(n2) * t.a;
                     const uint32_t r = dr.ramp;
-                    bg = r < LDS_RAMPS ? box_glyph(s_ramp[r], t, na_h, bx0, bx1, by0, by1)
-                                       : box_glyph(ramps[r], t, na_h, bx0, bx1, by0, by1);
+                    bg = r < LDS_RAMPS ? box_glyph(s_ramp[r], t, na_h, terms) : box_glyph(ramps[r], t, na_h, terms);
                 }
-                float w2 = __uint_as_float(bg | rgb);
+                uint32_t w2 = bg | rgb;
+                uint32_t w3 = ROW_CONST | (__float_as_uint(t.z1) == 0x80000000u ? ROW_NEGZ : 0u);
                 // the others keep the shade factor (rasterizer.rs:76
                 // multiplies the unit normal's z by a first)
-                if (bg == ~0u) w2 = nz / sqrtf(n2) * t.a;
-                const uint32_t w3 = rgb | (bg != ~0u ? 0xFFu : dr.ramp);
-                float4* row4 = (float4*)(cache + p * CACHE_WORDS);
-                row4[0] = make_float4(t.x1, t.y1, t.x2, t.y2);
-                row4[1] = make_float4(t.x3, t.y3, t.z1, t.z2 - t.z1);
-                row4[2] = make_float4(t.z3 - t.z1, t.a, w2, __uint_as_float(w3));
-                RowSpans spans;
-                // row spans cost set-up and per-row work that only boxes of
-                // some width repay; a wavefront walks as long as its widest
-                // box, so it takes them when any lane's box is that wide
-                const bool use_spans = __ballot(bx1 - bx0 + 1 >= (int)SPAN_MIN_W) != 0;
-                if (use_spans) {
-                    if (!given) row_spans_begin(t, bx0, bx1, by0, by1, max(by0, g.tr0), spans);
-                    else row_spans_none(spans);
+                if (bg == ~0u) {
+                    w2 = __float_as_uint(nz / sqrtf(n2) * t.a);
+                    w3 = rgb | dr.ramp;
                 }
+                rows.end[p] = make_uint2(w2, w3);
+                rows.v12[p] = make_float4(t.x1, t.y1, t.x2, t.y2);
+                rows.v3[p] = make_float2(t.x3, t.y3);
+                if constexpr (BIG) rows.depth[p] = make_float4(t.z1 + 0.0f, t.z2 - t.z1, t.z3 - t.z1, t.a);   // no -0, as walk_rect
+                const bool safe = __ballot(given || !depth_safe(t)) == 0;
                 if (bx0 <= bx1 && by0 <= by1) {
-                    auto test = [&](float px, float py, int slot, uint32_t sub) {
-                        float w0, w1, w2;
-                        edges(t, px, py, w0, w1, w2);
-                        const float z = depth(t, w1, w2);
-                        if (inside(w0, w1, w2) && z < F32_MAX)
-                            atomicMin((unsigned long long*)&keys[slot], (unsigned long long)make_tile_key(z, T, sub, p));
+                    auto hit = [&](int slot, float z, uint32_t sub) {
+                        atomicMin((unsigned long long*)&keys[slot], (unsigned long long)make_tile_key(z, T, sub, p));
                     };
+                    constexpr int XS = WRAP ? 2 : 1;
                     if constexpr (BIG) {
                         int xa, xb, ya, yb;
                         direct_rect(g, bx0, bx1, by0, by1, xa, xb, ya, yb);
@@ -1091,16 +1125,16 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                             big_rect =
                                 (uint32_t)xa | ((uint32_t)xb << 8) | ((uint32_t)ya << 16) | ((uint32_t)yb << 24);
                         } else {
-                            if (use_spans)
-                                walk_rect_spans(xa + (g.tc0 >> 1), xb + (g.tc0 >> 1), ya + g.tr0, yb + g.tr0,
-                                                (ya << sws) + xa, sws, 1, spans, test);
+                            if (safe)
+                                walk_rect<XS, false>(t, xa + (g.tc0 >> 1), xb + (g.tc0 >> 1), ya + g.tr0, yb + g.tr0,
+                                                     (ya << sws) + xa, sws, 1u, hit);
                             else
-                                walk_rect(xa + (g.tc0 >> 1), xb + (g.tc0 >> 1), ya + g.tr0, yb + g.tr0,
-                                          (ya << sws) + xa, sws, 1, 1u, test);
+                                walk_rect<XS, true>(t, xa + (g.tc0 >> 1), xb + (g.tc0 >> 1), ya + g.tr0, yb + g.tr0,
+                                                    (ya << sws) + xa, sws, 1u, hit);
                         }
-                        walk_wrapped(g, bx0, bx1, by0, by1, test);
+                        walk_wrapped<XS>(g, t, bx0, bx1, by0, by1, hit);
                     } else {
-                        walk_tile(g, bx0, bx1, by0, by1, use_spans, spans, test);
+                        walk_tile<XS>(g, t, bx0, bx1, by0, by1, safe, hit);
                     }
                 }
             }
@@ -1108,19 +1142,19 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                 // The wavefront's big boxes, one at a time: lane l of the box
                 // takes pixels i = l, l + 64, ... (row i / nx, column i % nx),
                 // with the expressions of edges() and depth() on the box's
-                // cache row (row p of the lane that holds it, written by this
+                // row (row p of the lane that holds it, written by this
                 // wavefront above).
                 uint64_t m = __ballot(big);
                 while (m) {
                     const int l = __builtin_ctzll(m);
                     m &= m - 1;
                     const uint32_t T = __builtin_amdgcn_readlane(big_T, l), rc = __builtin_amdgcn_readlane(big_rect, l);
-                    const uint32_t prow = (threadIdx.x & ~63u) + (uint32_t)l;   // the owner lane's cache row
-                    const float4* row4 = (const float4*)(cache + prow * CACHE_WORDS);
-                    const float4 q0 = row4[0], q1 = row4[1], q2 = row4[2];
-                    const float x1 = q0.x, y1 = q0.y, x2 = q0.z, y2 = q0.w, x3 = q1.x, y3 = q1.y;
+                    const uint32_t prow = (threadIdx.x & ~63u) + (uint32_t)l;   // the owner lane's row
+                    const float4 v12 = rows.v12[prow], q2 = rows.depth[prow];
+                    const float2 v3 = rows.v3[prow];
+                    const float x1 = v12.x, y1 = v12.y, x2 = v12.z, y2 = v12.w, x3 = v3.x, y3 = v3.y;
                     const float A0 = x3 - x2, B0 = y3 - y2, A1 = x1 - x3, B1 = y1 - y3, A2 = x2 - x1, B2 = y2 - y1;
-                    const float z1 = q1.z, dz2 = q1.w, dz3 = q2.x, a = q2.y;
+                    const float z1 = q2.x, dz2 = q2.y, dz3 = q2.z, a = q2.w;
                     const int xa = (int)(rc & 0xFFu), nx = (int)((rc >> 8) & 0xFFu) - xa + 1;
                     const int ya = (int)((rc >> 16) & 0xFFu), ny = (int)(rc >> 24) - ya + 1;
                     const int dy = 64 / nx, dx = 64 - dy * nx;
@@ -1145,50 +1179,105 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                 }
             }
             __syncthreads();
-            if (multi)
-                // slots whose key was written in this chunk (no stored flag)
-                // store that winner and flag the key; a later chunk that
-                // changes the key stores again.  The same thread owns slot s
-                // throughout, so its last store lands last.
-                for_my_slots([&](uint32_t s, int row, uint64_t id) {
-                    const uint64_t k = keys[s];
-                    if (k == KEY_EMPTY || (k & TILE_KEY_STORED)) return;
-                    uint32_t cell;
-                    float z;
-                    winner(my_col, row, k, cell, z);
-                    store(s, row, id, k, cell, z);
-                    keys[s] = k | TILE_KEY_STORED;
-                });
+            if constexpr (WRAP) {
+                if (multi)
+                    // slots whose key was written in this chunk (no stored
+                    // flag) store that winner and flag the key; a later chunk
+                    // that changes the key stores again.  The same thread
+                    // owns slot s throughout, so its last store lands last.
+                    for_my_slots([&](uint32_t s, int row, uint64_t id) {
+                        const uint64_t k = keys[s];
+                        if (k & TILE_KEY_STORED) return;   // or empty
+                        const uint2 w = row_end(k);
+                        uint32_t cell = w.x;
+                        float z = depth_of_code((uint32_t)(k >> 32));
+                        if (!plain(w)) winner_slow(my_col, row, k, cell, z);
+                        store_slot(s, id, k, cell, z);
+                        keys[s] = k | TILE_KEY_STORED;
+                    });
+            } else {
+                if (multi && base + CHUNK < n)
+                    // slots whose key was written in this chunk put their
+                    // cell aside (the rows go to the next chunk); a slot whose
+                    // depth is -0 is remembered for the tile
+                    for (uint32_t s = threadIdx.x; s < S; s += blockDim.x) {
+                        const uint64_t k = keys[s];
+                        if (k & TILE_KEY_STORED) continue;   // or empty
+                        const uint2 w = row_end(k);
+                        uint32_t cell = w.x;
+                        if (!plain(w)) {
+                            float z;
+                            winner_slow(g.tc0 + (int)((s & ((1u << sws) - 1)) << 1), g.tr0 + (int)(s >> sws), k, cell, z);
+                            if (__float_as_uint(z) == 0x80000000u) *s_negz = 1;
+                        }
+                        wcell[s] = cell;
+                        *(uint32_t*)(keys + s) = (uint32_t)k | (uint32_t)TILE_KEY_STORED;
+                    }
+            }
         }
-        if constexpr (ODD) {
+        if constexpr (WRAP) {
             for_my_slots([&](uint32_t s, int row, uint64_t id) {
                 const uint64_t k = keys[s];
-                if (multi && k != KEY_EMPTY) return;   // stored after its chunk
+                if (multi && !tile_empty(k)) return;   // stored after its chunk
                 uint32_t cell = CELL_BLANK;
                 float z = F32_MAX;
-                if (k != KEY_EMPTY) winner(my_col, row, k, cell, z);
-                store(s, row, id, k, cell, z);
+                if (!tile_empty(k)) {
+                    const uint2 w = row_end(k);
+                    cell = w.x;
+                    z = depth_of_code((uint32_t)(k >> 32));
+                    if (!plain(w)) winner_slow(my_col, row, k, cell, z);
+                }
+                store_slot(s, id, k, cell, z);
             });
         } else {
-            for_my_pairs([&](uint32_t s, int row, uint64_t id, int col, bool two) {
-                const uint64_t k0 = keys[s], k1 = two ? keys[s + 1] : KEY_EMPTY;
-                const bool need0 = !(multi && k0 != KEY_EMPTY);   // else stored after its chunk
-                const bool need1 = two && !(multi && k1 != KEY_EMPTY);
-                if (!need0 && !need1) return;
-                uint32_t c0 = CELL_BLANK, c1 = CELL_BLANK;
-                float z0 = F32_MAX, z1 = F32_MAX;
-                if (need0 && k0 != KEY_EMPTY) winner(col, row, k0, c0, z0);
-                if (need1 && k1 != KEY_EMPTY) winner(col + 2, row, k1, c1, z1);
-                store_pair(row, id, col, k0, c0, z0, need0, k1, c1, z1, need1);
+            const bool negz = multi && *s_negz != 0;
+            for_my_pairs([&](uint32_t s, int row, int col, uint32_t off, bool two) {
+                const uint4 kk = *(const uint4*)(keys + s);   // low and high words of the two keys
+                const uint2 w0 = rows.end[kk.x & 0xFFu], w1 = rows.end[kk.z & 0xFFu];
+                uint32_t c0 = w0.x, c1 = w1.x;
+                float z0 = depth_of_code(kk.y), z1 = depth_of_code(kk.w);
+                const bool own0 = !(kk.x & (uint32_t)TILE_KEY_STORED), own1 = !(kk.z & (uint32_t)TILE_KEY_STORED);
+                if (multi) {
+                    const uint2 st = *(const uint2*)(wcell + s);
+                    c0 = own0 ? c0 : st.x;
+                    c1 = own1 ? c1 : st.y;
+                }
+                // the few whose row does not say it all (empty and stored
+                // slots read some row too: never here), one after another
+                uint32_t rest = (own0 && !plain(w0) ? 1u : 0u) | (own1 && !plain(w1) ? 2u : 0u);
+                while (rest) {
+                    const bool second = rest == 2u;
+                    uint32_t cell;
+                    float zz;
+                    winner_slow(second ? col + 2 : col, row,
+                                second ? ((uint64_t)kk.w << 32) | kk.z : ((uint64_t)kk.y << 32) | kk.x, cell, zz);
+                    c0 = second ? c0 : cell;
+                    z0 = second ? z0 : zz;
+                    c1 = second ? cell : c1;
+                    z1 = second ? zz : z1;
+                    rest &= rest - 1;
+                }
+                if (negz) {
+                    // a stored winner's zero depth: its sign from its mesh
+                    for (int i = 0; i < 2; ++i) {
+                        const uint32_t lo = i ? kk.z : kk.x, hi = i ? kk.w : kk.y;
+                        if ((lo & (uint32_t)TILE_KEY_STORED) && hi == DEPTH_CODE_ZERO) {
+                            const float zi = mesh_depth(col + 2 * i, row, lo);
+                            z0 = i ? z0 : zi;
+                            z1 = i ? zi : z1;
+                        }
+                    }
+                }
+                store_pair(row, col, off, two, kk.x, tile_empty(kk.x) ? CELL_BLANK : c0, z0, kk.z,
+                           tile_empty(kk.z) ? CELL_BLANK : c1, z1);
             });
         }
     }
-    if constexpr (ODD) {
+    if constexpr (WRAP) {
         // Each cell: the later write of its own slot's winner and the left
         // slot's (write time = triangle, then the pixel's row and column,
         // as the sequential loop orders them), and for cell 1 the row's
         // newline, which follows its triangle's pixels of that row.
-        const uint64_t* keys = smem;
         const bool any = n > 0;
         if (any) __syncthreads();   // every slot's winner cell is in wcell
         auto slot_time = [&](uint64_t k, int row, int col) -> uint64_t {
@@ -1202,7 +1291,7 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
             uint32_t c_own = CELL_BLANK, best = CELL_BLANK;
             if (any) {
                 const uint64_t k = keys[s];
-                if (k != KEY_EMPTY) {
+                if (!tile_empty(k)) {
                     t_own = slot_time(k, row, my_col);
                     c_own = wcell[s];
                 }
@@ -1210,7 +1299,7 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                 best = c_own;
                 if (my_col > g.tc0) {
                     const uint64_t kl = keys[s - 1];
-                    if (kl != KEY_EMPTY) {
+                    if (!tile_empty(kl)) {
                         const uint64_t tl = slot_time(kl, row, my_col - 1);
                         if (tl > t_best) {
                             t_best = tl;
@@ -1239,15 +1328,11 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
 
 // One workgroup per tile; grid (tile x, tile y, frame - f_lo).  Blocks past a
 // smaller frame's tile grid return at once.
-// Occupancy: LDS allows 7 workgroups of 4 wavefronts per CU.  Left to itself
-// the compiler gives the instances 76-80 VGPRs (6 wavefronts per SIMD); held
-// to 7 they fit 72 and run ~3% faster.  Most fit with SGPR spills to VGPR
-// lanes only; the big-box instance for one draw per frame and the plain one
-// for several spill 2 VGPRs to scratch, still faster than at 6 (a batch of
-// uneven single-draw frames: 0.559 against 0.587 ms).  The big-box instance
-// for several draws per frame would spill more at 72 and keeps 6.
-template <bool BIG, bool ONE, bool ODD, bool FLAT>
-__global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_eu(BIG && !ONE ? 6 : 7, 8))) k_tile_raster(
+// Occupancy: LDS allows 7 workgroups of 4 wavefronts per CU at 64 x 32 cells,
+// and the instances fit the 72 VGPRs of 7 wavefronts per SIMD (1.10 ms for the
+// sweep at 7 wavefronts, 1.18 at 6, and 1.13 at 8, which spill).
+template <bool BIG, bool ONE, bool WRAP, bool FLAT>
+__global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8))) k_tile_raster(
     const Draw* __restrict__ draws, const Ramp* __restrict__ ramps, const Frame* __restrict__ frames, uint32_t f_lo,
     int tws, int ths, uint32_t* __restrict__ cursor, const uint64_t* __restrict__ off,
     const uint32_t* __restrict__ pool, int32_t* __restrict__ nl, const uint4* __restrict__ careful_box,
@@ -1259,6 +1344,7 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
     // the job's first LDS_RAMPS shaders, so that a glyph lookup reads LDS
     // (read only after the tile's first barrier)
     __shared__ Ramp s_ramp[LDS_RAMPS];
+    __shared__ uint32_t s_negz;
 
     // the careful list was read by k_careful, which ran before this launch
     if (careful_reset && (blockIdx.x | blockIdx.y | blockIdx.z | threadIdx.x) == 0) careful_reset[0] = 0;
@@ -1277,7 +1363,7 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
         ty = blockIdx.y;
     }
     const Frame& fr = frames[f];
-    if (tx >= fr.tiles_x || ty >= fr.tiles_y || ((fr.W & 1u) != 0) != ODD) return;
+    if (tx >= fr.tiles_x || ty >= fr.tiles_y || ((fr.W & 1u) != 0) != WRAP) return;
     const uint64_t gt = fr.tile_begin + (uint64_t)ty * fr.tiles_x + tx;
     const uint64_t o = off[gt];
     const uint32_t c = cursor[gt];
@@ -1285,14 +1371,14 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
     if (n > 0)
         for (uint32_t i = threadIdx.x; i < min(n_ramps, LDS_RAMPS) * (uint32_t)sizeof(Ramp) / 4; i += blockDim.x)
             ((uint32_t*)s_ramp)[i] = ((const uint32_t*)ramps)[i];
-    raster_tile<BIG, ONE, ODD, FLAT>(draws, ramps, s_ramp, fr, tx, ty, gt, o, n, tws, ths, pool, nl, careful_box, cells, zbuf,
-                               win, win_raw, edge_out, smem);
+    raster_tile<BIG, ONE, WRAP, FLAT>(draws, ramps, s_ramp, &s_negz, fr, tx, ty, gt, o, n, tws, ths, pool, nl, careful_box,
+                                      cells, zbuf, win, win_raw, edge_out, smem);
     // The tile leaves its binning state as k_tile_clear would for the next
     // render: its cursor at 0 and, for even widths (k_tile_edges reads odd
     // frames' rows after this), the newline rows of its tile row back at -1
     // (the first tile of the row is the one that read them).  Every wave
     // has read the cursor and the rows once the block has met here.
-    const bool reset_nl = !ODD && fr.image && tx == 0;
+    const bool reset_nl = !WRAP && fr.image && tx == 0;
     if (c != 0 || reset_nl) {
         __syncthreads();
         if (c != 0 && threadIdx.x == 0) cursor[gt] = 0;
@@ -1363,17 +1449,22 @@ int TiledPlan::set_tile(uint32_t tw, uint32_t th)
 
 size_t TiledPlan::raster_lds(bool odd) const
 {
-    // keys (8 B per slot), triangle rows; odd widths: a slot per cell and
-    // the slots' winning cells (4 B per slot)
-    size_t S = (size_t)(odd ? TW : TW / 2) * TH;
-    return S * 8 + (size_t)CHUNK * CACHE_WORDS * 4 + (odd ? S * 4 : 0);
+    // keys (8 B per slot), rows, and a cell per slot where a list may be
+    // longer than a chunk; odd widths: a slot and its cell per cell
+    const size_t S = (size_t)(odd ? TW : TW / 2) * TH;
+    return S * 8 + (size_t)CHUNK * row_bytes(!odd && walk()) + (odd || multi ? S * 4 : 0);
 }
 
 bool TiledPlan::tile_fits() const
 {
     // the raster's threads own whole columns of slots: a tile row holds at
-    // most one workgroup's worth (odd widths: a slot per cell)
-    auto fits = [&](bool odd) { return raster_lds(odd) <= 65536 && (odd ? TW : TW / 2) <= (uint32_t)RASTER_BLOCK; };
+    // most one workgroup's worth (odd widths: a slot per cell).  Sizes are
+    // taken or refused for any list: 12 KiB of rows, 8 bytes a slot (12 for
+    // odd widths).
+    auto fits = [&](bool odd) {
+        const size_t S = (size_t)(odd ? TW : TW / 2) * TH;
+        return S * (odd ? 12 : 8) + 12288 <= 65536 && (odd ? TW : TW / 2) <= (uint32_t)RASTER_BLOCK;
+    };
     return (!has_even || fits(false)) && (!has_odd || fits(true));
 }
 
@@ -1571,9 +1662,11 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
         HIP_TRY(hipMemcpyAsync(counts.data(), d_cursor.p, sizeof(uint32_t) * n_tiles, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     off.assign(n_tiles + 1, 0);
+    multi = false;
     for (uint64_t t = 0; t < n_tiles; ++t) {
         uint64_t c = counts[t];
         uint64_t cap = c ? c + c / 8 + 16 : 0;
+        multi = multi || cap > CHUNK;
         off[t + 1] = off[t] + cap;
     }
     if ((rc = d_pool.reserve(sizeof(uint32_t) * std::max<uint64_t>(1, off[n_tiles])))) return rc;
