@@ -3,12 +3,13 @@
 // The W x H cell grid of every frame is cut into TW x TH cell tiles (TW even,
 // tiles start on even columns).  With W even, z slot ids = y*W + 2x are even,
 // so a tile's slots and the two cells each slot writes (id, id+1) never cross
-// a tile edge, and a tile can resolve its cells alone.  Frames of odd width
-// take the raster's odd instance (described there).
+// a tile edge, and a tile can resolve its cells alone.  So can a tile of a frame
+// of odd width that wrapped pixels do not reach; the others take the raster's
+// odd instance (described there).
 //
 //   k_tile_clear   tile cursors <- 0, newline rows <- -1, overflow <- 0,
 //                  careful-list length <- 0; after sizing and before
-//                  renders of odd-width frames only: k_tile_raster leaves
+//                  renders of frames one column wide: k_tile_raster leaves
 //                  what it read in this state for the next render
 //   k_bin          1, 2 or 4 triangles per thread: setup, classification,
 //                  candidate box, newline rows (LDS max per block, one
@@ -56,13 +57,20 @@ constexpr uint32_t PIPE_MIN_FRAMES = 16;  // frames per group at least
 struct TiledPlan {
     uint32_t TW = 64, TH = 32;       // tile size in cells (TW even)
     bool user_tile = false;          // set_tile was called (keeps the size on a re-plan)
-    // Frames of even / odd width in the job.  Each parity has its raster
-    // instance (a launch skips the other parity's frames); odd widths hold a
-    // z slot on every cell column, resolve cells from two slots and finish
-    // first-column cells in k_tile_edges.
+    // Frames of even / odd width in the job.  A frame of odd width has its
+    // first odd_cols() tile columns rendered by the raster's odd instance
+    // (each launch skips the other's tiles), which holds a z slot on every
+    // cell column, resolves cells from two slots and finishes first-column
+    // cells in k_tile_edges.
     bool has_even = true, has_odd = false;
+    // odd_wraps: the tile columns that the counting run's boxes ask for
+    // (odd_cols_of); a later run that finds more raises the overflow flag.
+    // odd_narrow: frames one column wide (only newline cells).
+    uint32_t odd_wraps = 0;
+    bool odd_narrow = false;
+    uint32_t odd_cols() const { return !has_odd ? 0u : odd_narrow && !odd_wraps ? 1u : odd_wraps; }
     bool multi = false;              // set by size(): some tile's list may grow past one chunk of the raster
-    DevBuf d_edges;                  // odd: per tile and row, the first and last column slots' winners
+    DevBuf d_edges;                  // odd_cols() > 0: per tile and row, the first and last column slots' winners
     uint64_t n_tiles = 0;
     uint64_t n_rows = 0;
     bool sized = false;              // pool offsets match the current layout
@@ -122,8 +130,8 @@ struct TiledPlan {
     int set_tile(uint32_t tw, uint32_t th);
     // The raster variant the next launches use (-1 = the sizing run's choice).
     void set_walk(int mode) { walk_force = mode; }
-    // the even-width instance's variant (the odd one has no big-box walk)
-    bool walk() const { return has_even && (walk_force >= 0 ? walk_force == 1 : big_walk); }
+    // the common instance's variant (the odd one has no big-box walk)
+    bool walk() const { return walk_force >= 0 ? walk_force == 1 : big_walk; }
     // Triangles per thread of k_bin: 1, 2 or 4 (set by the autotuner).
     int bin_tpt = 4;
     void set_bin_tpt(int t) { bin_tpt = t; }
@@ -157,6 +165,7 @@ struct TiledPlan {
     int launch_clear(const std::vector<Frame>& frames, uint32_t f_lo, uint32_t f_hi, hipStream_t s);
     int launch_bin(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
                    const Draw* d_draws, uint32_t f_lo, uint32_t f_hi, bool count_only, hipStream_t s);
+    int reserve_edges();
     int launch_careful(const Frame* d_frames, const Draw* d_draws, bool count_only, uint32_t group, hipStream_t s);
     int launch_raster(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames, const Draw* d_draws,
                       const Ramp* d_ramps, uint32_t f_lo, uint32_t f_hi, uint32_t* cells, float* z, int32_t* win,

@@ -19,6 +19,9 @@ constexpr uint32_t BIG_CNT = 2 + MAX_GROUPS;
 // careful_cnt[TALL_CNT]: triangles the counting run finds spanning more than
 // TALL_ROWS rows (TiledPlan::bin_tree)
 constexpr uint32_t TALL_CNT = BIG_CNT + 1;
+// careful_cnt[WRAP_CNT]: the most tile columns odd_cols_of asks for in the
+// counting run (TiledPlan::odd_wraps)
+constexpr uint32_t WRAP_CNT = TALL_CNT + 1;
 constexpr int TALL_ROWS = 16;
 
 // ---------------------------------------------------------------------------
@@ -33,7 +36,8 @@ __global__ void k_tile_clear(uint32_t* __restrict__ cursor, uint64_t n_tiles, in
     for (uint64_t i = i0; i < n_tiles; i += stride) cursor[i] = 0;
     for (uint64_t i = i0; i < n_rows; i += stride) nl[i] = -1;
     for (uint64_t i = i0; i < n_frames; i += stride) overflow[i] = 0;
-    if (i0 == 0) careful_cnt[0] = careful_cnt[1] = careful_cnt[BIG_CNT] = careful_cnt[TALL_CNT] = 0;   // list length, first group's start
+    if (i0 == 0) careful_cnt[0] = careful_cnt[1] = careful_cnt[BIG_CNT] = careful_cnt[TALL_CNT] =
+            careful_cnt[WRAP_CNT] = 0;   // list length, first group's start; the counting run's
 }
 
 // ---------------------------------------------------------------------------
@@ -82,6 +86,17 @@ __device__ __forceinline__ void tile_rects(int bx0, int bx1, int by0, int by1, u
         r.wy0 = (by0 + 1) >> ths;
         r.wy1 = (by1 + 1) >> ths;
     }
+}
+
+// The tile columns of a frame of odd width that the raster's odd instance must
+// take for a box that ends at column bx1: none while it ends before the last
+// cell column (x = W / 2); the first for that column, whose slots' second cells
+// are the next rows' first; and for wrapped columns those they reach and one
+// more, whose first cells may be second cells of the last of them.
+__device__ __forceinline__ int odd_cols_of(int bx1, uint32_t W, int tws)
+{
+    const int last = (int)(W >> 1);
+    return bx1 < last ? 0 : bx1 == last ? 1 : ((2 * bx1 - (int)W) >> tws) + 2;
 }
 
 // Walks a lane's tiles: the direct rectangle, then the wrapped one minus the
@@ -244,7 +259,7 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
                                                    uint32_t* __restrict__ pool, int32_t* __restrict__ nl,
                                                    uint32_t* __restrict__ overflow, uint32_t* __restrict__ careful_cnt,
                                                    uint4* __restrict__ careful_in, uint32_t careful_cap,
-                                                   const uint2* __restrict__ flat_blocks)
+                                                   const uint2* __restrict__ flat_blocks, uint32_t odd_cols)
 {
     __shared__ uint32_t w_cnt[BIN_WIN * BIN_WIN];
     __shared__ uint64_t w_base[BIN_WIN * BIN_WIN];   // pool index of the tile's reserved run
@@ -316,9 +331,10 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
             // addresses.)
             bool has_direct, has_wrap;
             int qx0, qx1, qy0, qy1;
-            if (!__ballot(bx1 >= (int)((W + 1) >> 1))) {
+            if (!__ballot(bx1 >= (int)(W >> 1))) {
                 // no box of the wavefront reaches the wrapped region (x >=
-                // (W + 1) / 2): tile_rects' direct rectangle with x <= bx1
+                // (W + 1) / 2) or an odd frame's last column (x = W / 2):
+                // tile_rects' direct rectangle with x <= bx1
                 has_direct = bx0 <= bx1 && t.y0 < t.y1d;
                 has_wrap = false;
                 qx0 = (2 * bx0) >> tws;
@@ -326,6 +342,13 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
                 qy0 = t.y0 >> ths;
                 qy1 = (t.y1d - 1) >> ths;
             } else {
+                if (W & 1u) {
+                    const uint32_t need = (uint32_t)wave_max(boxed ? odd_cols_of(bx1, W, tws) : 0);
+                    if (__lane_id() == 0) {
+                        if (COUNT) atomicMax(&careful_cnt[WRAP_CNT], need);
+                        else if (need > odd_cols) overflow[frame] = 1u;
+                    }
+                }
                 TileRects r;
                 tile_rects(bx0, bx1, t.y0, t.y1d - 1, W, tws, ths, r);   // empty when bx0 > bx1
                 has_direct = r.dx0 <= r.dx1 && r.dy0 <= r.dy1;
@@ -530,7 +553,7 @@ __device__ __forceinline__ void careful_one(const Frame* __restrict__ frames, in
                                             int ths, uint32_t* __restrict__ cursor, const uint64_t* __restrict__ off,
                                             uint32_t* __restrict__ pool, uint32_t* __restrict__ overflow,
                                             const uint4* __restrict__ careful_in, uint4* __restrict__ careful_box,
-                                            uint32_t w, int lane)
+                                            uint32_t* __restrict__ careful_cnt, uint32_t odd_cols, uint32_t w, int lane)
 {
     // (frame, frame triangle index, screen vertices as k_bin transformed them)
     const uint4 in = careful_in[2 * w], in2 = careful_in[2 * w + 1];
@@ -569,6 +592,12 @@ __device__ __forceinline__ void careful_one(const Frame* __restrict__ frames, in
         careful_box[w] = make_uint4(T, (uint32_t)max(bx0, 0), (uint32_t)max(bx1, 0),
                                     (uint32_t)max(by0, 0) | ((uint32_t)max(by1, 0) << 16));
     if (bx0 > bx1 || by0 > by1) return;
+    if ((fr.W & 1u) && lane == 0) {
+        const uint32_t need = (uint32_t)odd_cols_of(bx1, fr.W, tws);
+        if (COUNT) {
+            if (need) atomicMax(&careful_cnt[WRAP_CNT], need);
+        } else if (need > odd_cols) overflow[frame] = 1u;
+    }
     TileRects r;
     tile_rects(bx0, bx1, by0, by1, fr.W, tws, ths, r);
     const int dw = r.dx1 - r.dx0 + 1, dh = r.dy1 - r.dy0 + 1;
@@ -600,7 +629,8 @@ __global__ void __launch_bounds__(256) k_careful(const Frame* __restrict__ frame
                                                  const uint64_t* __restrict__ off, uint32_t* __restrict__ pool,
                                                  uint32_t* __restrict__ overflow, uint32_t* __restrict__ careful_cnt,
                                                  uint32_t group, const uint4* __restrict__ careful_in,
-                                                 uint4* __restrict__ careful_box, uint32_t careful_cap)
+                                                 uint4* __restrict__ careful_box, uint32_t careful_cap,
+                                                 uint32_t odd_cols)
 {
     const int lane = (int)__lane_id();
     const uint32_t n = min(careful_cnt[0], careful_cap);
@@ -608,7 +638,8 @@ __global__ void __launch_bounds__(256) k_careful(const Frame* __restrict__ frame
     const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
     if (blockIdx.x == 0 && threadIdx.x == 0) careful_cnt[2 + group] = n;
     for (uint32_t w = first + ((blockIdx.x * blockDim.x + threadIdx.x) >> 6); w < n; w += n_waves)
-        careful_one<COUNT>(frames, tws, ths, cursor, off, pool, overflow, careful_in, careful_box, w, lane);
+        careful_one<COUNT>(frames, tws, ths, cursor, off, pool, overflow, careful_in, careful_box, careful_cnt, odd_cols,
+                           w, lane);
 }
 
 
@@ -767,9 +798,16 @@ __device__ __forceinline__ void direct_rect(const TileGeom& g, int bx0, int bx1,
                                             int& ya, int& yb)
 {
     xa = max(bx0, g.tc0 >> 1) - (g.tc0 >> 1);
-    xb = min(bx1, (g.tc1 >> 1) - 1) - (g.tc0 >> 1);
+    xb = min(bx1, (g.tc1 - 1) >> 1) - (g.tc0 >> 1);
     ya = max(by0, g.tr0) - g.tr0;
     yb = min(by1, g.tr1 - 1) - g.tr0;
+}
+
+// Order in which the pixels of a frame are written: by triangle, row, column
+// (0: never).
+__device__ __forceinline__ uint64_t pixel_time(uint32_t T, uint32_t py, uint32_t px)
+{
+    return (((uint64_t)T << 32) | ((uint64_t)py << 16) | px) + 1;
 }
 
 // Triangle index of a pool entry; the candidate box of a careful entry comes
@@ -818,7 +856,16 @@ __device__ __forceinline__ uint32_t entry_tri(uint32_t e, const uint4* __restric
 // same for the whole workgroup and its fields come through scalar loads that
 // do not wait for the list entries.
 //
-// WRAP: frames of odd width.  Every cell column holds a z slot (direct pixels
+// Frames of odd width: slots of direct pixels lie on even columns too, so most
+// of their tiles take the same way as even frames' (rows then start at any
+// 4-byte address, and a tile's last slot may have one cell).  Only wrapped
+// pixels lie on odd columns, and the last column's pixels have their second
+// cell in the next row: the first tile columns, as many as such boxes reach
+// (odd_cols_of), take WRAP.  64 frames of 1919x1079 and 81,920 triangles, whose
+// boxes reach one or two tile columns: 720 us a pass with all tiles WRAP, 420
+// this way (0.06 ms of it the WRAP tiles', 0.007 k_tile_edges').
+//
+// WRAP: those tiles.  Every cell column holds a z slot (direct pixels
 // on even columns, wrapped ones on odd columns) and a cell's final value is
 // the later write of two slots' winners: its own slot's and the one to its
 // left (rasterizer.rs:82-85 writes cells id and id + 1), and the row's
@@ -828,11 +875,13 @@ __device__ __forceinline__ uint32_t entry_tri(uint32_t e, const uint4* __restric
 // is finished by k_tile_edges, from the winners this tile and its left
 // neighbour leave in `edge_out` (first and last column, per row).
 // Tile (tx, ty) of frame fr, global tile index gt, whose list is pool[o, o + n).
-// FLAT is that of the calling kernel and changes nothing here: it gives each
+// KIND: EVEN for launches without odd widths, ANY for those with some, WRAPPED
+// for WRAP tiles.  FLAT is that of the calling kernel and changes nothing here: it gives each
 // kernel its own copy of the lambdas below, which the compiler then inlines
 // as it does for a single caller (shared by the two kernels, they cost the
 // 3-D instances two VGPRs spilled to scratch).
-template <bool BIG, bool ONE, bool WRAP, bool FLAT>
+enum RasterKind { EVEN, ANY, WRAPPED };
+template <bool BIG, bool ONE, RasterKind KIND, bool FLAT>
 __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, const Ramp* __restrict__ ramps,
                                             const Ramp* s_ramp, uint32_t* s_negz, const Frame& fr, uint32_t tx,
                                             uint32_t ty, uint64_t gt, uint64_t o, uint32_t n, int tws, int ths,
@@ -841,6 +890,7 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                                             float* __restrict__ zbuf, int32_t* __restrict__ win, uint32_t win_raw,
                                             uint4* __restrict__ edge_out, uint64_t* smem)
 {
+    constexpr bool WRAP = KIND == WRAPPED;
     static_assert(!(BIG && WRAP), "the big-box walk maps slots of even columns only");
     const uint32_t W = fr.W, H = fr.H;
     const int sws = tws - (WRAP ? 0 : 1);
@@ -895,40 +945,43 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
     // Otherwise a thread takes the slot pairs (2q, 2q + 1) of a row, q = thread
     // mod (slots a row / 2), every (512 >> sws)-th row: fn(first slot, row, its
     // first cell's column, that cell's byte offset from the tile's first cell,
-    // the second slot lies in the frame).  Addresses are the tile's (uniform)
+    // the cells of the four that lie in the frame).  Addresses are the tile's (uniform)
     // plus 32 bits a lane (a tile spans at most 64 rows of 65535 cells).
     auto for_my_pairs = [&](auto&& fn) {
         const uint32_t q = threadIdx.x & ((1u << (sws - 1)) - 1);
         const int col = g.tc0 + ((int)q << 2);
         if (col >= g.tc1) return;
-        const bool two = col + 2 < g.tc1;
+        const int have = KIND == EVEN ? (col + 2 < g.tc1 ? 4 : 2) : min(g.tc1 - col, 4);
         const int step = (int)(blockDim.x >> (sws - 1));
         int r = (int)(threadIdx.x >> (sws - 1));
         uint32_t off = ((uint32_t)r * W + (q << 2)) * 4u;
         for (; r < g.tr1 - g.tr0; r += step, off += (uint32_t)step * W * 4u)
-            fn(((uint32_t)r << sws) | (q << 1), g.tr0 + r, col, off, two);
+            fn(((uint32_t)r << sws) | (q << 1), g.tr0 + r, col, off, have);
     };
     const uint64_t tile0 = (uint64_t)g.tr0 * W + (uint64_t)g.tc0;
     uint8_t* tile_cells = (uint8_t*)(fc + tile0);
     uint8_t* tile_z = (uint8_t*)(fz + tile0);
     uint8_t* tile_win = win ? (uint8_t*)(win + fr.z_off + tile0) : nullptr;
-    // Four words of a pair, or the first two (streaming stores: the frame is
-    // written once and not read back here).  Words need only their own
-    // alignment: a 16-byte store at any 4-byte address is one instruction.
-    auto put = [](uint8_t* p, uint32_t a, uint32_t b, uint32_t c, uint32_t d, bool two) {
-        typedef unsigned int v4u __attribute__((ext_vector_type(4), aligned(4)));
-        typedef unsigned int v2u __attribute__((ext_vector_type(2), aligned(4)));
-        if (two) {
-            const v4u v = {a, b, c, d};
-            __builtin_nontemporal_store(v, (v4u*)p);
-        } else {
+    // Streaming stores: the frame is written once and not read back here.
+    // Words need only their own alignment: a 16-byte store at any 4-byte
+    // address is one instruction.
+    typedef unsigned int v4u __attribute__((ext_vector_type(4), aligned(4)));
+    typedef unsigned int v2u __attribute__((ext_vector_type(2), aligned(4)));
+    auto put4 = [](uint8_t* p, uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+        const v4u v = {a, b, c, d};
+        __builtin_nontemporal_store(v, (v4u*)p);
+    };
+    // the first `have` < 4 words (ANY: 1 and 3 at an odd width's last column)
+    auto put_some = [](uint8_t* p, uint32_t a, uint32_t b, uint32_t c, int have) {
+        if (KIND == EVEN || (have & 2)) {
             const v2u v = {a, b};
             __builtin_nontemporal_store(v, (v2u*)p);
         }
+        if (KIND == ANY && (have & 1)) __builtin_nontemporal_store(have == 1 ? a : c, (uint32_t*)p + (have - 1));
     };
     const bool nl_here = fr.image && tx == 0;
     // Stores a pair from its keys' low words, cells and depths.
-    auto store_pair = [&](int row, int col, uint32_t off, bool two, uint32_t k0, uint32_t c0, float z0, uint32_t k1,
+    auto store_pair = [&](int row, int col, uint32_t off, int have, uint32_t k0, uint32_t c0, float z0, uint32_t k1,
                           uint32_t c1, float z1) {
         uint32_t c0b = c0;
         if (nl_here && col == 0) {
@@ -939,9 +992,26 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
             const int32_t nlr = fnl[row];
             if (nlr >= 0 && (tile_empty(k0) || nlr >= (int32_t)tile_key_tri(k0))) c0b = CELL_NEWLINE;
         }
-        put(tile_cells + off, c0, c0b, c1, c1, two);
-        put(tile_z + off, __float_as_uint(z0), __float_as_uint(F32_MAX), __float_as_uint(z1), __float_as_uint(F32_MAX), two);
-        if (win) put(tile_win + off, win_of(k0), 0xFFFFFFFFu, win_of(k1), 0xFFFFFFFFu, two);
+        if (have == 4) {
+            put4(tile_cells + off, c0, c0b, c1, c1);
+            put4(tile_z + off, __float_as_uint(z0), __float_as_uint(F32_MAX), __float_as_uint(z1), __float_as_uint(F32_MAX));
+            if (win) put4(tile_win + off, win_of(k0), 0xFFFFFFFFu, win_of(k1), 0xFFFFFFFFu);
+            return;
+        }
+        put_some(tile_cells + off, c0, c0b, c1, have);
+        put_some(tile_z + off, __float_as_uint(z0), __float_as_uint(F32_MAX), __float_as_uint(z1), have);
+        if (win) put_some(tile_win + off, win_of(k0), 0xFFFFFFFFu, win_of(k1), have);
+        if (KIND == ANY && edge_out && (have & 1)) {
+            // the last column of an odd width: its second cell is k_tile_edges'
+            const uint32_t k = have == 1 ? k0 : k1;
+            uint4 e = make_uint4(have == 1 ? c0 : c1, 0u, 0u, 0u);
+            if (!tile_empty(k)) {
+                const uint64_t t = pixel_time(tile_key_tri(k), (uint32_t)row, W >> 1);
+                e.z = (uint32_t)t;
+                e.w = (uint32_t)(t >> 32);
+            }
+            edge_out[(gt * (1u << ths) + (uint64_t)(row - g.tr0)) * 2 + 1] = e;
+        }
     };
 
     if (n == 0) {
@@ -950,8 +1020,8 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
         if constexpr (WRAP)
             for_my_slots([&](uint32_t s, int, uint64_t id) { store_slot(s, id, TILE_EMPTY, CELL_BLANK, F32_MAX); });
         else
-            for_my_pairs([&](uint32_t, int row, int col, uint32_t off, bool two) {
-                store_pair(row, col, off, two, ~0u, CELL_BLANK, F32_MAX, ~0u, CELL_BLANK, F32_MAX);
+            for_my_pairs([&](uint32_t, int row, int col, uint32_t off, int have) {
+                store_pair(row, col, off, have, ~0u, CELL_BLANK, F32_MAX, ~0u, CELL_BLANK, F32_MAX);
             });
     } else {
         // glyph of shade sh under shader r: the first LDS_RAMPS shaders from
@@ -1231,7 +1301,7 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
             });
         } else {
             const bool negz = multi && *s_negz != 0;
-            for_my_pairs([&](uint32_t s, int row, int col, uint32_t off, bool two) {
+            for_my_pairs([&](uint32_t s, int row, int col, uint32_t off, int have) {
                 const uint4 kk = *(const uint4*)(keys + s);   // low and high words of the two keys
                 const uint2 w0 = rows.end[kk.x & 0xFFu], w1 = rows.end[kk.z & 0xFFu];
                 uint32_t c0 = w0.x, c1 = w1.x;
@@ -1268,7 +1338,7 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                         }
                     }
                 }
-                store_pair(row, col, off, two, kk.x, tile_empty(kk.x) ? CELL_BLANK : c0, z0, kk.z,
+                store_pair(row, col, off, have, kk.x, tile_empty(kk.x) ? CELL_BLANK : c0, z0, kk.z,
                            tile_empty(kk.z) ? CELL_BLANK : c1, z1);
             });
         }
@@ -1284,7 +1354,7 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
             const uint32_t sub = tile_key_sub(k);
             const uint32_t py = sub ? (uint32_t)row : (uint32_t)row - 1u;
             const uint32_t px = sub ? (uint32_t)col >> 1 : (uint32_t)(col + (int)W) >> 1;
-            return (((uint64_t)tile_key_tri(k) << 32) | ((uint64_t)py << 16) | px) + 1;
+            return pixel_time(tile_key_tri(k), py, px);
         };
         for_my_slots([&](uint32_t s, int row, uint64_t id) {
             uint64_t t_own = 0, t_best = 0;
@@ -1326,19 +1396,40 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
         for (uint32_t i = threadIdx.x; i < H; i += blockDim.x) __builtin_nontemporal_store(CELL_BLANK, fc + (uint64_t)W * H + i);
 }
 
+// The tile of a frame's workgroup r, ANY: workgroups go to the eight XCDs in
+// turn, so taking eight tile rows at a time gives each XCD, and its L2, whole
+// rows.  The rows of an odd width start at any 4-byte address, and the lines
+// that two tiles of a row share are then put together before they leave for
+// memory: 64 frames of 1919x1079 at 128 x 16 cells 474 -> 416 us, at 32 x 32
+// 1020 -> 727.  Even widths' tiles share no line: 256 frames of 1920x1080 lose
+// (1.79 -> 1.825 ms), so they keep the plain order.
+__device__ __forceinline__ void tile_of(uint32_t r, uint32_t nx, uint32_t ny, uint32_t& tx, uint32_t& ty)
+{
+    const uint32_t full = (ny & ~7u) * nx;
+    if (r < full) {
+        const uint32_t j = r >> 3, g = j / nx;
+        tx = j - g * nx;
+        ty = 8u * g + (r & 7u);
+    } else {
+        const uint32_t j = r - full, g = j / nx;
+        tx = j - g * nx;
+        ty = (ny & ~7u) + g;
+    }
+}
+
 // One workgroup per tile; grid (tile x, tile y, frame - f_lo).  Blocks past a
 // smaller frame's tile grid return at once.
 // Occupancy: LDS allows 7 workgroups of 4 wavefronts per CU at 64 x 32 cells,
 // and the instances fit the 72 VGPRs of 7 wavefronts per SIMD (1.10 ms for the
 // sweep at 7 wavefronts, 1.18 at 6, and 1.13 at 8, which spill).
-template <bool BIG, bool ONE, bool WRAP, bool FLAT>
+template <bool BIG, bool ONE, RasterKind KIND, bool FLAT>
 __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8))) k_tile_raster(
     const Draw* __restrict__ draws, const Ramp* __restrict__ ramps, const Frame* __restrict__ frames, uint32_t f_lo,
     int tws, int ths, uint32_t* __restrict__ cursor, const uint64_t* __restrict__ off,
     const uint32_t* __restrict__ pool, int32_t* __restrict__ nl, const uint4* __restrict__ careful_box,
     uint32_t* __restrict__ cells, float* __restrict__ zbuf, int32_t* __restrict__ win, uint32_t win_raw,
     uint32_t n_ramps, uint4* __restrict__ edge_out, uint32_t* __restrict__ careful_reset,
-    const uint2* __restrict__ tile_frame, uint32_t t_lo)
+    const uint2* __restrict__ tile_frame, uint32_t t_lo, uint32_t odd_cols)
 {
     extern __shared__ uint64_t smem[];
     // the job's first LDS_RAMPS shaders, so that a glyph lookup reads LDS
@@ -1361,9 +1452,12 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
         f = f_lo + blockIdx.z;
         tx = blockIdx.x;
         ty = blockIdx.y;
+        if constexpr (KIND == ANY) tile_of(ty * gridDim.x + tx, gridDim.x, gridDim.y, tx, ty);
     }
     const Frame& fr = frames[f];
-    if (tx >= fr.tiles_x || ty >= fr.tiles_y || ((fr.W & 1u) != 0) != WRAP) return;
+    constexpr bool WRAP = KIND == WRAPPED;
+    if (tx >= fr.tiles_x || ty >= fr.tiles_y) return;
+    if (KIND != EVEN && ((fr.W & 1u) && tx < odd_cols) != WRAP) return;
     const uint64_t gt = fr.tile_begin + (uint64_t)ty * fr.tiles_x + tx;
     const uint64_t o = off[gt];
     const uint32_t c = cursor[gt];
@@ -1371,14 +1465,14 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
     if (n > 0)
         for (uint32_t i = threadIdx.x; i < min(n_ramps, LDS_RAMPS) * (uint32_t)sizeof(Ramp) / 4; i += blockDim.x)
             ((uint32_t*)s_ramp)[i] = ((const uint32_t*)ramps)[i];
-    raster_tile<BIG, ONE, WRAP, FLAT>(draws, ramps, s_ramp, &s_negz, fr, tx, ty, gt, o, n, tws, ths, pool, nl, careful_box,
+    raster_tile<BIG, ONE, KIND, FLAT>(draws, ramps, s_ramp, &s_negz, fr, tx, ty, gt, o, n, tws, ths, pool, nl, careful_box,
                                       cells, zbuf, win, win_raw, edge_out, smem);
     // The tile leaves its binning state as k_tile_clear would for the next
-    // render: its cursor at 0 and, for even widths (k_tile_edges reads odd
-    // frames' rows after this), the newline rows of its tile row back at -1
+    // render: its cursor at 0 and, but for frames one column wide (k_tile_edges
+    // reads their rows after this), the newline rows of its tile row back at -1
     // (the first tile of the row is the one that read them).  Every wave
     // has read the cursor and the rows once the block has met here.
-    const bool reset_nl = !WRAP && fr.image && tx == 0;
+    const bool reset_nl = fr.image && tx == 0 && !(WRAP && fr.W == 1);
     if (c != 0 || reset_nl) {
         __syncthreads();
         if (c != 0 && threadIdx.x == 0) cursor[gt] = 0;
@@ -1389,7 +1483,7 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
     }
 }
 
-// Frames of odd width: the first-column cells of the tiles.  Cell (r, c)
+// Frames of odd width: the first-column cells of the odd instance's tiles.  Cell (r, c)
 // with c the first column of a tile is the later write of slot (r, c)'s
 // winner and slot (r, c - 1)'s, which the tile to the left holds; cell
 // (r, 0) takes the last slot of row r - 1 instead (id + 1 of the row's last
@@ -1397,7 +1491,7 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
 // column slot's winning cell and write time in `edges` (time 0: none).  A
 // frame one column wide has no pixels (the domain's x range is empty), and
 // its cell (r, 0) is row r - 1's newline cell (r - 1) * W + 1.
-// Grid (rows / 256, tile columns, frame - f_lo).
+// Grid (rows / 256, odd_cols, frame - f_lo).
 __global__ void __launch_bounds__(256) k_tile_edges(const Frame* __restrict__ frames, uint32_t f_lo, int tws,
                                                     int ths, const uint4* __restrict__ edges,
                                                     const int32_t* __restrict__ nl, uint32_t* __restrict__ cells)
@@ -1488,7 +1582,11 @@ TiledPlan::Range TiledPlan::range(const std::vector<Frame>& frames, const std::v
 int TiledPlan::plan(std::vector<Frame>& frames, const std::vector<Draw>& draws, uint64_t rows)
 {
     bool ev = false, od = false;
-    for (const Frame& f : frames) ((f.W & 1u) ? od : ev) = true;
+    odd_narrow = false;
+    for (const Frame& f : frames) {
+        ((f.W & 1u) ? od : ev) = true;
+        odd_narrow = odd_narrow || f.W == 1;
+    }
     if (ev != has_even || od != has_odd) sized = false;
     has_even = ev;
     has_odd = od;
@@ -1515,9 +1613,13 @@ int TiledPlan::plan(std::vector<Frame>& frames, const std::vector<Draw>& draws, 
     if ((rc = d_cursor.reserve(sizeof(uint32_t) * std::max<uint64_t>(1, n_tiles)))) return rc;
     if ((rc = d_off.reserve(sizeof(uint64_t) * (n_tiles + 1)))) return rc;
     if ((rc = d_nl.reserve(sizeof(int32_t) * std::max<uint64_t>(1, n_rows)))) return rc;
-    if ((rc = d_careful_cnt.reserve(sizeof(uint32_t) * (TALL_CNT + 1)))) return rc;
-    if (has_odd && (rc = d_edges.reserve(sizeof(uint4) * 2 * std::max<uint64_t>(1, n_tiles) * TH))) return rc;
-    return SLOTH_OK;
+    if ((rc = d_careful_cnt.reserve(sizeof(uint32_t) * (WRAP_CNT + 1)))) return rc;
+    return reserve_edges();
+}
+
+int TiledPlan::reserve_edges()
+{
+    return odd_cols() ? d_edges.reserve(sizeof(uint4) * 2 * std::max<uint64_t>(1, n_tiles) * TH) : SLOTH_OK;
 }
 
 int TiledPlan::launch_clear(const std::vector<Frame>& frames, uint32_t f_lo, uint32_t f_hi, hipStream_t s)
@@ -1545,7 +1647,7 @@ int TiledPlan::launch_bin(const std::vector<Frame>& frames, const std::vector<Dr
             hipLaunchKernelGGL(kernel, grid, dim3(BIN_BLOCK), 0, s, d_draws, d0, d_frames, tws, ths,
                                d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
                                d_nl.as<int32_t>(), overflow, d_careful_cnt.as<uint32_t>(),
-                               d_careful_in.as<uint4>(), careful_cap, flat);
+                               d_careful_in.as<uint4>(), careful_cap, flat, odd_cols());
         };
         // the counting run takes the tree variant (it counts the tall triangles)
         if (bin_tpt == 1)
@@ -1588,12 +1690,12 @@ int TiledPlan::launch_careful(const Frame* d_frames, const Draw* d_draws, bool c
         hipLaunchKernelGGL(k_careful<true>, grid, dim3(256), 0, s, d_frames, tws, ths,
                            d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
                            overflow, d_careful_cnt.as<uint32_t>(), group, d_careful_in.as<uint4>(),
-                           d_careful_box.as<uint4>(), careful_cap);
+                           d_careful_box.as<uint4>(), careful_cap, odd_cols());
     else
         hipLaunchKernelGGL(k_careful<false>, grid, dim3(256), 0, s, d_frames, tws, ths,
                            d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
                            overflow, d_careful_cnt.as<uint32_t>(), group, d_careful_in.as<uint4>(),
-                           d_careful_box.as<uint4>(), careful_cap);
+                           d_careful_box.as<uint4>(), careful_cap, odd_cols());
     HIP_TRY(hipGetLastError());
     return SLOTH_OK;
 }
@@ -1631,7 +1733,7 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     // 1. count tile entries of CLS_BOX triangles and the careful triangles
     if ((rc = launch_clear(frames, 0, F, s))) return rc;
     if ((rc = launch_bin(frames, draws, d_frames, d_draws, 0, F, true, s))) return rc;
-    uint32_t cnt[TALL_CNT + 1];
+    uint32_t cnt[WRAP_CNT + 1];
     HIP_TRY(hipMemcpyAsync(cnt, d_careful_cnt.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     const uint32_t n_careful = cnt[0];
@@ -1660,7 +1762,10 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     std::vector<uint32_t> counts(n_tiles);
     if (n_tiles)
         HIP_TRY(hipMemcpyAsync(counts.data(), d_cursor.p, sizeof(uint32_t) * n_tiles, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(cnt, d_careful_cnt.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
+    odd_wraps = cnt[WRAP_CNT];
+    if ((rc = reserve_edges())) return rc;
     off.assign(n_tiles + 1, 0);
     multi = false;
     for (uint64_t t = 0; t < n_tiles; ++t) {
@@ -1705,18 +1810,21 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     return SLOTH_OK;
 }
 
-// The raster instance for a width parity: big-box walk or not, one draw per
-// frame or not, flat grid (frames of different tile grids) or 3-D.  Each
-// instance is compiled on its own, so the 3-D instances carry no flat-grid
-// mapping and its registers.
-template <bool ODD, bool FLAT>
+// The common raster instance: with odd widths or not, big-box walk or not, one
+// draw per frame or not, flat grid (frames of different tile grids) or 3-D.  Each instance is compiled
+// on its own, so the 3-D instances carry no flat-grid mapping and its
+// registers.
+template <bool FLAT, RasterKind KIND>
 static auto raster_kernel(bool walk, bool one)
 {
-    if constexpr (ODD)
-        return one ? k_tile_raster<false, true, true, FLAT> : k_tile_raster<false, false, true, FLAT>;
-    else
-        return walk ? (one ? k_tile_raster<true, true, false, FLAT> : k_tile_raster<true, false, false, FLAT>)
-                    : (one ? k_tile_raster<false, true, false, FLAT> : k_tile_raster<false, false, false, FLAT>);
+    return walk ? (one ? k_tile_raster<true, true, KIND, FLAT> : k_tile_raster<true, false, KIND, FLAT>)
+                : (one ? k_tile_raster<false, true, KIND, FLAT> : k_tile_raster<false, false, KIND, FLAT>);
+}
+
+template <bool FLAT>
+static auto raster_kernel(bool walk, bool one, bool odd)
+{
+    return odd ? raster_kernel<FLAT, ANY>(walk, one) : raster_kernel<FLAT, EVEN>(walk, one);
 }
 
 int TiledPlan::launch_raster(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
@@ -1733,10 +1841,11 @@ int TiledPlan::launch_raster(const std::vector<Frame>& frames, const std::vector
         const Range rg = range(frames, draws, f0, f1);
         const uint32_t mx = rg.tiles_x, my = rg.tiles_y;
         if (mx == 0 || my == 0) continue;
-        const bool one = rg.one, ev = rg.even, od = rg.odd;
-        // one launch per width parity in the range; each skips the other's
-        // frames.  The grid: (tile x, tile y, frame) over the largest tile
-        // grid, or one workgroup per tile when the frames' tile grids differ
+        // one launch for the common instance's tiles and one for the odd
+        // one's; each skips the other's.  The grid: (tile x, tile y, frame)
+        // over the largest tile grid, or one workgroup per tile when the
+        // frames' tile grids differ
+        const bool one = rg.one, od = rg.odd && odd_cols(), ev = rg.even || !od || mx > odd_cols();
         const uint64_t t_lo = frames[f0].tile_begin;
         const uint64_t t_hi = frames[f1 - 1].tile_begin + (uint64_t)frames[f1 - 1].tiles_x * frames[f1 - 1].tiles_y;
         if (flat_raster && t_hi > 0x7FFFFFFFull) return fail(SLOTH_EINVAL, "too many tiles for a flat raster grid");
@@ -1744,26 +1853,25 @@ int TiledPlan::launch_raster(const std::vector<Frame>& frames, const std::vector
         const uint2* tf = !flat_raster ? nullptr
                           : f0 == 0 && f1 == (uint32_t)frames.size() ? d_tile_heavy.as<uint2>()
                                                                       : d_tile_frame.as<uint2>();
-        if (ev) {
-            const auto kern = flat_raster ? raster_kernel<false, true>(walk(), one) : raster_kernel<false, false>(walk(), one);
-            hipLaunchKernelGGL(kern, grid, dim3(RASTER_BLOCK), raster_lds(false), s, d_draws,
-                               d_ramps, d_frames, f0, log2u(TW), log2u(TH), d_cursor.as<uint32_t>(),
-                               d_off.as<uint64_t>(), d_pool.as<uint32_t>(), d_nl.as<int32_t>(),
-                               d_careful_box.as<uint4>(), cells, z, win, win_raw ? 1u : 0u, n_ramps, (uint4*)nullptr,
-                               careful_reset, tf, (uint32_t)t_lo);
-            HIP_TRY(hipGetLastError());
+        uint4* edges = od ? d_edges.as<uint4>() : nullptr;
+        auto go = [&](auto kern, dim3 grid, size_t lds) {
+            hipLaunchKernelGGL(kern, grid, dim3(RASTER_BLOCK), lds, s, d_draws, d_ramps, d_frames, f0, log2u(TW),
+                               log2u(TH), d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
+                               d_nl.as<int32_t>(), d_careful_box.as<uint4>(), cells, z, win, win_raw ? 1u : 0u,
+                               n_ramps, edges, careful_reset, tf, (uint32_t)t_lo, odd_cols());
             careful_reset = nullptr;
+        };
+        if (ev) {
+            go(flat_raster ? raster_kernel<true>(walk(), one, rg.odd) : raster_kernel<false>(walk(), one, rg.odd), grid,
+               raster_lds(false));
+            HIP_TRY(hipGetLastError());
         }
         if (od) {
-            const auto kern = flat_raster ? raster_kernel<true, true>(false, one) : raster_kernel<true, false>(false, one);
-            hipLaunchKernelGGL(kern, grid, dim3(RASTER_BLOCK), raster_lds(true), s, d_draws,
-                               d_ramps, d_frames, f0, log2u(TW), log2u(TH), d_cursor.as<uint32_t>(),
-                               d_off.as<uint64_t>(), d_pool.as<uint32_t>(), d_nl.as<int32_t>(),
-                               d_careful_box.as<uint4>(), cells, z, win, win_raw ? 1u : 0u, n_ramps,
-                               d_edges.as<uint4>(), careful_reset, tf, (uint32_t)t_lo);
+            const unsigned nx = std::min(odd_cols(), mx);
+            go(one ? k_tile_raster<false, true, WRAPPED, false> : k_tile_raster<false, false, WRAPPED, false>,
+               dim3(nx, my, f1 - f0), raster_lds(true));
             HIP_TRY(hipGetLastError());
-            careful_reset = nullptr;
-            hipLaunchKernelGGL(k_tile_edges, dim3(blocks(rg.H, 256), mx, f1 - f0), dim3(256), 0, s, d_frames, f0,
+            hipLaunchKernelGGL(k_tile_edges, dim3(blocks(rg.H, 256), nx, f1 - f0), dim3(256), 0, s, d_frames, f0,
                                log2u(TW), log2u(TH), (const uint4*)d_edges.as<uint4>(),
                                (const int32_t*)d_nl.as<int32_t>(), cells);
             HIP_TRY(hipGetLastError());
@@ -1792,11 +1900,10 @@ int TiledPlan::launch(const std::vector<Frame>& frames, const std::vector<Draw>&
         // Every render leaves the tile cursors, the even frames' newline
         // rows and the careful list's length as k_tile_clear sets them
         // (k_tile_raster resets what it has read; size() ends with a
-        // clear), so only ranges with odd widths, whose newline rows
-        // k_tile_edges reads after the raster, are cleared first.
-        const bool odd = range(frames, draws, f_lo, f_hi).odd;
+        // clear), but for frames one column wide, whose newline rows
+        // k_tile_edges reads after the raster.
         if (ev) HIP_TRY(hipEventRecord((*ev)[0], s));
-        if (odd && (rc = launch_clear(frames, f_lo, f_hi, s))) return rc;
+        if (odd_narrow && (rc = launch_clear(frames, f_lo, f_hi, s))) return rc;
         if (ev) HIP_TRY(hipEventRecord((*ev)[1], s));
         if ((rc = launch_bin(frames, draws, d_frames, d_draws, f_lo, f_hi, false, s))) return rc;
         if (ev) HIP_TRY(hipEventRecord((*ev)[2], s));
