@@ -375,17 +375,30 @@ struct Job {
         for (uint32_t d = d_lo; d < d_hi; ++d) max_n = std::max(max_n, draws[d].n);
         for (uint32_t d = d_lo; d < d_hi && max_n; d += 65535u) {
             const uint32_t nd = std::min<uint32_t>(65535u, d_hi - d);
-            hipLaunchKernelGGL(k_raster_global, dim3(blocks_for(max_n), nd), dim3(256), 0, s, dev_draws(), d,
-                               dev_frames(), d_keys.as<uint64_t>(), d_nl.as<int32_t>());
+            hipLaunchKernelGGL(k_raster_global, dim3(blocks_for(max_n, RASTER_GLOBAL_BLOCK), nd),
+                               dim3(RASTER_GLOBAL_BLOCK), 0, s, dev_draws(), d, dev_frames(), d_keys.as<uint64_t>(), d_nl.as<int32_t>());
             HIP_TRY(hipGetLastError());
         }
         if (ev) HIP_TRY(hipEventRecord((*ev)[2], s));
         // grids (cells of the largest frame / 256, frames), at most 65535
         // frames per launch
-        uint64_t max_wh = 0, max_cells = 0;
+        uint64_t max_wh = 0, max_cells = 0, max_even = 0;   // of odd and of even widths
         for (uint32_t f = f_lo; f < f_hi; ++f) {
-            max_wh = std::max<uint64_t>(max_wh, (uint64_t)frames[f].W * frames[f].H);
-            max_cells = std::max<uint64_t>(max_cells, frame_cells(frames[f]));
+            const uint64_t wh = (uint64_t)frames[f].W * frames[f].H, n = frame_cells(frames[f]);
+            if (frames[f].W & 1u) {
+                max_wh = std::max(max_wh, wh);
+                max_cells = std::max(max_cells, n);
+            } else {
+                max_even = std::max(max_even, n - wh / 2);
+            }
+        }
+        for (uint32_t f = f_lo; f < f_hi && max_even; f += 65535u) {
+            const uint32_t nf = std::min<uint32_t>(65535u, f_hi - f);
+            hipLaunchKernelGGL(k_finish_global, dim3(blocks_for(max_even), nf), dim3(256), 0, s, dev_draws(),
+                               dev_ramps(), dev_frames(), f, (const uint64_t*)d_keys.as<uint64_t>(),
+                               (const int32_t*)d_nl.as<int32_t>(), d_cells.as<uint32_t>(), d_z.as<float>(), win,
+                               win_raw ? 1u : 0u);
+            HIP_TRY(hipGetLastError());
         }
         for (uint32_t f = f_lo; f < f_hi && max_wh; f += 65535u) {
             const uint32_t nf = std::min<uint32_t>(65535u, f_hi - f);
@@ -1950,12 +1963,20 @@ int sloth::noalloc_init(int dev)
 }
 
 // Writes the launch's tables into scratch from kernel arguments (no host
-// buffer has to outlive the call).
-__global__ void k_noalloc_tables(Frame f, Draw d, Ramp r, uint8_t* base)
+// buffer has to outlive the call), and empties the frame's n_keys keys and
+// n_rows newline entries: the scratch holds whatever the previous call on this
+// device left.
+__global__ void __launch_bounds__(256) k_noalloc_begin(Frame f, Draw d, Ramp r, uint8_t* base, uint32_t n_keys,
+                                                       uint32_t n_rows)
 {
-    if (threadIdx.x == 0) *(Frame*)base = f;
-    if (threadIdx.x == 1) *(Draw*)(base + 256) = d;
-    if (threadIdx.x == 2) *(Ramp*)(base + 512) = r;
+    uint64_t* keys = (uint64_t*)(base + NOALLOC_TABLE_BYTES);
+    int32_t* nl = (int32_t*)(base + NOALLOC_TABLE_BYTES + NOALLOC_KEY_BYTES);
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n_keys) keys[i] = KEY_EMPTY;
+    if (i < n_rows) nl[i] = -1;
+    if (i == 0) *(Frame*)base = f;
+    if (i == 1) *(Draw*)(base + 256) = d;
+    if (i == 2) *(Ramp*)(base + 512) = r;
 }
 
 extern "C" {
@@ -2007,19 +2028,22 @@ int sloth_render_frame_noalloc(const float* d_positions, const uint8_t* d_colors
     int32_t* nl = (int32_t*)(base + NOALLOC_TABLE_BYTES + NOALLOC_KEY_BYTES);
     const uint64_t cells = frame_cells(f);
 
-    hipLaunchKernelGGL(k_noalloc_tables, dim3(1), dim3(64), 0, s, f, d, r, base);
+    // frames of even width hold a key per even cell id (key_at)
+    const bool even = (width & 1u) == 0;
+    const uint32_t n_keys = (uint32_t)(even ? WH / 2 : WH);
+    hipLaunchKernelGGL(k_noalloc_begin, dim3(Job::blocks_for(std::max(n_keys, height))), dim3(256), 0, s, f, d, r, base,
+                       n_keys, height);
     HIP_TRY(hipGetLastError());
-    {
-        // every key and newline entry of this frame starts empty: the scratch
-        // holds whatever the previous call on this device left
-        const unsigned g = std::max(1u, std::min<unsigned>(Job::blocks_for(std::max<uint64_t>(WH, height)), 8192u));
-        hipLaunchKernelGGL(k_clear_global, dim3(g), dim3(256), 0, s, keys, WH, nl, (uint64_t)height);
+    if (n) {
+        hipLaunchKernelGGL(k_raster_global, dim3(Job::blocks_for(n, RASTER_GLOBAL_BLOCK), 1),
+                           dim3(RASTER_GLOBAL_BLOCK), 0, s, d_draw, 0u, d_frame, keys, nl);
         HIP_TRY(hipGetLastError());
     }
-    if (n) {
-        hipLaunchKernelGGL(k_raster_global, dim3(Job::blocks_for(n), 1), dim3(256), 0, s, d_draw, 0u, d_frame, keys,
-                           nl);
+    if (even) {
+        hipLaunchKernelGGL(k_finish_global, dim3(Job::blocks_for(cells - WH / 2), 1), dim3(256), 0, s, d_draw, d_ramp,
+                           d_frame, 0u, (const uint64_t*)keys, (const int32_t*)nl, d_cells, d_z, (int32_t*)nullptr, 0u);
         HIP_TRY(hipGetLastError());
+        return SLOTH_OK;
     }
     hipLaunchKernelGGL(k_winner_global, dim3(Job::blocks_for(WH), 1), dim3(256), 0, s, d_draw, d_ramp, d_frame, 0u,
                        keys, d_z, (int32_t*)nullptr, 0u);

@@ -5,12 +5,21 @@
 //                     candidate pixels, 64-bit atomicMin of the packed key
 //                     into the frame's z-slot keys; newline rows by atomicMax,
 //                     reduced per block in LDS first
-//   k_winner_global   one thread per z slot: the winning fragment's cell and
-//                     depth, derived once from the slot's key; the depth and
-//                     winner go out, and the key's depth half is replaced by
-//                     the cell (the triangle and sub half stays)
-//   k_resolve_global  one thread per cell: last writer among the winners of
-//                     z slots c and c-1 and the row's newline
+//   k_finish_global   frames of even width, one thread per z slot: the winning
+//                     fragment's cell and depth from the slot's key, and the
+//                     slot's two cells, depths and winners written
+//   k_winner_global   frames of odd width, one thread per z slot: the winning
+//                     fragment's cell and depth, derived once from the slot's
+//                     key; the depth and winner go out, and the key's depth
+//                     half is replaced by the cell (the triangle and sub half
+//                     stays)
+//   k_resolve_global  frames of odd width, one thread per cell: last writer
+//                     among the winners of z slots c and c-1 and the row's
+//                     newline
+//
+// With an even width every z slot id y*W + 2x is even and owns the cells id and
+// id + 1: the keys lie densely (key_at), so that the atomics of neighbouring
+// pixels share more lines, and no cell has two slots to choose from.
 //
 // The order-independent packed key makes the result deterministic and equal
 // to the sequential loop of rasterizer.rs:43-45, 69-92.
@@ -28,6 +37,9 @@ __global__ void k_clear_global(uint64_t* __restrict__ keys, uint64_t n_keys, int
         nl[i] = -1;
 }
 
+// Index of a z slot's key among its frame's.
+__device__ __forceinline__ uint32_t key_at(uint32_t id, uint32_t W) { return id >> (~W & 1u); }
+
 __device__ __forceinline__ void plot(uint64_t* __restrict__ keys, const Tri& t, uint32_t W, uint32_t tri, int x,
                                      int y)
 {
@@ -38,16 +50,22 @@ __device__ __forceinline__ void plot(uint64_t* __restrict__ keys, const Tri& t, 
     if (!(z < F32_MAX)) return;   // the initial z-buffer value never loses; NaN never wins
     uint32_t id = (uint32_t)y * W + 2u * (uint32_t)x;
     uint32_t sub = (2u * (uint32_t)x < W) ? 1u : 0u;
-    atomicMin((unsigned long long*)&keys[id], (unsigned long long)make_key(z, tri, sub));
+    atomicMin((unsigned long long*)&keys[key_at(id, W)], (unsigned long long)make_key(z, tri, sub));
 }
 
 // Grid: x = blocks of one draw's triangles, y = draw index - d_lo, so the
 // draw, its frame and its matrix are uniform per block (scalar loads).
-__global__ void __launch_bounds__(256) k_raster_global(const Draw* __restrict__ draws, uint32_t d_lo,
+//
+// What bounds it: a small mesh leaves little more than a wavefront per SIMD, so
+// one triangle's chain (mesh, set-up, rows, box) and the key atomics at memory
+// add up: 81,920 triangles into 1280x720 take 15.6 us, 10 without the atomics.
+// (16.6 us in blocks of 256, 15.8 in blocks of 64; 21.1 with the rows' range by
+// an LDS atomic per lane and the keys of even widths twice as far apart.)
+__global__ void __launch_bounds__(RASTER_GLOBAL_BLOCK) k_raster_global(const Draw* __restrict__ draws, uint32_t d_lo,
                                                        const Frame* __restrict__ frames, uint64_t* __restrict__ keys,
                                                        int32_t* __restrict__ nl)
 {
-    __shared__ int32_t s_nl[256];
+    __shared__ int32_t s_nl[RASTER_GLOBAL_BLOCK];
     __shared__ int s_lo, s_hi;
     const Draw& dr = draws[d_lo + blockIdx.y];
     const uint32_t base = blockIdx.x * blockDim.x;
@@ -65,8 +83,9 @@ __global__ void __launch_bounds__(256) k_raster_global(const Draw* __restrict__ 
 
     // rasterizer.rs:89-91: every row of the domain ends with a newline cell;
     // the last triangle (in draw order) whose rows include r decides row r.
-    // The block reduces its rows in LDS, 256 rows at a time, with one global
-    // atomicMax per row and window.
+    // The block reduces its rows in LDS, a row a thread at a time, with one global
+    // atomicMax per row and window; their range comes from one LDS atomic per
+    // wavefront (lanes that meet on one address take turns).
     const bool has_rows = valid && fr.image && t.y0 < t.y1d;
     int32_t* fnl = nl + fr.nl_off;
     s_nl[threadIdx.x] = -1;
@@ -75,9 +94,10 @@ __global__ void __launch_bounds__(256) k_raster_global(const Draw* __restrict__ 
         s_hi = -1;
     }
     __syncthreads();
-    if (has_rows) {
-        atomicMin(&s_lo, t.y0);
-        atomicMax(&s_hi, t.y1d - 1);
+    const int wlo = wave_min(has_rows ? t.y0 : 1 << 30), whi = wave_max(has_rows ? t.y1d - 1 : -1);
+    if (__lane_id() == 0 && whi >= 0) {
+        atomicMin(&s_lo, wlo);
+        atomicMax(&s_hi, whi);
     }
     __syncthreads();
     const int lo = s_lo, hi = s_hi;   // uniform per block
@@ -154,12 +174,61 @@ __device__ __forceinline__ void winner_fragment(const Draw* __restrict__ draws, 
         derive(draw_of(draws, fr, tri));
 }
 
+// Frames of even width: grid (z slots and tail cells of the largest frame / 256,
+// frame - f_lo).  What bounds it is latency (key, then mesh, then a chain of
+// set-up and shading): a 1280x720 frame in 5.0 us, against 7.2 of
+// k_winner_global and 4.1 of k_resolve_global.
+__global__ void __launch_bounds__(256) k_finish_global(const Draw* __restrict__ draws, const Ramp* __restrict__ ramps,
+                                                       const Frame* __restrict__ frames, uint32_t f_lo,
+                                                       const uint64_t* __restrict__ keys, const int32_t* __restrict__ nl,
+                                                       uint32_t* __restrict__ cells, float* __restrict__ zbuf,
+                                                       int32_t* __restrict__ win, uint32_t win_raw)
+{
+    typedef unsigned int v2u __attribute__((ext_vector_type(2), aligned(4)));
+    const Frame& fr = frames[f_lo + blockIdx.y];
+    const uint32_t W = fr.W, H = fr.H;
+    if (W & 1u) return;
+    const uint32_t WH = W * H;   // W, H <= 65535: cell ids fit 32 bits
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t* fc = cells + fr.cell_off;
+    if (s >= WH / 2) {
+        // image mode: the H cells after the grid are never written (context.rs:38-40)
+        const uint32_t i = s - WH / 2;
+        if (fr.image && i < H) __builtin_nontemporal_store(CELL_BLANK, fc + WH + i);
+        return;
+    }
+    const uint32_t c = 2 * s;
+    const uint64_t k = keys[fr.z_off + s];
+    float z = F32_MAX;
+    uint32_t c0 = CELL_BLANK, wt = 0xFFFFFFFFu, tri = 0;
+    if (k != KEY_EMPTY) {
+        uint32_t px, py;
+        winner_fragment(draws, ramps, fr, c, k, c0, z, tri, px, py);
+        wt = win_raw ? (uint32_t)k : tri;   // raw: triangle << 1 | sub
+    }
+    uint32_t c1 = c0;
+    if (fr.image) {
+        // the newline of row r is cell r*W + 1; it comes after every pixel of
+        // its triangle's row r and before the next row's
+        const uint32_t row = c / W;
+        if (c == row * W) {
+            const int32_t n = nl[fr.nl_off + row];
+            if (n >= 0 && (k == KEY_EMPTY || (uint32_t)n >= tri)) c1 = CELL_NEWLINE;
+        }
+    }
+    // streaming stores: outputs are written once
+    const v2u vc = {c0, c1}, vz = {__float_as_uint(z), __float_as_uint(F32_MAX)}, vw = {wt, 0xFFFFFFFFu};
+    __builtin_nontemporal_store(vc, (v2u*)(fc + c));
+    __builtin_nontemporal_store(vz, (v2u*)(zbuf + fr.z_off + c));
+    if (win) __builtin_nontemporal_store(vw, (v2u*)(win + fr.z_off + c));
+}
+
 // Keys of slots that k_winner_global has resolved: the winning cell in the
 // high word, the key's (triangle << 1 | sub) in the low word.  Frames hold
 // fewer than 2^31 - 1 triangles, so the low word is never all ones and a
 // resolved slot never reads as KEY_EMPTY.
 //
-// Both kernels: grid (cells of the largest frame / 256, frame - f_lo).
+// Both kernels: odd widths, grid (cells of the largest frame / 256, frame - f_lo).
 __global__ void __launch_bounds__(256) k_winner_global(const Draw* __restrict__ draws, const Ramp* __restrict__ ramps,
                                                        const Frame* __restrict__ frames, uint32_t f_lo,
                                                        uint64_t* __restrict__ keys, float* __restrict__ zbuf,
@@ -167,7 +236,7 @@ __global__ void __launch_bounds__(256) k_winner_global(const Draw* __restrict__ 
 {
     const Frame& fr = frames[f_lo + blockIdx.y];
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;   // W, H <= 65535: cell ids fit 32 bits
-    if (c >= fr.W * fr.H) return;   // the frame's z slots are its first W*H cell ids
+    if (!(fr.W & 1u) || c >= fr.W * fr.H) return;   // the frame's z slots are its first W*H cell ids
     uint64_t* fk = keys + fr.z_off;
     const uint64_t k = fk[c];
     float z = F32_MAX;
@@ -202,7 +271,7 @@ __global__ void __launch_bounds__(256) k_resolve_global(const Frame* __restrict_
     const uint32_t W = fr.W, H = fr.H;
     const uint32_t WH = W * H;   // W, H <= 65535: cell ids fit 32 bits
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= frame_cells(fr)) return;
+    if (!(W & 1u) || c >= frame_cells(fr)) return;
     const uint64_t* fk = keys + fr.z_off;
     // cell c = (row, col); its left neighbour is (row, col - 1), or the last
     // cell of the row above when col = 0 (cells past W*H are the newline rows'
