@@ -1338,8 +1338,15 @@ int sloth_batch_profile(sloth_batch* b, float* out_ms, const char** names, uint3
     *n_stages = (uint32_t)nm.size();
     if (!rc && se == hipSuccess) {
         for (uint32_t i = 0; i < nm.size() && i < cap; ++i) {
+            // the general path: one event between two stages; the tiled one:
+            // each part's stages
             float ms = 0.0f;
-            (void)hipEventElapsedTime(&ms, ev[i], ev[i + 1]);
+            const size_t parts = b->job.path == PATH_TILED ? b->job.tiled.parts.size() : 2;
+            for (size_t p = 0; p + 1 < parts; ++p) {
+                float one = 0.0f;
+                (void)hipEventElapsedTime(&one, ev[5 * p + i], ev[5 * p + i + 1]);
+                ms += one;
+            }
             if (out_ms) out_ms[i] = ms;
             if (names) names[i] = nm[i];
         }

@@ -33,13 +33,15 @@
 //                  many boxes are big, a variant has each wavefront walk its
 //                  lanes' big boxes with all 64 lanes.
 //
-// Tile lists live in one pool at fixed per-tile offsets, sized from an exact
+// Tile lists live in one pool at fixed per-tile offsets (large jobs: per part
+// of their frames, see PART_BYTES), sized from an exact
 // counting run of k_bin plus headroom.  If a later run would exceed a tile's
 // capacity (the transforms changed), k_bin raises the overflow flag and the
 // host re-plans and renders again.
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "sloth_device.h"
@@ -53,6 +55,18 @@ constexpr uint32_t MAX_GROUPS = 8;        // frame groups of a pipelined launch
 // flag and the entry's 8-bit cache row in their low 32 bits.
 constexpr uint32_t TILED_MAX_TRIS = (1u << 22) - 1;
 constexpr uint32_t PIPE_MIN_FRAMES = 16;  // frames per group at least
+// A job whose tile lists take more is rendered in parts of whole frames that
+// share one pool.  k_bin writes a list and the raster reads it a launch later:
+// from the 256 MB last-level cache when the pool's lines are still there,
+// else from HBM between the frames' stores, which costs more than the bytes
+// do (the list's lines read ahead by other blocks cost the same).  A part
+// costs a launch's tail, about 15 us.  256 frames of 1920x1080 with 0.2 GB
+// of lists, three such batches in turn / one after another, each waited for:
+// one part 1.80 / 1.65 ms, two 1.79 / 1.57, three 1.60 / 1.52, four 1.49 /
+// 1.48, five 1.48 / 1.51, six 1.49 / 1.57.  A batch rendered over and over
+// with nothing in between, which finds its lists cached either way: 1.42 in
+// one part, 1.46 in four.
+constexpr uint64_t PART_BYTES = 64ull << 20;
 
 struct TiledPlan {
     uint32_t TW = 64, TH = 32;       // tile size in cells (TW even)
@@ -75,6 +89,15 @@ struct TiledPlan {
     uint64_t n_rows = 0;
     bool sized = false;              // pool offsets match the current layout
     std::vector<uint64_t> off;       // host copy of the per-tile pool offsets (n_tiles + 1)
+    // set by size(): the first frame of each part and, last, the number of
+    // frames.  The parts are binned and rendered one after another and share
+    // the pool.
+    std::vector<uint32_t> parts;
+    bool is_part(uint32_t f_lo, uint32_t f_hi) const
+    {
+        const auto it = std::lower_bound(parts.begin(), parts.end(), f_lo);
+        return it != parts.end() && *it == f_lo && it + 1 != parts.end() && it[1] == f_hi;
+    }
     DevBuf d_cursor, d_off, d_pool, d_nl;
     uint32_t* overflow = nullptr;    // per frame, the job's pinned memory: kernels write it (rarely), the host reads it after a wait
     // triangles whose candidate box k_careful computes: (frame, triangle,
@@ -146,8 +169,9 @@ struct TiledPlan {
     int size(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
              const Draw* d_draws, hipStream_t s);
 
-    // clear + bin + careful + raster over frames [f_lo, f_hi).  ev (optional)
-    // gets 5 events recorded around the 4 stages.  With a second stream s2
+    // clear + bin + careful + raster over frames [f_lo, f_hi), part by part.
+    // ev (optional) gets 5 events recorded around the 4 stages of each part,
+    // more of them made when it holds too few.  With a second stream s2
     // and join events (and no ev), ranges of at least 2 * PIPE_MIN_FRAMES
     // frames run as a pipeline of frame groups: the bins of one group overlap
     // the raster of the previous one (join needs groups + 1 events).
@@ -164,11 +188,12 @@ struct TiledPlan {
   private:
     int launch_clear(const std::vector<Frame>& frames, uint32_t f_lo, uint32_t f_hi, hipStream_t s);
     int launch_bin(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
-                   const Draw* d_draws, uint32_t f_lo, uint32_t f_hi, bool count_only, hipStream_t s);
+                   const Draw* d_draws, uint32_t f_lo, uint32_t f_hi, uint32_t* pool, bool count_only, hipStream_t s);
     int reserve_edges();
-    int launch_careful(const Frame* d_frames, const Draw* d_draws, bool count_only, uint32_t group, hipStream_t s);
+    uint32_t* pool_of(const std::vector<Frame>& frames, uint32_t part_begin) const;
+    int launch_careful(const Frame* d_frames, const Draw* d_draws, uint32_t* pool, bool count_only, uint32_t group, hipStream_t s);
     int launch_raster(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames, const Draw* d_draws,
-                      const Ramp* d_ramps, uint32_t f_lo, uint32_t f_hi, uint32_t* cells, float* z, int32_t* win,
+                      const Ramp* d_ramps, uint32_t f_lo, uint32_t f_hi, uint32_t* pool, uint32_t* cells, float* z, int32_t* win,
                       bool win_raw, uint32_t n_ramps, bool reset_careful, hipStream_t s);
 };
 

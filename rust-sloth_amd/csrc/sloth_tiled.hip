@@ -1597,6 +1597,12 @@ int TiledPlan::reserve_edges()
     return odd_cols() ? d_edges.reserve(sizeof(uint4) * 2 * std::max<uint64_t>(1, n_tiles) * TH) : SLOTH_OK;
 }
 
+uint32_t* TiledPlan::pool_of(const std::vector<Frame>& frames, uint32_t part_begin) const
+{
+    // off counts through all parts; each part's lists start at the pool's start
+    return (uint32_t*)((uintptr_t)d_pool.p - sizeof(uint32_t) * off[frames[part_begin].tile_begin]);
+}
+
 int TiledPlan::launch_clear(const std::vector<Frame>& frames, uint32_t f_lo, uint32_t f_hi, hipStream_t s)
 {
     const Frame& a = frames[f_lo];
@@ -1613,14 +1619,14 @@ int TiledPlan::launch_clear(const std::vector<Frame>& frames, uint32_t f_lo, uin
 }
 
 int TiledPlan::launch_bin(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
-                          const Draw* d_draws, uint32_t f_lo, uint32_t f_hi, bool count_only, hipStream_t s)
+                          const Draw* d_draws, uint32_t f_lo, uint32_t f_hi, uint32_t* pool, bool count_only, hipStream_t s)
 {
     const uint32_t d_lo = frames[f_lo].draw_begin, d_hi = frames[f_hi - 1].draw_end;
     const int tws = log2u(TW), ths = log2u(TH);
     auto go = [&](dim3 grid, uint32_t d0, const uint2* flat) {
         auto run = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, dim3(BIN_BLOCK), 0, s, d_draws, d0, d_frames, tws, ths,
-                               d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
+                               d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), pool,
                                d_nl.as<int32_t>(), overflow, d_careful_cnt.as<uint32_t>(),
                                d_careful_in.as<uint4>(), careful_cap, flat, odd_cols());
         };
@@ -1652,8 +1658,8 @@ int TiledPlan::launch_bin(const std::vector<Frame>& frames, const std::vector<Dr
     return SLOTH_OK;
 }
 
-int TiledPlan::launch_careful(const Frame* d_frames, const Draw* d_draws, bool count_only, uint32_t group,
-                              hipStream_t s)
+int TiledPlan::launch_careful(const Frame* d_frames, const Draw* d_draws, uint32_t* pool, bool count_only,
+                              uint32_t group, hipStream_t s)
 {
     if (careful_cap == 0) return SLOTH_OK;
     const int tws = log2u(TW), ths = log2u(TH);
@@ -1663,12 +1669,12 @@ int TiledPlan::launch_careful(const Frame* d_frames, const Draw* d_draws, bool c
     dim3 grid(std::min(blocks(careful_cap, 4), 4096u));
     if (count_only)
         hipLaunchKernelGGL(k_careful<true>, grid, dim3(256), 0, s, d_frames, tws, ths,
-                           d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
+                           d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), pool,
                            overflow, d_careful_cnt.as<uint32_t>(), group, d_careful_in.as<uint4>(),
                            d_careful_box.as<uint4>(), careful_cap, odd_cols());
     else
         hipLaunchKernelGGL(k_careful<false>, grid, dim3(256), 0, s, d_frames, tws, ths,
-                           d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
+                           d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), pool,
                            overflow, d_careful_cnt.as<uint32_t>(), group, d_careful_in.as<uint4>(),
                            d_careful_box.as<uint4>(), careful_cap, odd_cols());
     HIP_TRY(hipGetLastError());
@@ -1707,7 +1713,7 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     }
     // 1. count tile entries of CLS_BOX triangles and the careful triangles
     if ((rc = launch_clear(frames, 0, F, s))) return rc;
-    if ((rc = launch_bin(frames, draws, d_frames, d_draws, 0, F, true, s))) return rc;
+    if ((rc = launch_bin(frames, draws, d_frames, d_draws, 0, F, nullptr, true, s))) return rc;
     uint32_t cnt[WRAP_CNT + 1];
     HIP_TRY(hipMemcpyAsync(cnt, d_careful_cnt.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
@@ -1730,10 +1736,10 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
         if ((rc = d_careful_in.reserve(2 * sizeof(uint4) * careful_cap))) return rc;
         if ((rc = d_careful_box.reserve(sizeof(uint4) * careful_cap))) return rc;
         if ((rc = launch_clear(frames, 0, F, s))) return rc;
-        if ((rc = launch_bin(frames, draws, d_frames, d_draws, 0, F, true, s))) return rc;
+        if ((rc = launch_bin(frames, draws, d_frames, d_draws, 0, F, nullptr, true, s))) return rc;
     }
     // 3. the careful triangles' tile entries
-    if ((rc = launch_careful(d_frames, d_draws, true, 0, s))) return rc;
+    if ((rc = launch_careful(d_frames, d_draws, nullptr, true, 0, s))) return rc;
     std::vector<uint32_t> counts(n_tiles);
     if (n_tiles)
         HIP_TRY(hipMemcpyAsync(counts.data(), d_cursor.p, sizeof(uint32_t) * n_tiles, hipMemcpyDeviceToHost, s));
@@ -1749,7 +1755,17 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
         multi = multi || cap > CHUNK;
         off[t + 1] = off[t] + cap;
     }
-    if ((rc = d_pool.reserve(sizeof(uint32_t) * std::max<uint64_t>(1, off[n_tiles])))) return rc;
+    // the parts: frames in order, of near equal lists
+    const uint64_t n_parts = off[n_tiles] * sizeof(uint32_t) / PART_BYTES + 1;
+    parts.assign(1, 0);
+    uint64_t most = 0;
+    auto lists_from = [&](uint32_t f) { return f < F ? off[frames[f].tile_begin] : off[n_tiles]; };
+    for (uint32_t f = 1; f <= F; ++f)
+        if (f == F || (parts.size() < n_parts && lists_from(f) * n_parts >= off[n_tiles] * parts.size())) {
+            most = std::max(most, lists_from(f) - lists_from(parts.back()));
+            parts.push_back(f);
+        }
+    if ((rc = d_pool.reserve(sizeof(uint32_t) * std::max<uint64_t>(1, most)))) return rc;
     HIP_TRY(hipMemcpyAsync(d_off.p, off.data(), sizeof(uint64_t) * (n_tiles + 1), hipMemcpyHostToDevice, s));
     // 4. flat raster grids (frames of different tile grids): each tile's
     // (tile, frame) in tile order, and the same with the tiles of more than
@@ -1766,10 +1782,12 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
             for (uint64_t t = 0; t < (uint64_t)frames[f].tiles_x * frames[f].tiles_y; ++t)
                 tf[frames[f].tile_begin + t] = make_uint2((uint32_t)(frames[f].tile_begin + t), f);
         heavy = tf;
-        const auto split = std::stable_partition(heavy.begin(), heavy.end(),
-                                                 [&](const uint2& a) { return counts[a.x] > 4 * CHUNK; });
-        std::stable_sort(heavy.begin(), split,
-                         [&](const uint2& a, const uint2& b) { return counts[a.x] > counts[b.x]; });
+        for (size_t p = 0; p + 1 < parts.size(); ++p) {
+            const auto end = heavy.begin() + (parts[p + 1] < F ? frames[parts[p + 1]].tile_begin : n_tiles);
+            const auto begin = heavy.begin() + frames[parts[p]].tile_begin;
+            const auto split = std::stable_partition(begin, end, [&](const uint2& a) { return counts[a.x] > 4 * CHUNK; });
+            std::stable_sort(begin, split, [&](const uint2& a, const uint2& b) { return counts[a.x] > counts[b.x]; });
+        }
         if ((rc = d_tile_frame.reserve(sizeof(uint2) * std::max<uint64_t>(1, n_tiles))) ||
             (rc = d_tile_heavy.reserve(sizeof(uint2) * std::max<uint64_t>(1, n_tiles))))
             return rc;
@@ -1803,8 +1821,8 @@ static auto raster_kernel(bool walk, bool one, bool odd)
 }
 
 int TiledPlan::launch_raster(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
-                             const Draw* d_draws, const Ramp* d_ramps, uint32_t f_lo, uint32_t f_hi, uint32_t* cells, float* z, int32_t* win,
-                             bool win_raw, uint32_t n_ramps, bool reset_careful, hipStream_t s)
+                             const Draw* d_draws, const Ramp* d_ramps, uint32_t f_lo, uint32_t f_hi, uint32_t* pool, uint32_t* cells, float* z,
+                             int32_t* win, bool win_raw, uint32_t n_ramps, bool reset_careful, hipStream_t s)
 {
     // the first raster launch resets the careful list's length (k_careful
     // has read it) when asked
@@ -1826,12 +1844,12 @@ int TiledPlan::launch_raster(const std::vector<Frame>& frames, const std::vector
         if (flat_raster && t_hi > 0x7FFFFFFFull) return fail(SLOTH_EINVAL, "too many tiles for a flat raster grid");
         const dim3 grid = flat_raster ? dim3((unsigned)(t_hi - t_lo)) : dim3(mx, my, f1 - f0);
         const uint2* tf = !flat_raster ? nullptr
-                          : f0 == 0 && f1 == (uint32_t)frames.size() ? d_tile_heavy.as<uint2>()
-                                                                      : d_tile_frame.as<uint2>();
+                          : is_part(f0, f1) ? d_tile_heavy.as<uint2>()
+                                            : d_tile_frame.as<uint2>();
         uint4* edges = od ? d_edges.as<uint4>() : nullptr;
         auto go = [&](auto kern, dim3 grid, size_t lds) {
             hipLaunchKernelGGL(kern, grid, dim3(RASTER_BLOCK), lds, s, d_draws, d_ramps, d_frames, f0, log2u(TW),
-                               log2u(TH), d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), d_pool.as<uint32_t>(),
+                               log2u(TH), d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), pool,
                                d_nl.as<int32_t>(), d_careful_box.as<uint4>(), cells, z, win, win_raw ? 1u : 0u,
                                n_ramps, edges, careful_reset, tf, (uint32_t)t_lo, odd_cols());
             careful_reset = nullptr;
@@ -1870,39 +1888,56 @@ int TiledPlan::launch(const std::vector<Frame>& frames, const std::vector<Draw>&
     int rc;
     const uint32_t nf = f_hi - f_lo;
     uint32_t groups = 1;
-    if (s2 && join && !ev) groups = std::min<uint32_t>({MAX_GROUPS, nf / PIPE_MIN_FRAMES, (uint32_t)join->size() - 1});
+    if (s2 && join && !ev && parts.size() == 2)
+        groups = std::min<uint32_t>({MAX_GROUPS, nf / PIPE_MIN_FRAMES, (uint32_t)join->size() - 1});
     if (groups < 2) {
         // Every render leaves the tile cursors, the even frames' newline
         // rows and the careful list's length as k_tile_clear sets them
         // (k_tile_raster resets what it has read; size() ends with a
         // clear), but for frames one column wide, whose newline rows
         // k_tile_edges reads after the raster.
-        if (ev) HIP_TRY(hipEventRecord((*ev)[0], s));
-        if (odd_narrow && (rc = launch_clear(frames, f_lo, f_hi, s))) return rc;
-        if (ev) HIP_TRY(hipEventRecord((*ev)[1], s));
-        if ((rc = launch_bin(frames, draws, d_frames, d_draws, f_lo, f_hi, false, s))) return rc;
-        if (ev) HIP_TRY(hipEventRecord((*ev)[2], s));
-        if ((rc = launch_careful(d_frames, d_draws, false, 0, s))) return rc;
-        if (ev) HIP_TRY(hipEventRecord((*ev)[3], s));
-        if ((rc = launch_raster(frames, draws, d_frames, d_draws, d_ramps, f_lo, f_hi, cells, z, win, win_raw, n_ramps, true,
-                                s)))
-            return rc;
-        if (ev) HIP_TRY(hipEventRecord((*ev)[4], s));
+        size_t n_ev = 0;
+        auto mark = [&]() -> int {
+            if (!ev) return SLOTH_OK;
+            if (n_ev == ev->size()) {
+                ev->push_back(nullptr);
+                HIP_TRY(hipEventCreate(&ev->back()));
+            }
+            HIP_TRY(hipEventRecord((*ev)[n_ev++], s));
+            return SLOTH_OK;
+        };
+        for (size_t p = 0; p + 1 < parts.size(); ++p) {
+            const uint32_t a = std::max(f_lo, parts[p]), b = std::min(f_hi, parts[p + 1]);
+            if (a >= b) continue;
+            uint32_t* pool = pool_of(frames, parts[p]);
+            if ((rc = mark())) return rc;
+            if (odd_narrow && (rc = launch_clear(frames, a, b, s))) return rc;
+            if ((rc = mark())) return rc;
+            if ((rc = launch_bin(frames, draws, d_frames, d_draws, a, b, pool, false, s))) return rc;
+            if ((rc = mark())) return rc;
+            if ((rc = launch_careful(d_frames, d_draws, pool, false, 0, s))) return rc;
+            if ((rc = mark())) return rc;
+            if ((rc = launch_raster(frames, draws, d_frames, d_draws, d_ramps, a, b, pool, cells, z, win, win_raw,
+                                    n_ramps, true, s)))
+                return rc;
+            if ((rc = mark())) return rc;
+        }
         return SLOTH_OK;
     }
     // Pipeline over frame groups: s bins group g + 1 while s2 rasters group
     // g.  Group g's raster waits for its bins and careful boxes (event g); s
     // joins s2 at the end.
+    uint32_t* pool = d_pool.as<uint32_t>();
     if ((rc = launch_clear(frames, f_lo, f_hi, s))) return rc;
     for (uint32_t g = 0; g < groups; ++g) {
         const uint32_t a = f_lo + (uint32_t)((uint64_t)nf * g / groups);
         const uint32_t b = f_lo + (uint32_t)((uint64_t)nf * (g + 1) / groups);
-        if ((rc = launch_bin(frames, draws, d_frames, d_draws, a, b, false, s))) return rc;
-        if ((rc = launch_careful(d_frames, d_draws, false, g, s))) return rc;
+        if ((rc = launch_bin(frames, draws, d_frames, d_draws, a, b, pool, false, s))) return rc;
+        if ((rc = launch_careful(d_frames, d_draws, pool, false, g, s))) return rc;
         HIP_TRY(hipEventRecord((*join)[g], s));
         HIP_TRY(hipStreamWaitEvent(s2, (*join)[g], 0));
         // the last group's raster runs after every group's careful pass
-        if ((rc = launch_raster(frames, draws, d_frames, d_draws, d_ramps, a, b, cells, z, win, win_raw, n_ramps,
+        if ((rc = launch_raster(frames, draws, d_frames, d_draws, d_ramps, a, b, pool, cells, z, win, win_raw, n_ramps,
                                 g + 1 == groups, s2)))
             return rc;
     }
