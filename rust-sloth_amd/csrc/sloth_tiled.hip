@@ -778,6 +778,17 @@ __device__ __forceinline__ void direct_rect(const TileGeom& g, int bx0, int bx1,
     yb = min(by1, g.tr1 - 1) - g.tr0;
 }
 
+// The wrapped part, as the slots' columns and rows in the tile.
+__device__ __forceinline__ void wrapped_rect(const TileGeom& g, int bx0, int bx1, int by0, int by1, int& xa, int& xb,
+                                             int& ya, int& yb)
+{
+    const int ox = (g.tc0 + g.W + 1) >> 1;
+    xa = max(bx0, ox) - ox;
+    xb = min(bx1, (g.tc1 - 1 + g.W) >> 1) - ox;
+    ya = max(by0, g.tr0 - 1) - (g.tr0 - 1);
+    yb = min(by1, g.tr1 - 2) - (g.tr0 - 1);
+}
+
 // Order in which the pixels of a frame are written: by triangle, row, column
 // (0: never).
 __device__ __forceinline__ uint64_t pixel_time(uint32_t T, uint32_t py, uint32_t px)
@@ -1101,12 +1112,21 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
         for (uint32_t base = 0; base < n; base += CHUNK) {
             __syncthreads();   // keys cleared / the previous chunk's cells no longer read its rows
             const uint32_t p = threadIdx.x;
-            bool big = false;              // BIG: this lane's box is walked by its wavefront
-            uint32_t big_T = 0, big_rect = 0;
-            if (base + p < n) {
+            // BIG: the direct / wrapped part of this lane's box is walked by its
+            // wavefront (the wrapped part by its lane alone: a few triangles of
+            // 200 pixels a side on a 2560x1440 frame took 97 us, now 27)
+            bool big = false, big_w = false;
+            uint32_t big_T = 0, big_rect = 0, big_rect_w = 0;
+            // the entry of this thread.  BIG: a list of a few entries is dealt
+            // out over the wavefronts, which walk their big boxes one by one
+            // (30 unlike jobs in turn: 171 -> 158 us; dealing out up to 40
+            // entries costs batches of small triangles their set-up in four
+            // wavefronts: 523 -> 590 us for 64 frames of 1919x1079 at 64 x 16)
+            const uint32_t at = BIG && n <= 16 ? ((p & 63u) << 2) | (p >> 6) : base + p;
+            if (at < n) {
                 int bx0, bx1, by0, by1;
                 bool given, tight;
-                const uint32_t T = entry_tri(list[base + p], careful_box, bx0, bx1, by0, by1, given, tight);
+                const uint32_t T = entry_tri(list[at], careful_box, bx0, bx1, by0, by1, given, tight);
                 const Draw& dr = draw_of_tri(T);
                 const uint32_t li = T - dr.tri_begin;
                 Tri t;
@@ -1166,7 +1186,6 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                         direct_rect(g, bx0, bx1, by0, by1, xa, xb, ya, yb);
                         if (xa <= xb && ya <= yb && (xb - xa + 1) * (yb - ya + 1) > (int)BIG_BOX) {
                             big = true;
-                            big_T = T;
                             big_rect =
                                 (uint32_t)xa | ((uint32_t)xb << 8) | ((uint32_t)ya << 16) | ((uint32_t)yb << 24);
                         } else {
@@ -1177,7 +1196,14 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                                 walk_rect<XS, true>(t, xa + (g.tc0 >> 1), xb + (g.tc0 >> 1), ya + g.tr0, yb + g.tr0,
                                                     (ya << sws) + xa, sws, 1u, hit);
                         }
-                        walk_wrapped<XS>(g, t, bx0, bx1, by0, by1, hit);
+                        wrapped_rect(g, bx0, bx1, by0, by1, xa, xb, ya, yb);
+                        if (xa <= xb && ya <= yb) {
+                            big_w = (xb - xa + 1) * (yb - ya + 1) > (int)BIG_BOX;
+                            big_rect_w =
+                                (uint32_t)xa | ((uint32_t)xb << 8) | ((uint32_t)ya << 16) | ((uint32_t)yb << 24);
+                            if (!big_w) walk_wrapped<XS>(g, t, bx0, bx1, by0, by1, hit);
+                        }
+                        big_T = T;
                     } else {
                         walk_tile<XS>(g, t, bx0, bx1, by0, by1, safe, hit);
                     }
@@ -1189,11 +1215,16 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                 // with the expressions of edges() and depth() on the box's
                 // row (row p of the lane that holds it, written by this
                 // wavefront above).
-                uint64_t m = __ballot(big);
-                while (m) {
-                    const int l = __builtin_ctzll(m);
-                    m &= m - 1;
-                    const uint32_t T = __builtin_amdgcn_readlane(big_T, l), rc = __builtin_amdgcn_readlane(big_rect, l);
+                uint64_t m = __ballot(big), m_w = __ballot(big_w);
+                while (m | m_w) {
+                    const bool direct = m != 0;
+                    const int l = __builtin_ctzll(direct ? m : m_w);
+                    if (direct) m &= m - 1;
+                    else m_w &= m_w - 1;
+                    const uint32_t T = __builtin_amdgcn_readlane(big_T, l);
+                    const uint32_t rc = direct ? __builtin_amdgcn_readlane(big_rect, l) : __builtin_amdgcn_readlane(big_rect_w, l);
+                    // the pixel of the tile's first slot
+                    const int ox = direct ? g.tc0 >> 1 : (g.tc0 + g.W + 1) >> 1, oy = direct ? g.tr0 : g.tr0 - 1;
                     const uint32_t prow = (threadIdx.x & ~63u) + (uint32_t)l;   // the owner lane's row
                     const float4 v12 = rows.v12[prow], q2 = rows.depth[prow];
                     const float2 v3 = rows.v3[prow];
@@ -1206,14 +1237,14 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                     int i = (int)__lane_id(), yy = i / nx, xx = i - yy * nx;
                     for (; i < nx * ny; i += 64) {
                         const int x = xa + xx, y = ya + yy;
-                        const float px = (float)(x + (g.tc0 >> 1)), py = (float)(y + g.tr0);
+                        const float px = (float)(x + ox), py = (float)(y + oy);
                         const float w0 = A0 * (py - y2) - B0 * (px - x2);
                         const float w1 = A1 * (py - y3) - B1 * (px - x3);
                         const float w2 = A2 * (py - y1) - B2 * (px - x1);
                         const float z = z1 + a * (w1 * dz2 + w2 * dz3);
                         if (inside(w0, w1, w2) && z < F32_MAX)
                             atomicMin((unsigned long long*)&keys[(y << sws) + x],
-                                      (unsigned long long)make_tile_key(z, T, 1u, prow));
+                                      (unsigned long long)make_tile_key(z, T, direct ? 1u : 0u, prow));
                         xx += dx;
                         yy += dy;
                         if (xx >= nx) {
