@@ -15,11 +15,11 @@
 //                  candidate box, newline rows (LDS max per block, one
 //                  atomicMax per row), and the triangle index appended to
 //                  every tile its box reaches: boxes within 2 x 2 tiles of one
-//                  region count into a 16 x 16 LDS window of tiles, with one
-//                  global atomicAdd per window tile per block; others (and the
-//                  careful list) append directly
-//   k_careful      one wavefront per careful triangle: exact box from row
-//                  spans, then its tile entries
+//                  region count into an LDS window of tiles, with one global
+//                  atomicAdd per window tile per block; others go to the
+//                  careful list
+//   k_careful      one wavefront per careful triangle (many tiles, or an
+//                  exact box from row spans): its tile entries
 //   k_tile_raster  one 256-thread workgroup per tile, grid (tile x, tile y,
 //                  frame): each list entry is set up by a lane and its row
 //                  kept in LDS, its fragments do a 64-bit LDS atomicMin of
@@ -125,7 +125,8 @@ struct TiledPlan {
     // walk those boxes together; SLOTH_BIG_WALK=0/1 overrides
     bool big_walk = false;
     // set by size(): k_bin reduces newline rows through a segment tree
-    // (one triangle in 256 or more spans more than 16 rows); SLOTH_BIN_TREE
+    // (one triangle in 256 or more spans more than 16 rows, or a block's worth
+    // among draws of different sizes); SLOTH_BIN_TREE
     // =0/1 overrides
     bool bin_tree = false;
     // -1: the raster variant big_walk picks; 0 / 1: without / with the

@@ -99,64 +99,9 @@ __device__ __forceinline__ int odd_cols_of(int bx1, uint32_t W, int tws)
     return bx1 < last ? 0 : bx1 == last ? 1 : ((2 * bx1 - (int)W) >> tws) + 2;
 }
 
-// Walks a lane's tiles: the direct rectangle, then the wrapped one minus the
-// tiles the direct rectangle already holds.  phase 2 = done.
-struct TileIter {
-    int tx, ty, phase;
-};
-
 __device__ __forceinline__ bool in_direct(const TileRects& r, int tx, int ty)
 {
     return tx >= r.dx0 && tx <= r.dx1 && ty >= r.dy0 && ty <= r.dy1;
-}
-
-__device__ __forceinline__ void iter_settle(const TileRects& r, TileIter& it)
-{
-    for (;;) {
-        if (it.phase == 0) {
-            if (r.dx0 <= r.dx1 && it.ty <= r.dy1) return;
-            it.phase = 1;
-            it.tx = r.wx0;
-            it.ty = r.wy0;
-        }
-        if (it.phase == 1) {
-            if (!(r.wx0 <= r.wx1) || it.ty > r.wy1) {
-                it.phase = 2;
-                return;
-            }
-            if (!in_direct(r, it.tx, it.ty)) return;
-            if (++it.tx > r.wx1) {
-                it.tx = r.wx0;
-                ++it.ty;
-            }
-            continue;
-        }
-        return;
-    }
-}
-
-__device__ __forceinline__ void iter_begin(const TileRects& r, TileIter& it)
-{
-    it.phase = 0;
-    it.tx = r.dx0;
-    it.ty = r.dy0;
-    iter_settle(r, it);
-}
-
-__device__ __forceinline__ void iter_next(const TileRects& r, TileIter& it)
-{
-    if (it.phase == 0) {
-        if (++it.tx > r.dx1) {
-            it.tx = r.dx0;
-            ++it.ty;
-        }
-    } else if (it.phase == 1) {
-        if (++it.tx > r.wx1) {
-            it.tx = r.wx0;
-            ++it.ty;
-        }
-    }
-    iter_settle(r, it);
 }
 
 // One entry appended to tile `gt` at `pos` (when the pool has room).
@@ -173,13 +118,13 @@ __device__ __forceinline__ void put_entry(uint64_t gt, uint32_t pos, uint32_t en
 // ---------------------------------------------------------------------------
 // k_bin
 // ---------------------------------------------------------------------------
-constexpr int BIN_WIN = 16;   // the block aggregates appends in a 16 x 16 window of tiles
+constexpr int BIN_CELLS = 512;   // the block aggregates appends in a window of up to so many tiles
 
 // Grid: x = blocks of TPT * BIN_BLOCK consecutive triangles of one draw,
 // y = draw index - d_lo, so the draw, its frame and its matrix are uniform
-// per block (scalar loads).  CLS_BOX / CLS_TIGHT triangles are appended to
-// their tiles here; CLS_SPANS / CLS_FULL ones go to the careful list for
-// k_careful.
+// per block (scalar loads).  CLS_BOX / CLS_TIGHT triangles of few tiles are
+// appended to them here; others and CLS_SPANS / CLS_FULL ones go to the
+// careful list for k_careful.
 //
 // Each thread takes TPT triangles (k * BIN_BLOCK + thread), set up one after
 // another with their loads in flight together, so that the block's barriers
@@ -192,11 +137,17 @@ constexpr int BIN_WIN = 16;   // the block aggregates appends in a 16 x 16 windo
 // Appends: a block's consecutive triangles lie close together on screen.
 // Triangles whose box touches at most 2 x 2 tiles, all in the direct region
 // or all in the wrapped one (nearly all), count themselves into LDS counters
-// of a 16 x 16 tile window anchored at the block's smallest tile coordinates;
-// one global atomicAdd per window tile then reserves that tile's run (the
-// thread that reserves it also reads the tile's pool range), and each
-// triangle writes its entry at run + its LDS count.  Others append with one
-// global atomicAdd per tile.
+// of a window of tiles anchored at the block's smallest tile coordinates; one
+// global atomicAdd per window tile then reserves that tile's run (the thread
+// that reserves it also reads the tile's pool range), and each triangle
+// writes its entry at run + its LDS count.  The window has 512 tiles in rows
+// as long as the block's tiles need (a strip of a large mesh's face is wide
+// and low, or slanted); those outside append with one global atomicAdd per
+// tile, up to four in flight together.  Larger boxes and part-wrapping ones
+// go to k_careful: appended here, one tile after another, they held up their
+// block (972 triangles of about 20 tiles each on 2560x1440: 70 us, now 29 for
+// the launch; 519,168 small ones, some across the wrap: 106 us, now 21).
+// 30 unlike jobs: k_bin 110-255 us, now 53-59 (with bin_tree's rule).
 //
 // geo word: qx0 (bits 0-13), qy0 (14-27) of the tile rectangle, wide (28),
 // tall (29), CLS_BOX (30); tile coordinates stay below 2^14 (frames of at
@@ -236,13 +187,13 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
                                                    uint4* __restrict__ careful_in, uint32_t careful_cap,
                                                    const uint2* __restrict__ flat_blocks, uint32_t odd_cols)
 {
-    __shared__ uint32_t w_cnt[BIN_WIN * BIN_WIN];
-    __shared__ uint64_t w_base[BIN_WIN * BIN_WIN];   // pool index of the tile's reserved run
-    __shared__ uint64_t w_end[BIN_WIN * BIN_WIN];    // end of the tile's pool range
+    __shared__ uint32_t w_cnt[BIN_CELLS];
+    __shared__ uint64_t w_base[BIN_CELLS];   // pool index of the tile's reserved run
+    __shared__ uint32_t w_room[BIN_CELLS];   // entries of it that the tile's pool range holds
     // newline rows: a window of rows, or (TREE) its segment tree (nl_raise)
     __shared__ int32_t s_nl[TREE ? 2 * BIN_BLOCK : BIN_BLOCK];
     constexpr int LEAF = TREE ? BIN_BLOCK : 0;   // row r of the window at s_nl[LEAF + r]
-    __shared__ int s_tx0, s_ty0, s_lo, s_hi;
+    __shared__ int s_tx0, s_ty0, s_tx1, s_ty1, s_lo, s_hi;
 
     // the block's draw and first triangle: from the grid, or (flat grids of
     // draws of different sizes) from its table entry
@@ -263,12 +214,12 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
     const uint64_t tile_begin = fr.tile_begin;
     const uint32_t tiles_x = fr.tiles_x;
 
-    w_cnt[threadIdx.x] = 0;
+    for (int c = threadIdx.x; c < BIN_CELLS; c += BIN_BLOCK) w_cnt[c] = 0;
     s_nl[threadIdx.x] = -1;
     if (TREE) s_nl[LEAF + threadIdx.x] = -1;
     if (threadIdx.x == 0) {
         s_tx0 = s_ty0 = s_lo = 1 << 30;
-        s_hi = -1;
+        s_tx1 = s_ty1 = s_hi = -1;
     }
 
     // Phase 1: set-up and classes.  Lanes past the draw's end set up its
@@ -276,8 +227,9 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
     // it (the lanes of a wavefront take different classes; selects cost less
     // than divergent paths).
     uint32_t geo[TPT], rows[TPT];
-    uint32_t tiled = 0, small = 0;   // bit k: triangle k has tiles here / has a small rectangle
-    int acc_lo = 1 << 30, acc_hi = -1, acc_tx = 1 << 30, acc_ty = 1 << 30;
+    uint32_t small = 0;   // bit k: triangle k has a small rectangle, appended here
+    int acc_lo = 1 << 30, acc_hi = -1;
+    uint32_t acc_t0 = 0x7FFF7FFFu, acc_t1 = 0;   // least and largest tile: x, y << 16
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
         const uint32_t local = base + (uint32_t)k * BIN_BLOCK + threadIdx.x;
@@ -286,7 +238,7 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
         setup_draw_tri(dr, valid ? local : dr.n - 1, W, H, t);
         const uint32_t cls = valid ? setup_class(t) : CLS_EMPTY;
         const bool boxed = cls == CLS_BOX || cls == CLS_TIGHT;
-        const bool careful = cls == CLS_SPANS || cls == CLS_FULL;
+        bool careful = cls == CLS_SPANS || cls == CLS_FULL;
         uint32_t g = cls == CLS_BOX ? GEO_LOOSE : 0u;
         // A wavefront whose triangles are all back faces or empty (half of
         // a closed mesh's, in runs) has no tiles to find: a uniform branch.
@@ -299,11 +251,10 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
                 if (__lane_id() == 0 && m) atomicAdd(&careful_cnt[BIG_CNT], (uint32_t)__popcll(m));
             }
             // A box in one region appends through that region's tile
-            // rectangle [qx0, qx1] x [qy0, qy1]; a box that wraps in part
-            // (it spans 2x = W) takes the per-tile path.  (Meshes wider than
-            // the frame's logical width put whole patches of triangles in
-            // the wrapped region, whose per-tile atomics would meet on few
-            // addresses.)
+            // rectangle [qx0, qx1] x [qy0, qy1]; k_careful takes a box that
+            // wraps in part (it spans 2x = W).  (Meshes wider than the frame's
+            // logical width put whole patches of triangles in the wrapped
+            // region.)
             bool has_direct, has_wrap;
             int qx0, qx1, qy0, qy1;
             if (!__ballot(bx1 >= (int)(W >> 1))) {
@@ -335,12 +286,13 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
                 qy1 = wrap_only ? r.wy1 : r.dy1;
             }
             const bool sm = has_direct != has_wrap && qx1 - qx0 <= 1 && qy1 - qy0 <= 1;
-            if (has_direct || has_wrap) tiled |= 1u << k;
+            // larger and part-wrapping boxes: appended by k_careful
+            careful = careful || ((has_direct || has_wrap) && !sm);
             if (sm) {
                 small |= 1u << k;
                 g |= (uint32_t)qx0 | ((uint32_t)qy0 << 14) | (qx1 > qx0 ? GEO_WIDE : 0u) | (qy1 > qy0 ? GEO_TALL : 0u);
-                acc_tx = min(acc_tx, qx0);
-                acc_ty = min(acc_ty, qy0);
+                acc_t0 = min_u16x2(acc_t0, (uint32_t)qx0 | ((uint32_t)qy0 << 16));
+                acc_t1 = max_u16x2(acc_t1, (uint32_t)qx1 | ((uint32_t)qy1 << 16));
             }
         }
         geo[k] = g;
@@ -375,10 +327,13 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
             atomicMax(&s_hi, whi);
         }
         if (__ballot(small != 0)) {
-            const int wtx = wave_min(acc_tx), wty = wave_min(acc_ty);
+            const uint32_t t0 = wave_reduce((int)acc_t0, [](int a, int b) { return (int)min_u16x2((uint32_t)a, (uint32_t)b); });
+            const uint32_t t1 = wave_reduce((int)acc_t1, [](int a, int b) { return (int)max_u16x2((uint32_t)a, (uint32_t)b); });
             if (__lane_id() == 0) {
-                atomicMin(&s_tx0, wtx);
-                atomicMin(&s_ty0, wty);
+                atomicMin(&s_tx0, (int)(t0 & 0xFFFFu));
+                atomicMin(&s_ty0, (int)(t0 >> 16));
+                atomicMax(&s_tx1, (int)(t1 & 0xFFFFu));
+                atomicMax(&s_ty1, (int)(t1 >> 16));
             }
         }
     }
@@ -391,12 +346,19 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
     // when they span fewer than BIN_BLOCK rows, else in windows of BIN_BLOCK
     // rows at the end (tall triangles put every row of a tall frame under
     // the atomics of each triangle that covers it).
-    const int ox = s_tx0, oy = s_ty0, lo = s_lo, hi = s_hi;
+    const int ox = __builtin_amdgcn_readfirstlane(s_tx0), oy = __builtin_amdgcn_readfirstlane(s_ty0);
+    const int lo = s_lo, hi = s_hi;
+    // the window: the block's tiles, in rows of 2^ws, when there are that few
+    // (one tile where no rectangle is small)
+    const int tiles_w = max(__builtin_amdgcn_readfirstlane(s_tx1) - ox + 1, 1);
+    const int tiles_h = max(__builtin_amdgcn_readfirstlane(s_ty1) - oy + 1, 1);
+    const int ws_all = 31 - __builtin_clz(2 * tiles_w - 1);
+    const int ws = ((int64_t)tiles_h << ws_all) <= BIN_CELLS ? ws_all : min(ws_all, 5);
     const bool nl_lds = hi >= lo && hi - lo < BIN_BLOCK;
     auto in_window = [&](uint32_t g, int& c) {
         const int qx0 = (int)(g & 0x3FFFu), qy0 = (int)((g >> 14) & 0x3FFFu);
-        c = (qy0 - oy) * BIN_WIN + (qx0 - ox);
-        return qx0 + (int)((g >> 28) & 1u) - ox < BIN_WIN && qy0 + (int)((g >> 29) & 1u) - oy < BIN_WIN;
+        c = ((qy0 - oy) << ws) + (qx0 - ox);
+        return qx0 + (int)((g >> 28) & 1u) - ox < 1 << ws && qy0 + (int)((g >> 29) & 1u) - oy < BIN_CELLS >> ws;
     };
     const uint32_t tri0 = dr.tri_begin + base + threadIdx.x;
     uint32_t lpa[TPT], lpb[TPT];   // LDS counts: tiles (0,0) | (1,0) << 16, (0,1) | (1,1) << 16
@@ -408,8 +370,8 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
             const bool wide = geo[k] & GEO_WIDE, tall = geo[k] & GEO_TALL;
             uint32_t l0 = atomicAdd(&w_cnt[c], 1u), l1 = 0, l2 = 0, l3 = 0;
             if (wide) l1 = atomicAdd(&w_cnt[c + 1], 1u);
-            if (tall) l2 = atomicAdd(&w_cnt[c + BIN_WIN], 1u);
-            if (wide && tall) l3 = atomicAdd(&w_cnt[c + BIN_WIN + 1], 1u);
+            if (tall) l2 = atomicAdd(&w_cnt[c + (1 << ws)], 1u);
+            if (wide && tall) l3 = atomicAdd(&w_cnt[c + (1 << ws) + 1], 1u);
             lpa[k] = l0 | (l1 << 16);
             lpb[k] = l2 | (l3 << 16);
         }
@@ -423,15 +385,17 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
     __syncthreads();
 
     int32_t* fnl = nl + fr.nl_off;
-    {
-        const uint32_t n = w_cnt[threadIdx.x];
+    const uint32_t cells = (uint32_t)min(tiles_h << ws, BIN_CELLS);
+    for (uint32_t c = threadIdx.x; c < cells; c += BIN_BLOCK) {
+        const uint32_t n = w_cnt[c];
         if (n) {
-            const uint64_t gt = tile_begin + (uint64_t)(oy + (int)(threadIdx.x / BIN_WIN)) * tiles_x +
-                                (uint64_t)(ox + (int)(threadIdx.x % BIN_WIN));
+            const uint64_t gt = tile_begin + (uint64_t)(oy + (int)(c >> ws)) * tiles_x + (uint64_t)(ox + (int)(c & ((1u << ws) - 1)));
             const uint32_t pos = atomicAdd(&cursor[gt], n);
             if (!COUNT) {
-                w_base[threadIdx.x] = off[gt] + pos;
-                w_end[threadIdx.x] = off[gt + 1];
+                const uint64_t o = off[gt];
+                const uint32_t cap = (uint32_t)(off[gt + 1] - o);
+                w_base[c] = o + pos;
+                w_room[c] = pos < cap ? cap - pos : 0u;
             }
         }
     }
@@ -444,51 +408,34 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
     // Phase 3: entries.
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
-        if (!((tiled >> k) & 1u)) continue;
+        if (!((small >> k) & 1u)) continue;
         const uint32_t local = base + (uint32_t)k * BIN_BLOCK + threadIdx.x;
         const uint32_t entry = (dr.tri_begin + local) | ((geo[k] & GEO_LOOSE) ? LOOSE_FLAG : 0u);
+        const bool wide = geo[k] & GEO_WIDE, tall = geo[k] & GEO_TALL;
         int c;
-        if ((small >> k) & 1u) {
-            const bool wide = geo[k] & GEO_WIDE, tall = geo[k] & GEO_TALL;
-            if (in_window(geo[k], c)) {
-                if (!COUNT) {
-                    auto put = [&](int cc, uint32_t l) {
-                        const uint64_t p = w_base[cc] + l;
-                        if (p < w_end[cc]) pool[p] = entry;
-                        else overflow[frame] = 1u;
-                    };
-                    put(c, lpa[k] & 0xFFFFu);
-                    if (wide) put(c + 1, lpa[k] >> 16);
-                    if (tall) put(c + BIN_WIN, lpb[k] & 0xFFFFu);
-                    if (wide && tall) put(c + BIN_WIN + 1, lpb[k] >> 16);
-                }
-            } else {
-                // a small rectangle outside the window: one global atomic per tile
-                const int qx0 = (int)(geo[k] & 0x3FFFu), qy0 = (int)((geo[k] >> 14) & 0x3FFFu);
-                for (int j = 0; j <= (int)tall; ++j)
-                    for (int i = 0; i <= (int)wide; ++i) {
-                        const uint64_t gt = tile_begin + (uint64_t)(qy0 + j) * tiles_x + (uint64_t)(qx0 + i);
-                        const uint32_t pos = atomicAdd(&cursor[gt], 1u);
-                        put_entry<COUNT>(gt, pos, entry, off, pool, overflow, frame);
-                    }
+        if (in_window(geo[k], c)) {
+            if (!COUNT) {
+                auto put = [&](int cc, uint32_t l) {
+                    if (l < w_room[cc]) pool[w_base[cc] + l] = entry;
+                    else overflow[frame] = 1u;
+                };
+                put(c, lpa[k] & 0xFFFFu);
+                if (wide) put(c + 1, lpa[k] >> 16);
+                if (tall) put(c + (1 << ws), lpb[k] & 0xFFFFu);
+                if (wide && tall) put(c + (1 << ws) + 1, lpb[k] >> 16);
             }
         } else {
-            // large or part-wrapping boxes (few): set up again, one global
-            // atomic per tile
-            Tri t;
-            setup_draw_tri(dr, local, W, H, t);
-            int bx0, bx1;
-            box_x(t, !(geo[k] & GEO_LOOSE), bx0, bx1);
-            TileRects r;
-            tile_rects(bx0, bx1, t.y0, t.y1d - 1, W, tws, ths, r);
-            TileIter it;
-            iter_begin(r, it);
-            while (it.phase < 2) {
-                const uint64_t gt = tile_begin + (uint64_t)it.ty * tiles_x + (uint64_t)it.tx;
-                const uint32_t pos = atomicAdd(&cursor[gt], 1u);
-                put_entry<COUNT>(gt, pos, entry, off, pool, overflow, frame);
-                iter_next(r, it);
-            }
+            // outside the window: one global atomic per tile, in flight together
+            const uint64_t gt = tile_begin + (uint64_t)((geo[k] >> 14) & 0x3FFFu) * tiles_x + (uint64_t)(geo[k] & 0x3FFFu);
+            uint32_t p1 = 0, p2 = 0, p3 = 0;
+            const uint32_t p0 = atomicAdd(&cursor[gt], 1u);
+            if (wide) p1 = atomicAdd(&cursor[gt + 1], 1u);
+            if (tall) p2 = atomicAdd(&cursor[gt + tiles_x], 1u);
+            if (wide && tall) p3 = atomicAdd(&cursor[gt + tiles_x + 1], 1u);
+            put_entry<COUNT>(gt, p0, entry, off, pool, overflow, frame);
+            if (wide) put_entry<COUNT>(gt + 1, p1, entry, off, pool, overflow, frame);
+            if (tall) put_entry<COUNT>(gt + tiles_x, p2, entry, off, pool, overflow, frame);
+            if (wide && tall) put_entry<COUNT>(gt + tiles_x + 1, p3, entry, off, pool, overflow, frame);
         }
     }
     if (hi >= lo && !nl_lds) {   // uniform per block
@@ -517,12 +464,13 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(const Draw* __restrict__ draw
 }
 
 // ---------------------------------------------------------------------------
-// k_careful: exact boxes of the triangles the bound could not decide
+// k_careful: triangles of many tiles, and exact boxes of those the bound could not decide
 // ---------------------------------------------------------------------------
 // One wavefront per careful triangle.  CLS_SPANS: the lanes split the rows of
 // the domain, each row's exact span comes from row_span(), and the box is the
-// wave's min/max; CLS_FULL: the whole domain.  The lanes then append the
-// triangle to every tile of the box, and lane 0 stores the box for the raster.
+// wave's min/max; CLS_FULL: the whole domain.  CLS_BOX / CLS_TIGHT triangles
+// come here for their many tiles.  The lanes then append the triangle to every
+// tile of the box, and lane 0 stores a box that the raster cannot derive.
 template <bool COUNT>
 __device__ __forceinline__ void careful_one(const Frame* __restrict__ frames, int tws,
                                             int ths, uint32_t* __restrict__ cursor, const uint64_t* __restrict__ off,
@@ -545,6 +493,7 @@ __device__ __forceinline__ void careful_one(const Frame* __restrict__ frames, in
     const uint32_t T = in.y;
     const uint32_t cls = setup_class(t);
     int bx0 = t.x0, bx1 = t.x1d - 1, by0 = t.y0, by1 = t.y1d - 1;
+    uint32_t entry = CAREFUL_FLAG | w;
     if (cls == CLS_SPANS) {
         int lo_x = 1 << 30, hi_x = -1, first = 1 << 30, last = -1;
         for (int y = t.y0 + lane; y < t.y1d; y += 64) {
@@ -560,10 +509,13 @@ __device__ __forceinline__ void careful_one(const Frame* __restrict__ frames, in
         bx1 = wave_max(hi_x);
         by0 = wave_min(first);
         by1 = wave_max(last);
+    } else if (cls == CLS_BOX || cls == CLS_TIGHT) {
+        box_x(t, cls == CLS_TIGHT, bx0, bx1);
+        entry = T | (cls == CLS_BOX ? LOOSE_FLAG : 0u);
     } else if (cls != CLS_FULL) {
         bx1 = -1;   // decided after all (cannot happen for entries k_bin sent here)
     }
-    if (lane == 0 && !COUNT)
+    if (lane == 0 && !COUNT && entry == (CAREFUL_FLAG | w))
         careful_box[w] = make_uint4(T, (uint32_t)max(bx0, 0), (uint32_t)max(bx1, 0),
                                     (uint32_t)max(by0, 0) | ((uint32_t)max(by1, 0) << 16));
     if (bx0 > bx1 || by0 > by1) return;
@@ -591,7 +543,7 @@ __device__ __forceinline__ void careful_one(const Frame* __restrict__ frames, in
         }
         const uint64_t gt = fr.tile_begin + (uint64_t)ty * fr.tiles_x + (uint64_t)tx;
         const uint32_t pos = atomicAdd(&cursor[gt], 1u);
-        put_entry<COUNT>(gt, pos, CAREFUL_FLAG | w, off, pool, overflow, frame);
+        put_entry<COUNT>(gt, pos, entry, off, pool, overflow, frame);
     }
 }
 
@@ -1757,13 +1709,14 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     if (const char* e = getenv("SLOTH_BIG_WALK")) big_walk = e[0] == '1';
     // the binning kernel's segment-tree newline rows pay once one triangle
     // in 256 spans more than TALL_ROWS rows (a wavefront's row loop lasts as
-    // long as its tallest triangle's)
-    const bool tree = (uint64_t)cnt[TALL_CNT] * 256 >= n_tri && cnt[TALL_CNT] > 0;
-    bin_tree = tree;
+    // long as its tallest triangle's); among draws of different sizes a block
+    // of them is enough, since the launch waits for the few blocks of a small
+    // draw of tall triangles (30 unlike jobs: 104-131 -> 53-59 us)
+    bin_tree = cnt[TALL_CNT] > 0 && ((uint64_t)cnt[TALL_CNT] * 256 >= n_tri || (flat_bin && cnt[TALL_CNT] >= (uint32_t)BIN_BLOCK));
     if (const char* e = getenv("SLOTH_BIN_TREE")) bin_tree = e[0] == '1';
     if (n_careful > careful_cap) {
         // 2. room for the careful list, then count again so that it is filled
-        careful_cap = n_careful + n_careful / 4 + 256;
+        careful_cap = n_careful + n_careful / 2 + 1024;
         if ((rc = d_careful_in.reserve(2 * sizeof(uint4) * careful_cap))) return rc;
         if ((rc = d_careful_box.reserve(sizeof(uint4) * careful_cap))) return rc;
         if ((rc = launch_clear(frames, 0, F, s))) return rc;
