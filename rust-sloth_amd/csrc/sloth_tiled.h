@@ -156,9 +156,14 @@ struct TiledPlan {
     void set_walk(int mode) { walk_force = mode; }
     // the common instance's variant (the odd one has no big-box walk)
     bool walk() const { return walk_force >= 0 ? walk_force == 1 : big_walk; }
-    // Triangles per thread of k_bin: 1, 2 or 4 (set by the autotuner).
+    // Triangles per thread of k_bin: 1, 2 or 4 (plan()'s choice until set).
     int bin_tpt = 4;
-    void set_bin_tpt(int t) { bin_tpt = t; }
+    bool user_tpt = false;
+    void set_bin_tpt(int t)
+    {
+        bin_tpt = t;
+        user_tpt = true;
+    }
     // LDS of the even- or odd-width raster instance at the current tile size
     size_t raster_lds(bool odd) const;
     // Both parities' instances the job needs can take the current tile size

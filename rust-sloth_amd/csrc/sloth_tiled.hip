@@ -1552,8 +1552,39 @@ int TiledPlan::plan(std::vector<Frame>& frames, const std::vector<Draw>& draws, 
     if (ev != has_even || od != has_odd) sized = false;
     has_even = ev;
     has_odd = od;
-    // odd widths hold twice the slots per tile: half the default height
-    if (!user_tile) TH = has_odd ? 16 : 32;
+    // Jobs that were not tuned.  Tiles of 64 x 32 cells when there are as many
+    // as the chip takes at once (7 workgroups per CU); else lower ones, and for
+    // the smallest jobs 16 x 16, since a launch lasts as long as one tile then.
+    // Odd widths hold twice the slots in some tiles: half the height.  A render
+    // at 64 x 32 / 64 x 16 / 16 x 16 cells: 80x24 (2 tiles of 64 x 32) 17.3 /
+    // 16.5 / 14.4 us, 240x70 (12) 23.3 / 19.0 / 15.9, four meshes on 640x480
+    // (150) 30.0 / 27.1 / 27.9, 100 frames of 100x100 (800) 29.0 / 23.6 / 29.1,
+    // six meshes on 1920x1080 (1020) 60.1 / 43.7 / 43.7, four frames of 1280x720
+    // (1840) 38.2 / 45.1 / 80.7; 641x481 at half the heights 52.1 / 46.6 / 47.6.
+    if (!user_tile) {
+        auto count = [&](uint32_t tw, uint32_t th) {
+            uint64_t n = 0;
+            for (const Frame& f : frames) n += (uint64_t)((f.W + tw - 1) / tw) * ((f.H + th - 1) / th);
+            return n;
+        };
+        const uint32_t odd = has_odd ? 2 : 1;
+        const uint32_t tw = TW, th = TH;
+        TW = 64;
+        TH = 32;
+        if (count(TW, TH) < 1792) TH = 16;
+        if (TH == 16 && count(TW, TH) < 256) TW = 16;
+        TH /= odd;
+        if (tw != TW || th != TH) sized = false;
+    }
+    // k_bin's triangles per thread: several serve jobs whose blocks wait in
+    // line, one the others (the same jobs: 10.6 us with 4 / 6.7 with 1, 11.3 /
+    // 6.9, 13.0 / 7.4, 12.5 / 8.3, 16.4 / 12.9, 14.4 / 7.9; 1,310,720 triangles
+    // 17.9 / 14.8, and 15.5 with 2; 5 million in 30 draws 57 / 113)
+    if (!user_tpt) {
+        uint64_t n = 0;
+        for (const Draw& d : draws) n += d.n;
+        bin_tpt = n <= 1u << 20 ? 1 : n <= 1u << 21 ? 2 : 4;
+    }
     uint64_t tiles = 0;
     for (Frame& f : frames) {
         f.tiles_x = (f.W + TW - 1) / TW;
