@@ -141,6 +141,7 @@ struct TiledPlan {
         uint32_t tiles_x = 0, tiles_y = 0, H = 0;  // of the largest frame, each
         bool one = true;                           // every frame has exactly one draw
         bool even = false, odd = false;            // width parities
+        bool ragged = false;                       // most cells lie in frames whose width is no multiple of 32
     };
     Range whole;
     uint32_t n_frames = 0;
@@ -164,6 +165,15 @@ struct TiledPlan {
         bin_tpt = t;
         user_tpt = true;
     }
+    // The default plan's tiles of 64 x 32 cells keep the memory lines that they
+    // share with the tiles beside them (widths that are no multiples of 32
+    // cells) in the L2 until those have written their part; memory reads a line
+    // that it is given a part of.  Three batches in turn: 64 frames of 1918x1079
+    // 513 -> 406 us, of 1919x1079 527 -> 427, 120 of 641x480 162 -> 130.  Narrower
+    // and lower tiles lose (32 x 16: 838 -> 930, 64 x 16: 506 -> 597), and the wider
+    // ones that tuning finds are as fast without (128 x 16: 402 and 411, 512 x 8:
+    // 371 and 404), which repeated renders of one batch do not tell it.
+    bool keep_lines() const { return !user_tile && TW == 64 && TH == 32; }
     // LDS of the even- or odd-width raster instance at the current tile size
     size_t raster_lds(bool odd) const;
     // Both parities' instances the job needs can take the current tile size

@@ -813,12 +813,13 @@ __device__ __forceinline__ uint32_t entry_tri(uint32_t e, const uint4* __restric
 // is finished by k_tile_edges, from the winners this tile and its left
 // neighbour leave in `edge_out` (first and last column, per row).
 // Tile (tx, ty) of frame fr, global tile index gt, whose list is pool[o, o + n).
-// KIND: EVEN for launches without odd widths, ANY for those with some, WRAPPED
-// for WRAP tiles.  FLAT is that of the calling kernel and changes nothing here: it gives each
+// KIND: EVEN for launches most of whose widths are multiples of 32 cells (a
+// 128-byte line), RAGGED for the others of even widths, ANY for those with odd
+// ones, WRAPPED for WRAP tiles.  FLAT is that of the calling kernel and changes nothing here: it gives each
 // kernel its own copy of the lambdas below, which the compiler then inlines
 // as it does for a single caller (shared by the two kernels, they cost the
 // 3-D instances two VGPRs spilled to scratch).
-enum RasterKind { EVEN, ANY, WRAPPED };
+enum RasterKind { EVEN, RAGGED, ANY, WRAPPED };
 template <bool BIG, bool ONE, RasterKind KIND, bool FLAT>
 __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, const Ramp* __restrict__ ramps,
                                             const Ramp* s_ramp, uint32_t* s_negz, const Frame& fr, uint32_t tx,
@@ -826,9 +827,9 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
                                             const uint32_t* __restrict__ pool, const int32_t* __restrict__ nl,
                                             const uint4* __restrict__ careful_box, uint32_t* __restrict__ cells,
                                             float* __restrict__ zbuf, int32_t* __restrict__ win, uint32_t win_raw,
-                                            uint4* __restrict__ edge_out, uint64_t* smem)
+                                            uint4* __restrict__ edge_out, uint64_t* smem, uint32_t keep)
 {
-    constexpr bool WRAP = KIND == WRAPPED;
+    constexpr bool WRAP = KIND == WRAPPED, EVENS = KIND == EVEN || KIND == RAGGED;
     static_assert(!(BIG && WRAP), "the big-box walk maps slots of even columns only");
     const uint32_t W = fr.W, H = fr.H;
     const int sws = tws - (WRAP ? 0 : 1);
@@ -889,7 +890,7 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
         const uint32_t q = threadIdx.x & ((1u << (sws - 1)) - 1);
         const int col = g.tc0 + ((int)q << 2);
         if (col >= g.tc1) return;
-        const int have = KIND == EVEN ? (col + 2 < g.tc1 ? 4 : 2) : min(g.tc1 - col, 4);
+        const int have = EVENS ? (col + 2 < g.tc1 ? 4 : 2) : min(g.tc1 - col, 4);
         const int step = (int)(blockDim.x >> (sws - 1));
         int r = (int)(threadIdx.x >> (sws - 1));
         uint32_t off = ((uint32_t)r * W + (q << 2)) * 4u;
@@ -905,13 +906,25 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
     // address is one instruction.
     typedef unsigned int v4u __attribute__((ext_vector_type(4), aligned(4)));
     typedef unsigned int v2u __attribute__((ext_vector_type(2), aligned(4)));
-    auto put4 = [](uint8_t* p, uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    // But where `keep` says so, the lines that a row shares with the tiles beside
+    // it are written by ordinary stores, which stay in the L2 until the
+    // neighbour's part has come (TiledPlan::keep_lines).
+    const bool shared_lines = keep && (W & 31u);
+    auto put4 = [&](uint8_t* p, uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
         const v4u v = {a, b, c, d};
+        if (KIND != EVEN && shared_lines) {
+            const uint32_t at = (uint32_t)(uintptr_t)p, row = at - ((threadIdx.x & ((1u << (tws - 2)) - 1)) << 4);
+            if ((at & ~127u) < row || ((at + 15u) | 127u) >= row + (4u << tws)) {
+                *(v4u*)p = v;
+                asm volatile("");   // keeps the two stores two
+                return;
+            }
+        }
         __builtin_nontemporal_store(v, (v4u*)p);
     };
     // the first `have` < 4 words (ANY: 1 and 3 at an odd width's last column)
     auto put_some = [](uint8_t* p, uint32_t a, uint32_t b, uint32_t c, int have) {
-        if (KIND == EVEN || (have & 2)) {
+        if (EVENS || (have & 2)) {
             const v2u v = {a, b};
             __builtin_nontemporal_store(v, (v2u*)p);
         }
@@ -1358,13 +1371,13 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
         for (uint32_t i = threadIdx.x; i < H; i += blockDim.x) __builtin_nontemporal_store(CELL_BLANK, fc + (uint64_t)W * H + i);
 }
 
-// The tile of a frame's workgroup r, ANY: workgroups go to the eight XCDs in
-// turn, so taking eight tile rows at a time gives each XCD, and its L2, whole
-// rows.  The rows of an odd width start at any 4-byte address, and the lines
-// that two tiles of a row share are then put together before they leave for
-// memory: 64 frames of 1919x1079 at 128 x 16 cells 474 -> 416 us, at 32 x 32
-// 1020 -> 727.  Even widths' tiles share no line: 256 frames of 1920x1080 lose
-// (1.79 -> 1.825 ms), so they keep the plain order.
+// The tile of a frame's workgroup r, RAGGED and ANY: workgroups go to the eight
+// XCDs in turn, so taking eight tile rows at a time gives each XCD, and its L2,
+// whole rows.  The rows of such widths start within a line, and the lines that
+// two tiles of a row share are then put together before they leave for memory:
+// 64 frames of 1919x1079 at 128 x 16 cells 474 -> 416 us, at 32 x 32 1020 -> 727;
+// of 1918x1079 at 128 x 16 465 -> 410, at 64 x 32 620 -> 524.  Where tiles share
+// no line, 256 frames of 1920x1080 lose (1.79 -> 1.825 ms) and keep the plain order.
 __device__ __forceinline__ void tile_of(uint32_t r, uint32_t nx, uint32_t ny, uint32_t& tx, uint32_t& ty)
 {
     const uint32_t full = (ny & ~7u) * nx;
@@ -1391,7 +1404,7 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
     const uint32_t* __restrict__ pool, int32_t* __restrict__ nl, const uint4* __restrict__ careful_box,
     uint32_t* __restrict__ cells, float* __restrict__ zbuf, int32_t* __restrict__ win, uint32_t win_raw,
     uint32_t n_ramps, uint4* __restrict__ edge_out, uint32_t* __restrict__ careful_reset,
-    const uint2* __restrict__ tile_frame, uint32_t t_lo, uint32_t odd_cols)
+    const uint2* __restrict__ tile_frame, uint32_t t_lo, uint32_t odd_cols, uint32_t keep)
 {
     extern __shared__ uint64_t smem[];
     // the job's first LDS_RAMPS shaders, so that a glyph lookup reads LDS
@@ -1414,12 +1427,12 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
         f = f_lo + blockIdx.z;
         tx = blockIdx.x;
         ty = blockIdx.y;
-        if constexpr (KIND == ANY) tile_of(ty * gridDim.x + tx, gridDim.x, gridDim.y, tx, ty);
+        if constexpr (KIND == RAGGED || KIND == ANY) tile_of(ty * gridDim.x + tx, gridDim.x, gridDim.y, tx, ty);
     }
     const Frame& fr = frames[f];
     constexpr bool WRAP = KIND == WRAPPED;
     if (tx >= fr.tiles_x || ty >= fr.tiles_y) return;
-    if (KIND != EVEN && ((fr.W & 1u) && tx < odd_cols) != WRAP) return;
+    if ((KIND == ANY || WRAP) && ((fr.W & 1u) && tx < odd_cols) != WRAP) return;
     const uint64_t gt = fr.tile_begin + (uint64_t)ty * fr.tiles_x + tx;
     const uint64_t o = off[gt];
     const uint32_t c = cursor[gt];
@@ -1428,7 +1441,7 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
         for (uint32_t i = threadIdx.x; i < min(n_ramps, LDS_RAMPS) * (uint32_t)sizeof(Ramp) / 4; i += blockDim.x)
             ((uint32_t*)s_ramp)[i] = ((const uint32_t*)ramps)[i];
     raster_tile<BIG, ONE, KIND, FLAT>(draws, ramps, s_ramp, &s_negz, fr, tx, ty, gt, o, n, tws, ths, pool, nl, careful_box,
-                                      cells, zbuf, win, win_raw, edge_out, smem);
+                                      cells, zbuf, win, win_raw, edge_out, smem, keep);
     // The tile leaves its binning state as k_tile_clear would for the next
     // render: its cursor at 0 and, but for frames one column wide (k_tile_edges
     // reads their rows after this), the newline rows of its tile row back at -1
@@ -1529,6 +1542,7 @@ TiledPlan::Range TiledPlan::range(const std::vector<Frame>& frames, const std::v
 {
     if (f_lo == 0 && f_hi == n_frames) return whole;
     Range r;
+    uint64_t slots = 0, ragged = 0;
     for (uint32_t f = f_lo; f < f_hi; ++f) {
         const Frame& fr = frames[f];
         r.tiles_x = std::max(r.tiles_x, fr.tiles_x);
@@ -1536,8 +1550,11 @@ TiledPlan::Range TiledPlan::range(const std::vector<Frame>& frames, const std::v
         r.H = std::max(r.H, fr.H);
         r.one = r.one && fr.draw_end - fr.draw_begin == 1;
         ((fr.W & 1u) ? r.odd : r.even) = true;
+        slots += (uint64_t)fr.W * fr.H;
+        if (fr.W & 31u) ragged += (uint64_t)fr.W * fr.H;
         for (uint32_t d = fr.draw_begin; d < fr.draw_end; ++d) r.max_draw = std::max(r.max_draw, draws[d].n);
     }
+    r.ragged = ragged * 2 > slots;
     return r;
 }
 
@@ -1555,7 +1572,8 @@ int TiledPlan::plan(std::vector<Frame>& frames, const std::vector<Draw>& draws, 
     // Jobs that were not tuned.  Tiles of 64 x 32 cells when there are as many
     // as the chip takes at once (7 workgroups per CU); else lower ones, and for
     // the smallest jobs 16 x 16, since a launch lasts as long as one tile then.
-    // Odd widths hold twice the slots in some tiles: half the height.  A render
+    // Odd widths hold twice the slots in some tiles: half the height of the
+    // smaller two (120 frames of 641x480 at 64 x 32 / 64 x 16 158 / 199 us).  A render
     // at 64 x 32 / 64 x 16 / 16 x 16 cells: 80x24 (2 tiles of 64 x 32) 17.3 /
     // 16.5 / 14.4 us, 240x70 (12) 23.3 / 19.0 / 15.9, four meshes on 640x480
     // (150) 30.0 / 27.1 / 27.9, 100 frames of 100x100 (800) 29.0 / 23.6 / 29.1,
@@ -1571,9 +1589,11 @@ int TiledPlan::plan(std::vector<Frame>& frames, const std::vector<Draw>& draws, 
         const uint32_t tw = TW, th = TH;
         TW = 64;
         TH = 32;
-        if (count(TW, TH) < 1792) TH = 16;
-        if (TH == 16 && count(TW, TH) < 256) TW = 16;
-        TH /= odd;
+        if (count(TW, TH) < 1792) {
+            TH = 16;
+            if (count(TW, TH) < 256) TW = 16;
+            TH /= odd;
+        }
         if (tw != TW || th != TH) sized = false;
     }
     // k_bin's triangles per thread: several serve jobs whose blocks wait in
@@ -1822,7 +1842,7 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     return SLOTH_OK;
 }
 
-// The common raster instance: with odd widths or not, big-box walk or not, one
+// The common raster instance: odd widths, ragged ones or neither, big-box walk or not, one
 // draw per frame or not, flat grid (frames of different tile grids) or 3-D.  Each instance is compiled
 // on its own, so the 3-D instances carry no flat-grid mapping and its
 // registers.
@@ -1834,9 +1854,10 @@ static auto raster_kernel(bool walk, bool one)
 }
 
 template <bool FLAT>
-static auto raster_kernel(bool walk, bool one, bool odd)
+static auto raster_kernel(bool walk, bool one, bool odd, bool ragged)
 {
-    return odd ? raster_kernel<FLAT, ANY>(walk, one) : raster_kernel<FLAT, EVEN>(walk, one);
+    return odd ? raster_kernel<FLAT, ANY>(walk, one)
+               : ragged ? raster_kernel<FLAT, RAGGED>(walk, one) : raster_kernel<FLAT, EVEN>(walk, one);
 }
 
 int TiledPlan::launch_raster(const std::vector<Frame>& frames, const std::vector<Draw>& draws, const Frame* d_frames,
@@ -1870,12 +1891,12 @@ int TiledPlan::launch_raster(const std::vector<Frame>& frames, const std::vector
             hipLaunchKernelGGL(kern, grid, dim3(RASTER_BLOCK), lds, s, d_draws, d_ramps, d_frames, f0, log2u(TW),
                                log2u(TH), d_cursor.as<uint32_t>(), d_off.as<uint64_t>(), pool,
                                d_nl.as<int32_t>(), d_careful_box.as<uint4>(), cells, z, win, win_raw ? 1u : 0u,
-                               n_ramps, edges, careful_reset, tf, (uint32_t)t_lo, odd_cols());
+                               n_ramps, edges, careful_reset, tf, (uint32_t)t_lo, odd_cols(), keep_lines() ? 1u : 0u);
             careful_reset = nullptr;
         };
         if (ev) {
-            go(flat_raster ? raster_kernel<true>(walk(), one, rg.odd) : raster_kernel<false>(walk(), one, rg.odd), grid,
-               raster_lds(false));
+            go(flat_raster ? raster_kernel<true>(walk(), one, rg.odd, rg.ragged) : raster_kernel<false>(walk(), one, rg.odd, rg.ragged),
+               grid, raster_lds(false));
             HIP_TRY(hipGetLastError());
         }
         if (od) {

@@ -14,7 +14,7 @@ EYE = np.eye(4, dtype=np.float32).reshape(16)
 # width, height, frames -> tile
 PLANS = [(80, 24, 1, (16, 16)), (1, 1, 1, (16, 8)), (1020, 240, 1, (16, 16)), (1024, 256, 1, (64, 16)),
          (1024, 256, 13, (64, 16)), (1024, 256, 14, (64, 32)), (81, 25, 1, (16, 8)), (1023, 256, 1, (64, 8)),
-         (1023, 256, 14, (64, 16)), (65, 40, 300, (64, 8))]
+         (1023, 256, 13, (64, 8)), (1023, 256, 14, (64, 32)), (65, 40, 300, (64, 8))]
 
 
 @pytest.mark.parametrize("W,H,frames,tile", PLANS)
