@@ -845,6 +845,9 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
 
     const uint32_t* list = pool + o;
     uint64_t* keys = smem;
+    // (S, the tile's slots, is a power of two of at least 16)
+    static_assert(CHUNK * sizeof(uint2) % 16 == 0 && CHUNK * sizeof(float4) % 16 == 0 && CHUNK * sizeof(float2) % 16 == 0,
+                  "each array of the rows, and the cells after them, start on 16 bytes");
     Rows rows;
     rows.end = (uint2*)(keys + S);
     rows.v12 = (float4*)(rows.end + CHUNK);
@@ -1406,7 +1409,8 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
     uint32_t n_ramps, uint4* __restrict__ edge_out, uint32_t* __restrict__ careful_reset,
     const uint2* __restrict__ tile_frame, uint32_t t_lo, uint32_t odd_cols, uint32_t keep)
 {
-    extern __shared__ uint64_t smem[];
+    // keys, rows and cells are read and written in 16-byte words
+    extern __shared__ __align__(16) uint64_t smem[];
     // the job's first LDS_RAMPS shaders, so that a glyph lookup reads LDS
     // (read only after the tile's first barrier)
     __shared__ Ramp s_ramp[LDS_RAMPS];
