@@ -15,8 +15,9 @@
 
 namespace sloth {
 
-// The pool keeps freed blocks while a handle lives (at most PIN_POOL_BYTES)
-// and frees them with the last one.  Safe from any thread.
+// The pool keeps freed blocks while a handle lives (at most PIN_POOL_BYTES,
+// the latest ones; sizes are powers of two, and a lease takes a block of its
+// own size only) and frees them with the last one.  Safe from any thread.
 constexpr size_t PIN_POOL_BYTES = 64u << 20;
 struct PinPoolUser {
     PinPoolUser();

@@ -17,9 +17,16 @@ struct Block {
 };
 struct Pool {
     std::mutex mu;
-    std::array<Block, 32> idle;
+    std::array<Block, 32> idle;   // longest idle first
     size_t n = 0, bytes = 0;
     int users = 0;
+    Block remove(size_t i)
+    {
+        const Block b = idle[i];
+        bytes -= b.bytes;
+        std::copy(idle.begin() + i + 1, idle.begin() + n--, idle.begin() + i);
+        return b;
+    }
 };
 // never destroyed: handles may outlive static destructors
 Pool& pool()
@@ -54,16 +61,15 @@ int PinLease::take(size_t need, hipStream_t s)
     Pool& q = pool();
     {
         std::lock_guard<std::mutex> lk(q.mu);
-        size_t best = q.n;
-        for (size_t i = 0; i < q.n; ++i)
-            if (q.idle[i].bytes >= want && (best == q.n || q.idle[i].bytes < q.idle[best].bytes)) best = i;
-        if (best < q.n) {
-            p = q.idle[best].p;
-            bytes = q.idle[best].bytes;
-            q.bytes -= bytes;
-            q.idle[best] = q.idle[--q.n];
-            return SLOTH_OK;
-        }
+        // only a block of this size: a handle that kept a larger one for its
+        // life would hold more than it needs, and the next large copy would
+        // allocate anew
+        for (size_t i = q.n; i-- > 0;)
+            if (q.idle[i].bytes == want) {
+                p = q.remove(i).p;
+                bytes = want;
+                return SLOTH_OK;
+            }
     }
     const hipError_t e = hipHostMalloc(&p, want, hipHostMallocPortable);
     if (e != hipSuccess) {
@@ -82,15 +88,19 @@ void PinLease::end()
     const Block own{p, bytes};
     p = nullptr;
     Pool& q = pool();
+    std::array<Block, std::tuple_size<decltype(q.idle)>::value> out;   // freed, those longest idle
+    size_t n_out = 0;
     {
         std::lock_guard<std::mutex> lk(q.mu);
-        if (q.users > 0 && q.n < q.idle.size() && q.bytes + own.bytes <= PIN_POOL_BYTES) {
+        if (q.users > 0 && own.bytes <= PIN_POOL_BYTES) {
+            while (q.n == q.idle.size() || q.bytes + own.bytes > PIN_POOL_BYTES) out[n_out++] = q.remove(0);
             q.idle[q.n++] = own;
             q.bytes += own.bytes;
-            return;
+        } else {
+            out[n_out++] = own;
         }
     }
-    (void)hipHostFree(own.p);
+    for (size_t i = 0; i < n_out; ++i) (void)hipHostFree(out[i].p);
 }
 
 int copy_in(const Span* spans, int n, PinLease& lease, hipStream_t s)
