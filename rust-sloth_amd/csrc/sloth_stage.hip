@@ -4,6 +4,8 @@
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -153,6 +155,40 @@ static void on_threads(int n, F&& work, G&& before_own)
     }
 }
 
+// A value that one thread sets and others wait for: awake for as long as a
+// short render and its copy take (a thread that sleeps is back tens of
+// microseconds late), asleep from then on (the stream may hold any amount of
+// work).
+class Gate {
+  public:
+    int wait()
+    {
+        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+        while (!value.load(std::memory_order_acquire)) {
+            if (std::chrono::steady_clock::now() >= until) {
+                std::unique_lock<std::mutex> lk(mu);
+                set.wait(lk, [&] { return value.load(std::memory_order_relaxed) != 0; });
+                break;
+            }
+            std::this_thread::yield();
+        }
+        return value.load(std::memory_order_acquire);
+    }
+    void open(int v)
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            value.store(v, std::memory_order_release);
+        }
+        set.notify_all();
+    }
+
+  private:
+    std::atomic<int> value{0};
+    std::mutex mu;
+    std::condition_variable set;
+};
+
 static size_t room(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // All spans through one pinned block of `total` bytes.
@@ -179,17 +215,16 @@ static int copy_out_block(const Span* spans, int n, size_t total, hipStream_t s)
         e = hipStreamSynchronize(s);
         if (e == hipSuccess) empty(0, total);
     } else {
-        std::atomic<int> there{0};   // 1: the block is filled, 2: it never will be
+        Gate there;   // 1: the block is filled, 2: it never will be
         on_threads(
             COPY_THREADS,
             [&](int w) {
-                while (!there.load(std::memory_order_acquire)) std::this_thread::yield();
-                if (there.load(std::memory_order_relaxed) == 1)
+                if (there.wait() == 1)
                     empty(total * (size_t)w / COPY_THREADS, total * (size_t)(w + 1) / COPY_THREADS);
             },
             [&] {
                 e = hipStreamSynchronize(s);
-                there.store(e == hipSuccess ? 1 : 2, std::memory_order_release);
+                there.open(e == hipSuccess ? 1 : 2);
             });
     }
     HIP_TRY(e);

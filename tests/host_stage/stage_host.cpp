@@ -4,12 +4,15 @@
 #define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
+#include <ctime>
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "sloth_stage.hip"
@@ -19,6 +22,13 @@ using namespace sloth;
 static std::mutex mu;
 static std::map<void*, size_t> pinned;
 static int allocations = 0;
+// the stream's work lasts until then; a waiting thread is awake, as it is in
+// the runtime
+static std::chrono::steady_clock::time_point busy_until;
+static void wait_for_stream()
+{
+    while (std::chrono::steady_clock::now() < busy_until) std::this_thread::yield();
+}
 
 int sloth::fail(int code, const char* fmt, ...)
 {
@@ -50,7 +60,11 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
     memcpy(d, s, n);
     return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    wait_for_stream();
+    return hipSuccess;
+}
 hipError_t hipGetDevice(int* d)
 {
     *d = 0;
@@ -63,7 +77,11 @@ hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned)
     return hipSuccess;
 }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t)
+{
+    wait_for_stream();
+    return hipSuccess;
+}
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "error"; }
@@ -128,10 +146,31 @@ static int pool_bound()
     return 0;
 }
 
+// A read-back behind a long render leaves the processors to others: the
+// copying threads sleep until there is something to copy.
+static int waits_asleep()
+{
+    PinPoolUser user;
+    std::vector<uint8_t> src(4u << 20), dst(src.size());
+    for (size_t i = 0; i < src.size(); ++i) src[i] = (uint8_t)(i * 7 + (i >> 12));
+    const Span s{dst.data(), src.data(), src.size()};
+    CHECK(copy_out(&s, 1, nullptr) == SLOTH_OK && dst == src);
+    std::fill(dst.begin(), dst.end(), 0);
+    busy_until = std::chrono::steady_clock::now() + std::chrono::milliseconds(400);
+    const clock_t t0 = clock();   // of all threads
+    CHECK(copy_out(&s, 1, nullptr) == SLOTH_OK);
+    const double used = (double)(clock() - t0) / CLOCKS_PER_SEC;
+    CHECK(dst == src);
+    printf("%.3f s of processor time in a wait of 0.4 s\n", used);
+    CHECK(used < 0.6);   // one thread's wait
+    return 0;
+}
+
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "small_lease") return small_lease();
     if (what == "pool_bound") return pool_bound();
+    if (what == "waits_asleep") return waits_asleep();
     return 2;
 }

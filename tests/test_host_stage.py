@@ -18,7 +18,15 @@ def host(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["small_lease", "pool_bound"])
-def test_pinned_pool(host, what):
+def _run(host, what):
     r = subprocess.run([host, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("what", ["small_lease", "pool_bound"])
+def test_pinned_pool(host, what):
+    _run(host, what)
+
+
+def test_read_back_waits_asleep(host):
+    _run(host, "waits_asleep")
