@@ -265,25 +265,32 @@ int copy_out(const Span* spans, int n, hipStream_t s)
         return Span{(uint8_t*)spans[i].host + at, (uint8_t*)spans[i].dev + at, std::min(COPY_SLOT, spans[i].bytes - at)};
     };
     // thread w takes pieces w, w + COPY_THREADS, ... through its own two slots
+    auto slot = [&](int w, int q) { return lease.as<uint8_t>() + (size_t)(2 * w + q) * COPY_SLOT; };
+    auto issue = [&](int w, size_t k, int q) {
+        const Span c = piece(k);
+        return note(hipMemcpyAsync(slot(w, q), c.dev, c.bytes, hipMemcpyDeviceToHost, s)) &&
+               note(hipEventRecord(ev[2 * w + q], s));
+    };
+    Gate begun;   // 1: the first piece is there, 2: it never will be
     auto work = [&](int w) {
-        if (w && !note(hipSetDevice(dev))) return;
-        uint8_t* slot = lease.as<uint8_t>() + (size_t)(2 * w) * COPY_SLOT;
-        auto issue = [&](size_t k, int q) {
-            const Span c = piece(k);
-            return note(hipMemcpyAsync(slot + (size_t)q * COPY_SLOT, c.dev, c.bytes, hipMemcpyDeviceToHost, s)) &&
-                   note(hipEventRecord(ev[2 * w + q], s));
-        };
-        size_t k = (size_t)w;
+        if (begun.wait() != 1 || (w && !note(hipSetDevice(dev)))) return;
         int q = 0;
-        if (k < pieces && !issue(k, q)) return;
-        for (; k < pieces; k += COPY_THREADS, q ^= 1) {
-            if (k + COPY_THREADS < pieces && !issue(k + COPY_THREADS, q ^ 1)) return;
+        for (size_t k = (size_t)w; k < pieces; k += COPY_THREADS, q ^= 1) {
+            if (k + COPY_THREADS < pieces && !issue(w, k + COPY_THREADS, q ^ 1)) return;
             if (!note(hipEventSynchronize(ev[2 * w + q]))) return;
             const Span c = piece(k);
-            memcpy(c.host, slot + (size_t)q * COPY_SLOT, c.bytes);
+            memcpy(c.host, slot(w, q), c.bytes);
         }
     };
-    if (bad.load() == (int)hipSuccess) on_threads(COPY_THREADS, work, [] {});
+    // this thread alone waits for the work before the copy, with every
+    // thread's first piece enqueued behind it
+    auto begin = [&] {
+        for (int w = 0; w < COPY_THREADS && (size_t)w < pieces; ++w)
+            if (!issue(w, (size_t)w, 0)) break;
+        if (bad.load() == (int)hipSuccess) note(hipEventSynchronize(ev[0]));
+        begun.open(bad.load() == (int)hipSuccess ? 1 : 2);
+    };
+    if (bad.load() == (int)hipSuccess) on_threads(COPY_THREADS, work, begin);
     const hipError_t e = (hipError_t)bad.load();
     if (e == hipSuccess) lease.done();   // every piece has been waited for
     for (hipEvent_t v : ev)

@@ -148,10 +148,10 @@ static int pool_bound()
 
 // A read-back behind a long render leaves the processors to others: the
 // copying threads sleep until there is something to copy.
-static int waits_asleep()
+static int waits_asleep(size_t bytes)
 {
     PinPoolUser user;
-    std::vector<uint8_t> src(4u << 20), dst(src.size());
+    std::vector<uint8_t> src(bytes), dst(src.size());
     for (size_t i = 0; i < src.size(); ++i) src[i] = (uint8_t)(i * 7 + (i >> 12));
     const Span s{dst.data(), src.data(), src.size()};
     CHECK(copy_out(&s, 1, nullptr) == SLOTH_OK && dst == src);
@@ -171,6 +171,7 @@ int main(int argc, char** argv)
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "small_lease") return small_lease();
     if (what == "pool_bound") return pool_bound();
-    if (what == "waits_asleep") return waits_asleep();
+    if (what == "waits_asleep") return waits_asleep(4u << 20);
+    if (what == "waits_asleep_long") return waits_asleep((33u << 20) + 5);
     return 2;
 }

@@ -28,5 +28,6 @@ def test_pinned_pool(host, what):
     _run(host, what)
 
 
-def test_read_back_waits_asleep(host):
-    _run(host, "waits_asleep")
+@pytest.mark.parametrize("what", ["waits_asleep", "waits_asleep_long"])
+def test_read_back_waits_asleep(host, what):
+    _run(host, what)
