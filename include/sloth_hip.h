@@ -270,9 +270,11 @@ int sloth_batch_device_frame(sloth_batch *b, uint32_t frame, uint32_t **d_cells,
 
 /* Times each stage of one run with HIP events on the batch's
  * stream: out_ms[i] = milliseconds of stage i, names[i] its kernel name;
- * *n_stages in: capacity, out: count.  On the tiled path the first stage
- * (k_tile_clear) runs only for batches with frames of odd width; otherwise
- * it times two adjacent events. */
+ * *n_stages in: capacity, out: count.  A stage that does not run times two
+ * adjacent events: on the tiled path the first (k_tile_clear), which only
+ * batches with frames one column wide need; on the general path
+ * k_winner_global and k_resolve_global without frames of odd width,
+ * k_finish_global without frames of even width. */
 int sloth_batch_profile(sloth_batch *b, float *out_ms, const char **names, uint32_t *n_stages);
 
 /* Runs `warmup` untimed renders, then `steps` timed renders bracketed by HIP

@@ -380,8 +380,8 @@ struct Job {
             HIP_TRY(hipGetLastError());
         }
         if (ev) HIP_TRY(hipEventRecord((*ev)[2], s));
-        // grids (cells of the largest frame / 256, frames), at most 65535
-        // frames per launch
+        // frames of odd widths by two kernels, of even ones by the last: grids
+        // (cells of the largest frame / 256, frames), at most 65535 frames per launch
         uint64_t max_wh = 0, max_cells = 0, max_even = 0;   // of odd and of even widths
         for (uint32_t f = f_lo; f < f_hi; ++f) {
             const uint64_t wh = (uint64_t)frames[f].W * frames[f].H, n = frame_cells(frames[f]);
@@ -391,14 +391,6 @@ struct Job {
             } else {
                 max_even = std::max(max_even, n - wh / 2);
             }
-        }
-        for (uint32_t f = f_lo; f < f_hi && max_even; f += 65535u) {
-            const uint32_t nf = std::min<uint32_t>(65535u, f_hi - f);
-            hipLaunchKernelGGL(k_finish_global, dim3(blocks_for(max_even), nf), dim3(256), 0, s, dev_draws(),
-                               dev_ramps(), dev_frames(), f, (const uint64_t*)d_keys.as<uint64_t>(),
-                               (const int32_t*)d_nl.as<int32_t>(), d_cells.as<uint32_t>(), d_z.as<float>(), win,
-                               win_raw ? 1u : 0u);
-            HIP_TRY(hipGetLastError());
         }
         for (uint32_t f = f_lo; f < f_hi && max_wh; f += 65535u) {
             const uint32_t nf = std::min<uint32_t>(65535u, f_hi - f);
@@ -416,6 +408,15 @@ struct Job {
             HIP_TRY(hipGetLastError());
         }
         if (ev) HIP_TRY(hipEventRecord((*ev)[4], s));
+        for (uint32_t f = f_lo; f < f_hi && max_even; f += 65535u) {
+            const uint32_t nf = std::min<uint32_t>(65535u, f_hi - f);
+            hipLaunchKernelGGL(k_finish_global, dim3(blocks_for(max_even), nf), dim3(256), 0, s, dev_draws(),
+                               dev_ramps(), dev_frames(), f, (const uint64_t*)d_keys.as<uint64_t>(),
+                               (const int32_t*)d_nl.as<int32_t>(), d_cells.as<uint32_t>(), d_z.as<float>(), win,
+                               win_raw ? 1u : 0u);
+            HIP_TRY(hipGetLastError());
+        }
+        if (ev) HIP_TRY(hipEventRecord((*ev)[5], s));
         return SLOTH_OK;
     }
 
@@ -1333,7 +1334,7 @@ int sloth_batch_profile(sloth_batch* b, float* out_ms, const char** names, uint3
     if (b->job.path == PATH_TILED)
         nm = TiledPlan::stage_names();
     else
-        nm = {"k_clear_global", "k_raster_global", "k_winner_global", "k_resolve_global"};
+        nm = {"k_clear_global", "k_raster_global", "k_winner_global", "k_resolve_global", "k_finish_global"};
     uint32_t cap = *n_stages;
     *n_stages = (uint32_t)nm.size();
     if (!rc && se == hipSuccess) {
