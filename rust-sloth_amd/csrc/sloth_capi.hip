@@ -1584,7 +1584,11 @@ struct sloth_shading {
     bool has_target = false;
     bool has_params = false;
     DevBuf d_faces, d_vis, d_G, d_vcolor, d_vnormal, d_light, d_target, d_out, d_partial, d_vert_acc;
-    // the visibility as fragment lists (k_frag_plan)
+    // the visibility as fragment lists (k_frag_plan), made by the first
+    // backward pass after it: forward passes do without.  The visibility's
+    // tables are kept for that, since the batch's may have new transforms by then.
+    bool lists = false;
+    DevBuf d_vis_tables;
     DevBuf d_seg, d_entries, d_chunks;
     uint64_t n_chunks = 0;
     DevBuf d_dcolor, d_dnormal, d_sum;
@@ -1641,9 +1645,11 @@ static void normal_map(const float* M, float* G)
         for (int c = 0; c < 3; ++c) G[r * 3 + c] = (float)(cof[r][c] / k);
 }
 
-// The fragment lists of the visibility: counted, sized, filled.
+// The fragment lists of the visibility, unless they are there: counted, sized,
+// filled.
 static int shading_lists(sloth_shading* sh)
 {
+    if (sh->lists) return SLOTH_OK;
     Job& j = sh->b->job;
     hipStream_t s = sh->b->stream;
     const uint64_t segs = frag_segments(sh->n_tris, (uint32_t)j.draws.size());
@@ -1652,8 +1658,8 @@ static int shading_lists(sloth_shading* sh)
     PinLease totals;
     if ((rc = totals.take(16, s))) return rc;
     FragPlan p;
-    p.frames = j.dev_frames();
-    p.draws = j.dev_draws();
+    p.frames = sh->d_vis_tables.as<Frame>();
+    p.draws = (const Draw*)(sh->d_vis_tables.as<uint8_t>() + j.draws_at);
     p.n_draws = (uint32_t)j.draws.size();
     p.vis = sh->d_vis.as<int32_t>();
     p.n_segs = segs;
@@ -1676,6 +1682,7 @@ static int shading_lists(sloth_shading* sh)
     p.chunks = sh->d_chunks.as<uint4>();
     if ((rc = launch_frag_fill(p, sh->n_tris, s))) return rc;
     sh->n_chunks = n_chunks;
+    sh->lists = true;
     return SLOTH_OK;
 }
 
@@ -1685,13 +1692,16 @@ static int shading_visibility(sloth_shading* sh)
     sloth_batch* b = sh->b;
     Job& j = b->job;
     int rc;
+    sh->lists = false;
+    if ((rc = sh->d_vis_tables.reserve(j.ramps_at))) return rc;
+    HIP_TRY(hipMemcpyAsync(sh->d_vis_tables.p, j.d_tables.p, j.ramps_at, hipMemcpyDeviceToDevice, b->stream));
     if ((rc = j.prepare(b->stream))) return rc;
     if ((rc = j.launch(0, (uint32_t)j.frames.size(), b->stream, sh->d_vis.as<int32_t>(), nullptr, true))) return rc;
     HIP_TRY(hipStreamSynchronize(b->stream));
     if ((rc = j.finish(0, (uint32_t)j.frames.size(), b->stream, sh->d_vis.as<int32_t>(), nullptr, true))) return rc;
     b->ran = true;
     b->checked = true;
-    return shading_lists(sh);
+    return SLOTH_OK;
 }
 
 extern "C" {
@@ -1722,6 +1732,7 @@ int sloth_shading_create(sloth_batch* b, const uint32_t* faces, uint32_t n_tris,
         (rc = sh->d_vnormal.reserve(std::max<size_t>(4, (size_t)n_verts * 12))) ||
         (rc = sh->d_light.reserve(16)) ||
         (rc = sh->d_sum.reserve(32)) ||
+        (rc = sh->d_partial.reserve((size_t)shade_blocks(sh->n_slots) * 32 + 32)) ||
         (rc = sh->d_vert_acc.reserve(std::max<size_t>(8, (size_t)n_verts * 6 * 8))) ||
         (rc = sh->d_dcolor.reserve(std::max<size_t>(4, (size_t)n_verts * 12))) ||
         (rc = sh->d_dnormal.reserve(std::max<size_t>(4, (size_t)n_verts * 12)))) {
@@ -1806,8 +1817,9 @@ static int shading_params(sloth_shading* sh, const float* vcolor, const float* v
 static int shading_backward_launch(sloth_shading* sh)
 {
     hipStream_t s = sh->b->stream;
-    const ShadeArgs a = shade_args(sh, true, nullptr);
     int rc;
+    if ((rc = shading_lists(sh))) return rc;
+    const ShadeArgs a = shade_args(sh, true, nullptr);
     if (!sh->acc_zero && (rc = launch_shade_zero(a, s))) return rc;
     sh->acc_zero = false;
     if ((rc = launch_shade_bwd(a, sh->d_dcolor.as<float>(), sh->d_dnormal.as<float>(), sh->d_sum.as<double>(), s)))
@@ -1889,6 +1901,7 @@ int sloth_shading_time(sloth_shading* sh, uint32_t steps, uint32_t warmup, float
     int rc = ensure_device();
     if (rc) return rc;
     hipStream_t s = sh->b->stream;
+    if ((rc = shading_lists(sh))) return rc;
     auto step = [&]() -> int { return shading_backward_launch(sh); };   // loss and gradients in one pass
     for (uint32_t i = 0; i < warmup; ++i)
         if ((rc = step())) return rc;
