@@ -1645,6 +1645,14 @@ static void normal_map(const float* M, float* G)
         for (int c = 0; c < 3; ++c) G[r * 3 + c] = (float)(cof[r][c] / k);
 }
 
+// Room for n bytes, and when that takes a new allocation for a quarter more:
+// views that move show a little more again and again.
+static int reserve_ahead(DevBuf& b, size_t n)
+{
+    if (n <= b.bytes || b.reserve(n + n / 4) == SLOTH_OK) return SLOTH_OK;
+    return b.reserve(n);
+}
+
 // The fragment lists of the visibility, unless they are there: counted, sized,
 // filled.
 static int shading_lists(sloth_shading* sh)
@@ -1674,8 +1682,8 @@ static int shading_lists(sloth_shading* sh)
     HIP_TRY(hipStreamSynchronize(s));
     totals.done();
     const uint64_t n_entries = p.totals[0], n_chunks = p.totals[1];
-    if ((rc = sh->d_entries.reserve(std::max<uint64_t>(1, n_entries) * sizeof(uint4))) ||
-        (rc = sh->d_chunks.reserve(std::max<uint64_t>(1, n_chunks) * sizeof(uint4))) ||
+    if ((rc = reserve_ahead(sh->d_entries, std::max<uint64_t>(1, n_entries) * sizeof(uint4))) ||
+        (rc = reserve_ahead(sh->d_chunks, std::max<uint64_t>(1, n_chunks) * sizeof(uint4))) ||
         (rc = sh->d_partial.reserve(std::max<uint64_t>(shade_blocks(sh->n_slots), bwd_blocks(n_chunks)) * 32 + 32)))
         return rc;
     p.entries = sh->d_entries.as<uint4>();
