@@ -442,7 +442,7 @@ struct Job {
             int rc = tiled.overflowed((uint32_t)frames.size(), s, ovf);
             if (rc) return rc;
             if (!ovf) return SLOTH_OK;
-            tiled.sized = false;
+            tiled.outgrow();
             if (replanned) *replanned = true;
             if ((rc = prepare(s))) return rc;
             if ((rc = launch(f_lo, f_hi, s, win, nullptr, win_raw))) return rc;

@@ -88,6 +88,13 @@ struct TiledPlan {
     uint64_t n_tiles = 0;
     uint64_t n_rows = 0;
     bool sized = false;              // pool offsets match the current layout
+    // a render outgrew its lists: the next sizing keeps what room they had
+    bool outgrown = false;
+    void outgrow()
+    {
+        sized = false;
+        outgrown = true;
+    }
     std::vector<uint64_t> off;       // host copy of the per-tile pool offsets (n_tiles + 1)
     // set by size(): the first frame of each part and, last, the number of
     // frames.  The parts are binned and rendered one after another and share
@@ -101,8 +108,9 @@ struct TiledPlan {
     DevBuf d_cursor, d_off, d_pool, d_nl;
     uint32_t* overflow = nullptr;    // per frame, the job's pinned memory: kernels write it (rarely), the host reads it after a wait
     // triangles whose candidate box k_careful computes: (frame, triangle,
-    // screen vertices) in, 32 bytes each, (triangle, box) out; capacity from
-    // the counting run plus headroom
+    // screen vertices) in, 32 bytes each, (triangle, box) out.  careful_cap is
+    // the counting run's number plus headroom, 0 for none (k_careful is then
+    // not launched); the memory only grows.
     DevBuf d_careful_cnt, d_careful_in, d_careful_box;
     uint32_t careful_cap = 0;
     // Batches whose draws differ in size, or whose frames differ in tile

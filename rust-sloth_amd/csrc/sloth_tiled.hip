@@ -1754,6 +1754,9 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
         }
     }
     // 1. count tile entries of CLS_BOX triangles and the careful triangles
+    const uint32_t cap_before = careful_cap;
+    auto careful_room = [&] { return (uint32_t)(std::min(d_careful_in.bytes / 2, d_careful_box.bytes) / sizeof(uint4)); };
+    careful_cap = careful_room();
     if ((rc = launch_clear(frames, 0, F, s))) return rc;
     if ((rc = launch_bin(frames, draws, d_frames, d_draws, 0, F, nullptr, true, s))) return rc;
     uint32_t cnt[WRAP_CNT + 1];
@@ -1773,9 +1776,12 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     // draw of tall triangles (30 unlike jobs: 104-131 -> 53-59 us)
     bin_tree = cnt[TALL_CNT] > 0 && ((uint64_t)cnt[TALL_CNT] * 256 >= n_tri || (flat_bin && cnt[TALL_CNT] >= (uint32_t)BIN_BLOCK));
     if (const char* e = getenv("SLOTH_BIN_TREE")) bin_tree = e[0] == '1';
+    // (those of other tiles than the present ones do not count: their boxes
+    // take other paths)
+    const uint32_t want = std::max(n_careful ? n_careful + n_careful / 2 + 1024 : 0u, outgrown ? cap_before : 0u);
     if (n_careful > careful_cap) {
         // 2. room for the careful list, then count again so that it is filled
-        careful_cap = n_careful + n_careful / 2 + 1024;
+        careful_cap = want;
         if ((rc = d_careful_in.reserve(2 * sizeof(uint4) * careful_cap))) return rc;
         if ((rc = d_careful_box.reserve(sizeof(uint4) * careful_cap))) return rc;
         if ((rc = launch_clear(frames, 0, F, s))) return rc;
@@ -1788,6 +1794,7 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
         HIP_TRY(hipMemcpyAsync(counts.data(), d_cursor.p, sizeof(uint32_t) * n_tiles, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipMemcpyAsync(cnt, d_careful_cnt.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
+    careful_cap = std::min(want, careful_room());
     odd_wraps = cnt[WRAP_CNT];
     if ((rc = reserve_edges())) return rc;
     off.assign(n_tiles + 1, 0);
@@ -1843,6 +1850,7 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     if ((rc = launch_clear(frames, 0, F, s))) return rc;
     HIP_TRY(hipStreamSynchronize(s));
     sized = true;
+    outgrown = false;
     return SLOTH_OK;
 }
 
