@@ -513,18 +513,43 @@ struct Encoder {
     int run(const Job& job, uint32_t first, uint32_t count, bool framing, int mode, char* out, uint64_t cap,
             uint64_t* len, hipStream_t s)
     {
-        uint64_t most = 0;
-        for (uint32_t f = first; f < first + count; ++f) most = std::max(most, frame_cells(job.frames[f]));
         EncodeJob j;
         j.cells = job.d_cells.as<uint32_t>();
         j.frames = job.dev_frames();
         j.first = first;
         j.count = count;
-        j.max_blocks = encode_blocks(most);
         j.mode = mode;
         j.framing = framing ? 1 : 0;
+        // the runs (ENC_RUN_BLOCKS): one, unless the frames' sizes are far apart
+        struct Run {
+            uint32_t lo, max_blocks;
+            uint64_t at;   // its place in the block tables
+        };
+        std::vector<Run> runs(1, Run{0, 0, 0});
+        uint64_t used = 0, most = 0, at = 0;
+        for (uint32_t f = 0; f < count; ++f) {
+            const uint64_t n = frame_cells(job.frames[first + f]);
+            most = std::max(most, n);
+            const uint32_t nb = encode_blocks(n), max_blocks = std::max(runs.back().max_blocks, nb);
+            const uint64_t blocks = (uint64_t)(f + 1 - runs.back().lo) * max_blocks;
+            used += nb;
+            if (blocks <= std::max(2 * used, ENC_RUN_BLOCKS)) {
+                runs.back().max_blocks = max_blocks;
+            } else {
+                at += (uint64_t)(f - runs.back().lo) * runs.back().max_blocks;
+                runs.push_back(Run{f, nb, at});
+                used = nb;
+            }
+        }
+        const uint64_t blocks = at + (uint64_t)(count - runs.back().lo) * runs.back().max_blocks;
+        auto use = [&](size_t r) {
+            j.lo = runs[r].lo;
+            j.hi = r + 1 < runs.size() ? runs[r + 1].lo : count;
+            j.max_blocks = runs[r].max_blocks;
+            j.block_len = d_len.as<uint32_t>() + runs[r].at;
+            j.block_off = d_off.as<uint64_t>() + runs[r].at;
+        };
         const bool one = count == 1 && most <= ENC_ONE_CELLS;
-        const uint64_t blocks = (uint64_t)count * j.max_blocks;
         // pinned: the frame offsets, and a small stream's bytes after them
         PinLease pin;
         const uint64_t off_bytes = (((uint64_t)count + 1) * 8 + 255) & ~255ull;
@@ -533,14 +558,14 @@ struct Encoder {
         j.frame_off = pin.as<uint64_t>();
         uint8_t* h_one = pin.as<uint8_t>() + off_bytes;
         if (one) {
-            j.block_len = nullptr;
-            j.block_off = nullptr;
+            use(0);   // without block tables
             if ((rc = launch_encode_one(j, out ? h_one : nullptr, s))) return rc;
         } else {
             if ((rc = d_len.reserve(blocks * 4)) || (rc = d_off.reserve(blocks * 8))) return rc;
-            j.block_len = d_len.as<uint32_t>();
-            j.block_off = d_off.as<uint64_t>();
-            if ((rc = launch_encode_len(j, s))) return rc;
+            for (size_t r = 0; r < runs.size(); ++r) {
+                use(r);
+                if ((rc = launch_encode_len(j, s))) return rc;
+            }
         }
         HIP_TRY(hipStreamSynchronize(s));
         pin.done();
@@ -556,12 +581,19 @@ struct Encoder {
             return SLOTH_OK;
         }
         // groups of whole frames of up to GROUP_BYTES (one frame at least)
+        size_t r = 0;
         for (uint32_t f0 = 0; f0 < count;) {
             uint32_t f1 = f0 + 1;
             while (f1 < count && off[f1 + 1] - off[f0] <= GROUP_BYTES) ++f1;
             const uint64_t bytes = off[f1] - off[f0];
             if ((rc = d_out.reserve(bytes))) return rc;
-            if ((rc = launch_encode_write(j, f0, f1, off[f0], d_out.as<uint8_t>(), s))) return rc;
+            for (uint32_t f = f0; f < f1;) {
+                use(r);
+                const uint32_t end = std::min(f1, j.hi);
+                if ((rc = launch_encode_write(j, f, end, off[f0], d_out.as<uint8_t>(), s))) return rc;
+                if (end == j.hi) ++r;
+                f = end;
+            }
             const Span whole{out + off[f0], d_out.p, bytes};
             if ((rc = copy_out(&whole, 1, s))) return rc;
             f0 = f1;

@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(ENC_BLOCK) k_enc_len(EncodeJob j, uint32_t f_l
     const Frame& fr = j.frames[j.first + f];
     const uint64_t n = frame_cells(fr);
     const uint32_t nb = (uint32_t)((n + ENC_CELLS - 1) / ENC_CELLS);
-    uint32_t* out = j.block_len + (uint64_t)f * j.max_blocks + b;
+    uint32_t* out = j.block_len + (uint64_t)(f - j.lo) * j.max_blocks + b;
     if (b >= nb) {
         if (threadIdx.x == 0) *out = 0;
         return;
@@ -172,14 +172,15 @@ __global__ void __launch_bounds__(ENC_BLOCK) k_enc_len(EncodeJob j, uint32_t f_l
         *out = total + (b == 0 ? prefix_len(j, f, fr.image != 0) : 0u) + (b == nb - 1 ? suffix_len(j, f) : 0u);
 }
 
-// Exclusive scan of the block lengths (one workgroup, SCAN_ITEMS a thread and
-// round).  frame_off[f] = where frame f starts, frame_off[count] = the length
-// (host memory: the caller reads it after the stream).
+// Exclusive scan of the run's block lengths (one workgroup, SCAN_ITEMS a thread
+// and round), from where the run before ended.  frame_off[f] = where frame f
+// starts, frame_off[hi] = the length so far (host memory: the caller reads it
+// after the stream).
 __global__ void __launch_bounds__(SCAN_BLOCK) k_enc_scan(EncodeJob j)
 {
     __shared__ uint64_t s_wave[SCAN_BLOCK / 64];
-    const uint64_t n = (uint64_t)j.count * j.max_blocks;
-    uint64_t carry = 0;
+    const uint64_t n = (uint64_t)(j.hi - j.lo) * j.max_blocks;
+    uint64_t carry = j.lo ? j.frame_off[j.lo] : 0;
     for (uint64_t base = 0; base < n; base += SCAN_BLOCK * SCAN_ITEMS) {
         const uint64_t i0 = base + threadIdx.x * SCAN_ITEMS;
         uint32_t l[SCAN_ITEMS];
@@ -195,14 +196,14 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_enc_scan(EncodeJob j)
         for (uint32_t k = 0; k < SCAN_ITEMS; ++k) {
             if (i0 + k < n) {
                 j.block_off[i0 + k] = run;
-                if ((i0 + k) % j.max_blocks == 0) j.frame_off[(i0 + k) / j.max_blocks] = run;
+                if ((i0 + k) % j.max_blocks == 0) j.frame_off[j.lo + (i0 + k) / j.max_blocks] = run;
             }
             run += l[k];
         }
         carry += total;
         __syncthreads();   // s_wave is free for the next round
     }
-    if (threadIdx.x == 0) j.frame_off[j.count] = carry;
+    if (threadIdx.x == 0) j.frame_off[j.hi] = carry;
 }
 
 __device__ __forceinline__ uint32_t put_dec(uint8_t* p, uint32_t v)
@@ -318,7 +319,7 @@ __global__ void __launch_bounds__(ENC_BLOCK) k_enc_write(EncodeJob j, uint32_t f
     const uint64_t n = frame_cells(fr);
     const uint32_t nb = (uint32_t)((n + ENC_CELLS - 1) / ENC_CELLS);
     if (b >= nb) return;
-    enc_block<MODE>(j, f, fr, n, b, nb, out + (j.block_off[(uint64_t)f * j.max_blocks + b] - base), stage, s_wave);
+    enc_block<MODE>(j, f, fr, n, b, nb, out + (j.block_off[(uint64_t)(f - j.lo) * j.max_blocks + b] - base), stage, s_wave);
 }
 
 // A stream of one frame of few cells, in one launch: block b finds its place
@@ -372,8 +373,8 @@ uint64_t encode_bound(uint64_t n_cells, int mode)
 
 int launch_encode_len(const EncodeJob& j, hipStream_t s)
 {
-    for (uint32_t f = 0; f < j.count; f += 65535u) {
-        hipLaunchKernelGGL(k_enc_len, dim3(j.max_blocks, std::min(65535u, j.count - f)), dim3(ENC_BLOCK), 0, s, j, f);
+    for (uint32_t f = j.lo; f < j.hi; f += 65535u) {
+        hipLaunchKernelGGL(k_enc_len, dim3(j.max_blocks, std::min(65535u, j.hi - f)), dim3(ENC_BLOCK), 0, s, j, f);
         HIP_TRY(hipGetLastError());
     }
     hipLaunchKernelGGL(k_enc_scan, dim3(1), dim3(SCAN_BLOCK), 0, s, j);
