@@ -1795,10 +1795,7 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     HIP_TRY(hipMemcpyAsync(cnt, d_careful_cnt.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     careful_cap = std::min(want, careful_room());
-    // a job that has outgrown its columns moves: room for half as many more, and
-    // no narrower again (it may move back)
-    const uint32_t need = cnt[WRAP_CNT];
-    odd_wraps = !outgrown ? need : need > odd_wraps ? need + need / 2 + 1 : odd_wraps;
+    odd_wraps = cnt[WRAP_CNT];
     if ((rc = reserve_edges())) return rc;
     off.assign(n_tiles + 1, 0);
     multi = false;
