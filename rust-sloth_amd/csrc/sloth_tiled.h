@@ -78,7 +78,8 @@ struct TiledPlan {
     // cells in k_tile_edges.
     bool has_even = true, has_odd = false;
     // odd_wraps: the tile columns that the counting run's boxes ask for
-    // (odd_cols_of); a later run that finds more raises the overflow flag.
+    // (odd_cols_of), a third more after a run that found more and so raised the
+    // overflow flag.
     // odd_narrow: frames one column wide (only newline cells).
     uint32_t odd_wraps = 0;
     bool odd_narrow = false;

@@ -1795,7 +1795,11 @@ int TiledPlan::size(const std::vector<Frame>& frames, const std::vector<Draw>& d
     HIP_TRY(hipMemcpyAsync(cnt, d_careful_cnt.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     careful_cap = std::min(want, careful_room());
-    odd_wraps = cnt[WRAP_CNT];
+    // a reach that outgrew its columns may go on growing: room for a third more.
+    // (Columns kept, or one more at least, cost a view that moves to and fro more
+    // than its re-sizes: 641x480 turned by 3.6 degrees a frame 99 -> 115 us.)
+    const uint32_t need = cnt[WRAP_CNT];
+    odd_wraps = need + (outgrown && need > odd_wraps ? need / 3 : 0u);
     if ((rc = reserve_edges())) return rc;
     off.assign(n_tiles + 1, 0);
     multi = false;

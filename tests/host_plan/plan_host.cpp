@@ -187,9 +187,38 @@ static int careful_room()
     return 0;
 }
 
+// Odd widths: a view whose wrapped boxes reach further and further is sized
+// again a few times, not for each tile column; any other sizing has the columns
+// that the scene needs and no more.
+static int odd_reach()
+{
+    Scene sc(1919, 1079);
+    CHECK(sc.plan.set_tile(64, 32) == SLOTH_OK);
+    careful = 0;
+    wraps = 2;
+    CHECK(sc.render() == SLOTH_OK && sc.sizings == 1 && sc.plan.odd_cols() == 2);
+    for (wraps = 2; wraps <= 30; ++wraps) {
+        CHECK(sc.render() == SLOTH_OK && sc.plan.odd_cols() >= wraps);
+        CHECK(find("k_tile_edges")->grid.y <= 30);   // the frame has 30 columns
+    }
+    printf("%d sizings\n", sc.sizings);
+    CHECK(sc.sizings <= 8);
+    careful = 7;   // outgrown for another reason
+    for (uint32_t w : {1, 0, 17}) {
+        wraps = w;
+        sc.plan.outgrow();
+        CHECK(sc.size() == SLOTH_OK && sc.plan.odd_cols() == (w == 17 ? 22 : w));
+    }
+    CHECK(sc.plan.set_tile(128, 16) == SLOTH_OK);   // other tiles: sized for what is there
+    wraps = 9;
+    CHECK(sc.render() == SLOTH_OK && sc.plan.odd_cols() == 9);
+    return 0;
+}
+
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "careful_room") return careful_room();
+    if (what == "odd_reach") return odd_reach();
     return 2;
 }

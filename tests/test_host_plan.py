@@ -19,7 +19,7 @@ def host(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["careful_room"])
+@pytest.mark.parametrize("what", ["careful_room", "odd_reach"])
 def test_plan(host, what):
     r = subprocess.run([host, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
