@@ -116,11 +116,11 @@ def main() -> int:
                     help="only the 4K-frame leg, at this plan instead of the autotuner's (for profilers)")
     ap.add_argument("--uneven-only", default=None, metavar="WxH,WALK,TPT",
                     help="only the uneven-batch leg, at this plan instead of the autotuner's (for profilers)")
-    ap.add_argument("--graph-only", action="store_true",
+    ap.add_argument("--batched-only", "--graph-only", action="store_true",
                     help="only the batched renders (for profilers): no plain, stage, CPU or other legs")
     ap.add_argument("--no-extra", action="store_true", help="skip the 4K, uneven-batch and shading legs")
     args = ap.parse_args()
-    if args.graph_only:
+    if args.batched_only:
         args.plain_steps = args.profile_runs = args.cpu_frames = 0
         args.repeats = 1
         args.no_extra = True
@@ -257,7 +257,7 @@ def main() -> int:
             counts.append(int(fr.stats[1]))
         frags = statistics.mean(counts)
 
-    atom = atomic_peak() if not args.graph_only else None
+    atom = atomic_peak() if not args.batched_only else None
     atomic_roof = None
     if atom and frags and dominant:
         per_sweep = frags * F
@@ -321,7 +321,7 @@ def _frac(alg_bytes, ms):
 def leg_4k(sloth_amd, meshgen, args):
     """One 3840x2160 frame of the 8-subdivision displaced icosphere
     (1,310,720 triangles, seed 1): plain form (launch sequence + sync) and
-    batched form (the keys `_graph`), median of 5 timings of 10 frames each."""
+    batched form, median of 5 timings of 10 frames each."""
     log("bench: 4K frame leg")
     m, W, H, U, R = meshgen.workload_icosphere_4k()
     mesh = sloth_amd.SimpleMesh.from_mesh(m)
@@ -339,8 +339,8 @@ def leg_4k(sloth_amd, meshgen, args):
     gbs, frac = _frac(alg, msg)
     return {"workload": f"displaced icosphere s8 ({m.n} tris, seed 1), 3840x2160 image mode, one frame",
             "plan": b.plan(), "ms_per_frame": round(ms, 4), "frames_per_s": round(1e3 / ms, 1),
-            "ms_per_frame_graph": round(msg, 4), "gtri_per_s": round(m.n / ms / 1e6, 3),
-            "alg_bytes": alg, "achieved_GBps_graph": gbs, "frac_graph": frac}
+            "ms_per_frame_batched": round(msg, 4), "gtri_per_s": round(m.n / ms / 1e6, 3),
+            "alg_bytes": alg, "achieved_GBps_batched": gbs, "frac_batched": frac}
 
 
 def leg_uneven(sloth_amd, meshgen, args):

@@ -1,4 +1,4 @@
-// Tiled raster path (even widths): bin-to-tile and LDS tile raster.
+// Tiled raster path: bin-to-tile and LDS tile raster.
 // The data flow is described in sloth_tiled.h.
 #include <algorithm>
 #include <cstdlib>
@@ -1374,7 +1374,8 @@ __device__ __forceinline__ void raster_tile(const Draw* __restrict__ draws, cons
         for (uint32_t i = threadIdx.x; i < H; i += blockDim.x) __builtin_nontemporal_store(CELL_BLANK, fc + (uint64_t)W * H + i);
 }
 
-// The tile of a frame's workgroup r, RAGGED and ANY: workgroups go to the eight
+// The tile of a frame's workgroup r, RAGGED and ANY (3-D grids; flat ones keep
+// their table's order): workgroups go to the eight
 // XCDs in turn, so taking eight tile rows at a time gives each XCD, and its L2,
 // whole rows.  The rows of such widths start within a line, and the lines that
 // two tiles of a row share are then put together before they leave for memory:
