@@ -201,8 +201,8 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade_fwd(ShadeArgs p)
 //   x, y = first entry (64 bits), z = entries, w = draw.
 // So a chunk is one wavefront's work with a uniform draw, and neighbouring
 // chunks, also those of other views, are of the same triangles.  Making the
-// lists takes 0.186 ms for 32 views of 99,904 triangles (0.077 counted, 0.034
-// scanned, 0.074 filled), at the first backward pass after a visibility.
+// lists takes 0.18 ms for 32 views of 99,904 triangles (0.074 counted, 0.034
+// scanned, 0.073 filled), at the first backward pass after a visibility.
 constexpr uint32_t FRAG_BLOCK = SHADE_BLOCK;
 constexpr int FRAG_SIDE = 8;
 constexpr int FRAG_OWN = 4;   // pixel blocks of a box that its lane scans by itself

@@ -779,13 +779,14 @@ __device__ __forceinline__ uint32_t entry_tri(uint32_t e, const uint4* __restric
 // What bounds it: VALU issue (a wave64 instruction takes four cycles of its
 // SIMD).  A wavefront of entries costs about 240 instructions of set-up and 23
 // per step of its largest box, and a slot pair about 35 at the end.
-// 256 frames of 1920x1080, 327,680 triangles: 592M wavefront instructions on
-// 1024 SIMDs, 1.02 ms (the stores of its 4.26 GB alone take 0.75 ms).  Before,
+// 256 frames of 1920x1080, 327,680 triangles: 600M wavefront instructions, 0.98
+// ms on 1024 SIMDs at 2.4 GHz, which is what it takes under the profiler (0.94 by
+// events; the stores of its 4.26 GB alone take 0.75 ms).  Before,
 // with rows of 48 bytes, nine operations more per pixel and chunk by chunk
 // stores, 762M and 1.19 ms.
 //
 // BIG: an entry whose box covers more than BIG_BOX of the tile's pixels in
-// its direct region is not walked by its own lane; after its own walk, each
+// its direct or its wrapped region is not walked there by its own lane; after its own walk, each
 // wavefront takes its lanes' big boxes one at a time and all 64 lanes stride
 // over the box.  The variant costs registers on every path, so it is launched
 // only for lists with many big boxes (TiledPlan::big_walk).
@@ -1410,7 +1411,8 @@ __global__ void __launch_bounds__(RASTER_BLOCK) __attribute__((amdgpu_waves_per_
     uint32_t n_ramps, uint4* __restrict__ edge_out, uint32_t* __restrict__ careful_reset,
     const uint2* __restrict__ tile_frame, uint32_t t_lo, uint32_t odd_cols, uint32_t keep)
 {
-    // keys, rows and cells are read and written in 16-byte words
+    // keys, rows and cells are read and written in 16-byte words (declared for 8
+    // it began at 360: 256 frames of 1920x1080 1495 us, now 1471)
     extern __shared__ __align__(16) uint64_t smem[];
     // the job's first LDS_RAMPS shaders, so that a glyph lookup reads LDS
     // (read only after the tile's first barrier)
